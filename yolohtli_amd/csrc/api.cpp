@@ -294,11 +294,13 @@ int yh_rd_step_dev_ex(const yh_params* p, float* const out[3], const float* cons
                          (hipStream_t)stream));
     return YH_OK;
   }
-  // the stages of RK2/RK4 need scratch fields: a plan owns them
-  if (p->timeIntOrder != 1) return YH_EUNSUPPORTED;
+  if (p->timeIntOrder != 1) return YH_EUNSUPPORTED;  // RK2 and RK4 are a plan's
   const GParams g = make_gparams(*p, stim_on, stim_x, stim_y);
-  YH_HIP(launch_general_step(p->model, g, 1, ci, co, cv, p->solidSwitch ? solid : nullptr,
-                             nullptr, (hipStream_t)stream, nullptr));
+  int dev = 0, cus = 0;
+  YH_HIP(hipGetDevice(&dev));
+  YH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  YH_HIP(launch_general(p->model, g, 1, general_shape(p->model, g, 1, 1, cus), ci, co, cv, nullptr,
+                        p->solidSwitch ? solid : nullptr, (hipStream_t)stream, nullptr));
   return YH_OK;
 }
 

@@ -1,22 +1,25 @@
 // general.hip -- the reference kernel's other branches on the device:
 // Dirichlet boundaries, the 4th-order compact Laplacian (lap4), the
 // anisotropic cross term, RK2 / RK4 and the circular mouse stimulus
-// (reactionDiffusion.cu:36-561).  One launch per Runge-Kutta stage, one
-// thread per cell.
+// (reactionDiffusion.cu:36-561).  One launch advances several Runge-Kutta
+// stages, and where they are few several steps, of a tile held in registers
+// and LDS.
 //
 // The reference writes each stage state into its input while neighbours read
 // it (:114-119) and reads lap4's neighbour currents J from the same launch
 // (:221-236).  Here a stage reads only the step's input y0 and the previous
-// stage's increments d: the stage field is y0 + ki*d_{s-1} (computed where it
-// is read), a neighbour's current is evaluated from that neighbour's stage
-// state, and the increments of all cells are complete before the next stage
-// starts.  Reads outside the domain that the reference makes in the masked
+// stage's increments d: the stage field is y0 + ki*d_{s-1}, a neighbour's
+// current is evaluated from that neighbour's stage state, and the stage field
+// of a tile is complete (a barrier, two LDS buffers) before the next stage
+// reads it.  Reads outside the domain that the reference makes in the masked
 // Dirichlet branch (:364-373 at the domain edge) count as non-tissue.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "plan.h"
+#include "tile.h"
 
 namespace yh {
 
@@ -71,270 +74,525 @@ GParams make_gparams(const yh_params& p, int stim_on, int stim_x, int stim_y) {
   g.tau_v2m = (float)f.tau_v2m;
   g.tau_wp = (float)f.tau_wp;
   g.tau_wm = (float)f.tau_wm;
+  g.tau_2si = 2.0f * g.tau_si;
+  auto recip = [](float t) { return (float)(1.0 / (double)t); };
+  g.r_d = recip(g.tau_d);
+  g.r_r = recip(g.tau_r);
+  g.r_2si = recip(g.tau_2si);
+  g.r_0 = recip(g.tau_0);
+  g.r_vp = recip(g.tau_vp);
+  g.r_v1m = recip(g.tau_v1m);
+  g.r_v2m = recip(g.tau_v2m);
+  g.r_wp = recip(g.tau_wp);
+  g.r_wm = recip(g.tau_wm);
   g.stim_on = stim_on;
   g.stim_x = stim_x;
   g.stim_y = stim_y;
   return g;
 }
 
+// a / t from the reciprocal r of t, itself correctly rounded: the quotient
+// estimate a*r and its exact remainder give the correctly rounded quotient
+// (Markstein, IBM J. Res. Dev. 34(1), 1990), in 3 instructions where a
+// division takes 11; the FK currents have eight.  An infinite a gives NaN.
+__device__ __forceinline__ float g_quotient(float a, float t, float r) {
+  const float e = a * r;
+  return __builtin_fmaf(__builtin_fmaf(-t, e, a), r, e);
+}
+
 // Ionic currents (:131-141 for 2V, Fenton & Karma 1998 for FK) at a cell of
-// the stage field, with the mouse stimulus when the cell is in its disk.
+// the stage field; st: the mouse stimulus, 24.7 for a cell in its disk, else 0.
 template <int MODEL>
-__device__ __forceinline__ void g_currents(const GParams& g, float u, float v, float w, int i,
-                                           int j, float& Iu, float& Iv, float& Iw) {
-  // :54-61: (ic-cx)^2 + (jc-cy)^2 < 400 with the point in cells
-  const int di = i - g.stim_x, dj = j - g.stim_y;
-  const float st = (g.stim_on && di * di + dj * dj < 400) ? 24.7f : 0.0f;
+__device__ __forceinline__ void g_currents(const GParams& g, float u, float v, float w, float st,
+                                           float& Iu, float& Iv, float& Iw) {
   if (MODEL == M2V) {
     Iu = -(g.mu * u * (1.0f - u) * (u - g.alpha) - u * v) - st;
     Iv = -(g.eps * (g.delta * (u - g.gamma) * (g.beta - u) - v - g.theta));
     Iw = 0.0f;
   } else {
-    const float p = u >= g.u_c ? 1.0f : 0.0f, q = u >= g.u_v ? 1.0f : 0.0f;
-    const float J_fi = -v * p * (1.0f - u) * (u - g.u_c) / g.tau_d;
-    const float J_so = u * (1.0f - p) / g.tau_0 + p / g.tau_r;
-    const float J_si = -w * (1.0f + tanhf(g.kk * (u - g.u_csi))) / (2.0f * g.tau_si);
-    const float tvm = (1.0f - q) * g.tau_v1m + q * g.tau_v2m;
-    Iu = J_fi + J_so + J_si - st;
-    Iv = -((1.0f - p) * (1.0f - v) / tvm - p * v / g.tau_vp);
-    Iw = -((1.0f - p) * (1.0f - w) / g.tau_wm - p * w / g.tau_wp);
+    // J_fi = -p v (1-u)(u-u_c)/tau_d, J_so = (1-p) u/tau_0 + p/tau_r,
+    // J_si = -w (1 + tanh(k(u-u_csi)))/(2 tau_si), and the gates' rates: p and
+    // q are 0 or 1, so each sum of two branches is the quotient of one.
+    const bool p = u >= g.u_c, q = u >= g.u_v;
+    const float J = g_quotient(p ? -v * (1.0f - u) * (u - g.u_c) : u, p ? g.tau_d : g.tau_0,
+                               p ? g.r_d : g.r_0);
+    const float J_si = g_quotient(-w * (1.0f + tanhf(g.kk * (u - g.u_csi))), g.tau_2si, g.r_2si);
+    const float tvm = q ? g.tau_v2m : g.tau_v1m, rvm = q ? g.r_v2m : g.r_v1m;
+    Iu = (p ? J + g.r_r : J) + J_si - st;
+    Iv = g_quotient(p ? v : v - 1.0f, p ? g.tau_vp : tvm, p ? g.r_vp : rvm);
+    Iw = g_quotient(p ? w : w - 1.0f, p ? g.tau_wp : g.tau_wm, p ? g.r_wp : g.r_wm);
   }
 }
 
-// Stage field of variable a at cell index c.
-struct StageField {
-  CFields y0, dp;
-  float ki;
-  __device__ __forceinline__ float operator()(int a, int c) const {
-    const float x = y0.f[a][c];
-    return ki != 0.0f ? __builtin_fmaf(ki, dp.f[a][c], x) : x;
-  }
+// Neighbour rules of a launch (a template constant: each keeps only its own
+// registers and LDS arrays).
+enum { G_SQUARE = 0, G_LAP4 = 1, G_ANISO = 2, G_LAP4_ANISO = 3, G_MASKED = 4, G_DIRICHLET = 5 };
+
+// A launch advances K steps of `order` stages each, T = K * order stages in
+// all.  A workgroup owns a region of 64 columns (one per lane) x `rows` rows;
+// row lr belongs to wave lr % 16, so every stage's rows spread evenly over the
+// four SIMDs as the region shrinks.  After T stages the inner region, `halo` =
+// T * rad cells in from each side, is exact and written out; the ring is
+// recomputed by the neighbouring workgroups.  rad is 1 cell per stage, 2 for
+// the anisotropic no-flux branch (its edge corrections read two cells along
+// the edge).
+//
+// What bounds it: a stage needs only the stage field and (lap4) the currents
+// of the four to eight neighbours, so they live in LDS and every other value
+// of a cell (the step's start, the accumulated rhs, the field itself, its
+// current, its coefficients) stays in its lane's registers from load to store.
+// Neighbours sit at fixed LDS offsets: a cell next to the domain edge also
+// writes its value to its mirror image outside (no flux), or the outside holds
+// the boundary value (Dirichlet), so no lane computes an index in the loop,
+// and a cell's current is evaluated once per stage, not once per neighbour.
+// One stage a launch through global memory, as this was before, took 8.7-9.1
+// us a stage at 512 x 512 whatever the rule (40 dependent loads a cell).
+constexpr int kGenWaves = 16, kGenThreads = 64 * kGenWaves;
+constexpr int kGenPer = 3;                     // rows of a wave, at most
+constexpr int kGenRows = kGenWaves * kGenPer;  // rows of a region, at most
+constexpr int kGenPad = 2;                     // pad cells around the region in LDS
+constexpr int kGenStride = 64 + 2 * kGenPad;
+constexpr int kGenHalo = 8;
+
+struct GenRun {
+  int K, order, rad, rows, halo, out_w, out_h, tiles_x, ntiles;
+  float ki[5], sw[4];  // :70-95
 };
 
-// Diagonal neighbours of the Neumann square branch (:207-221, :250-264).
-__device__ __forceinline__ void g_diag(int nx, int ny, int i, int j, int& SW, int& SE, int& NW,
-                                       int& NE) {
-  SW = (i > 0 && j > 0) ? i - 1 + nx * (j - 1)
-       : ((i == 0 && j > 0) ? i + 1 + nx * (j - 1)
-                            : ((i > 0 && j == 0) ? i - 1 + nx * (j + 1) : i + 1 + nx * (j + 1)));
-  SE = (i < nx - 1 && j > 0) ? i + 1 + nx * (j - 1)
-       : ((i == nx - 1 && j > 0) ? i - 1 + nx * (j - 1)
-                                 : ((i < nx - 1 && j == 0) ? i + 1 + nx * (j + 1) : i - 1 + nx * (j + 1)));
-  NW = (i > 0 && j < ny - 1) ? i - 1 + nx * (j + 1)
-       : ((i == 0 && j < ny - 1) ? i + 1 + nx * (j + 1)
-                                 : ((i > 0 && j == ny - 1) ? i - 1 + nx * (j - 1) : i + 1 + nx * (j - 1)));
-  NE = (i < nx - 1 && j < ny - 1) ? i + 1 + nx * (j + 1)
-       : ((i == nx - 1 && j < ny - 1) ? i - 1 + nx * (j + 1)
-                                      : ((i < nx - 1 && j == ny - 1) ? i + 1 + nx * (j - 1) : i - 1 + nx * (j - 1)));
-}
+// The values of a cell that neighbours read: u, and v of the 2V model (a
+// 64-bit LDS access for the pair).
+template <int MODEL>
+struct GenPair {
+  using type = float;
+  static __device__ __forceinline__ float make(float u, float) { return u; }
+  static __device__ __forceinline__ float get(float p, int) { return p; }
+};
+template <>
+struct GenPair<M2V> {
+  using type = float2;
+  static __device__ __forceinline__ float2 make(float u, float v) { return make_float2(u, v); }
+  static __device__ __forceinline__ float get(float2 p, int a) { return a ? p.y : p.x; }
+};
 
-// Anisotropic term of variable a on the Neumann square branch (:266-313),
-// scaled by s (1 for u, rscale for v).
-__device__ __forceinline__ float g_aniso_neumann(const GParams& g, const StageField& Y, int a,
-                                                 int i, int j, float s) {
-  const int nx = g.nx, ny = g.ny, c = i + nx * j;
-  int SW, SE, NW, NE;
-  g_diag(nx, ny, i, j, SW, SE, NW, NE);
-  const float b_S = (j > 0) ? 0.0f : ((i == 0 || i == nx - 1) ? 0.0f
-                    : g.rby * (Y(a, c + 1) - Y(a, c - 1)));
-  const float b_N = (j < ny - 1) ? 0.0f : ((i == 0 || i == nx - 1) ? 0.0f
-                    : -g.rby * (Y(a, c + 1) - Y(a, c - 1)));
-  const float b_W = (i > 0) ? 0.0f : ((j == 0 || j == ny - 1) ? 0.0f
-                    : g.rbx * (Y(a, c + nx) - Y(a, c - nx)));
-  const float b_E = (i < nx - 1) ? 0.0f : ((j == 0 || j == ny - 1) ? 0.0f
-                    : -g.rbx * (Y(a, c + nx) - Y(a, c - nx)));
+template <int MODEL, int KIND>
+struct GenLds {
+  static constexpr bool LAP4 = KIND == G_LAP4 || KIND == G_LAP4_ANISO;
+  static constexpr int N = (kGenRows + 2 * kGenPad) * kGenStride;
+  typename GenPair<MODEL>::type y[2][N];               // stage field
+  typename GenPair<MODEL>::type j[LAP4 ? 2 : 1][LAP4 ? N : 1];  // currents of the stage field
+};
+
+// Anisotropic term of variable a on the Neumann square branch (:249-356),
+// scaled by s (1 for u, rscale for v).  Y(a, dx, dy) is the stage field at an
+// offset from the cell; past an edge it is the mirrored cell (:207-221), whose
+// value the corrections b amend.  edges: the workgroup holds cells of the west
+// or east edge.
+template <class YF>
+__device__ __forceinline__ float g_aniso_neumann(const GParams& g, const YF& Y, int a, int i,
+                                                 int j, float s, bool edges) {
+  const int nx = g.nx, ny = g.ny;
+  float b_S = 0.0f, b_N = 0.0f, b_W = 0.0f, b_E = 0.0f;
+  float b_SW = 0.0f, b_SE = 0.0f, b_NW = 0.0f, b_NE = 0.0f;
+  if (j == 0 || j == ny - 1) {  // the same for the whole wave
+    const bool in = i > 0 && i < nx - 1, lo = j == 0;
+    const float t = g.rby * (Y(a, 1, 0) - Y(a, -1, 0));
+    b_S = lo && in ? t : 0.0f;
+    b_N = !lo && in ? -t : 0.0f;
+    // in the corner columns the west and east corrections take the side
+    // away from this edge
+    const float w2 = g.rby * (Y(a, 0, 0) - Y(a, -2, 0)), e2 = g.rby * (Y(a, 2, 0) - Y(a, 0, 0));
+    const float w = i > 1 ? w2 : 0.0f, e = i < nx - 2 ? e2 : 0.0f;
+    b_SW = lo ? w : 0.0f;
+    b_SE = lo ? e : 0.0f;
+    b_NW = lo ? 0.0f : -w;
+    b_NE = lo ? 0.0f : -e;
+  }
+  if (edges) {  // some lane may hold a cell of the west or east edge
+    const bool W = i == 0, E = i == nx - 1;
+    const float t = j > 0 && j < ny - 1 ? g.rbx * (Y(a, 0, 1) - Y(a, 0, -1)) : 0.0f;
+    b_W = W ? t : 0.0f;
+    b_E = E ? -t : 0.0f;
+    if (j > 1) {
+      const float s2 = g.rbx * (Y(a, 0, 0) - Y(a, 0, -2));
+      b_SW = W ? s2 : b_SW;
+      b_SE = E ? -s2 : b_SE;
+    }
+    if (j < ny - 2) {
+      const float n2 = g.rbx * (Y(a, 0, 2) - Y(a, 0, 0));
+      b_NW = W ? n2 : b_NW;
+      b_NE = E ? -n2 : b_NE;
+    }
+  }
   float d = ((b_S + b_N) * g.ry + (b_W + b_E) * g.rx) * s;
-  const float b_SW = (i > 0 && j > 0) ? 0.0f
-                     : ((i == 0 && j > 1) ? g.rbx * (Y(a, c) - Y(a, c - 2 * nx))
-                        : ((i > 1 && j == 0) ? g.rby * (Y(a, c) - Y(a, c - 2)) : 0.0f));
-  const float b_SE = (i < nx - 1 && j > 0) ? 0.0f
-                     : ((i == nx - 1 && j > 1) ? -g.rbx * (Y(a, c) - Y(a, c - 2 * nx))
-                        : ((i < nx - 2 && j == 0) ? g.rby * (Y(a, c + 2) - Y(a, c)) : 0.0f));
-  const float b_NW = (i > 0 && j < ny - 1) ? 0.0f
-                     : ((i == 0 && j < ny - 2) ? g.rbx * (Y(a, c + 2 * nx) - Y(a, c))
-                        : ((i > 1 && j == ny - 1) ? -g.rby * (Y(a, c) - Y(a, c - 2)) : 0.0f));
-  const float b_NE = (i < nx - 1 && j < ny - 1) ? 0.0f
-                     : ((i == nx - 1 && j < ny - 2) ? -g.rbx * (Y(a, c + 2 * nx) - Y(a, c))
-                        : ((i < nx - 2 && j == ny - 1) ? -g.rby * (Y(a, c + 2) - Y(a, c)) : 0.0f));
-  d += g.rxy * ((Y(a, SW) + b_SW) + (Y(a, NE) + b_NE) - (Y(a, SE) + b_SE) - (Y(a, NW) + b_NW)) * s;
+  d += g.rxy * ((Y(a, -1, -1) + b_SW) + (Y(a, 1, 1) + b_NE) - (Y(a, 1, -1) + b_SE) -
+                (Y(a, -1, 1) + b_NW)) * s;
   return d;
 }
 
-// Dirichlet neighbour (:362-373, :399-408, :434-437): the field inside the
-// domain where (with a mask) the cell and the neighbour are tissue, else the
-// boundary value.
-__device__ __forceinline__ float g_dir(const GParams& g, const StageField& Y, int a,
-                                       const uint8_t* solid, bool sc, int ni, int nj) {
-  if (ni < 0 || ni >= g.nx || nj < 0 || nj >= g.ny) return g.bval;
-  const int n = ni + g.nx * nj;
-  if (g.masked && !(sc && solid[n])) return g.bval;
-  return Y(a, n);
+// What a lane keeps of a cell for the whole launch.
+struct GenCell {
+  float y0[3], rhs[3], y[3], I[3];
+  float stim;
+  float cxx, cxy, cxz, cyx, cyy, cyz;  // G_MASKED: coefficients of :156-169
+  uint32_t flags;                      // kGenTissue, kGenOut, kGenSide + n
+};
+constexpr uint32_t kGenTissue = 1u, kGenOut = 2u;
+constexpr int kGenSide = 8;  // bits 8..15: neighbours W E N S SW NE SE NW usable (Dirichlet)
+
+// The neighbours of a cell: the stage field W E N S SW NE SE NW, and the
+// currents W E N S (lap4).
+template <int MODEL>
+struct GenNear {
+  typename GenPair<MODEL>::type y[8], j[4];
+};
+
+// Increment of variable a in one stage at a cell, diffusion only (:97-490).
+// Y2(a, dx, dy): the stage field two cells away (the anisotropic edges).
+template <int MODEL, int KIND, bool LAP4, class Y2F>
+__device__ __forceinline__ float g_diffusion(const GParams& g, const GenCell& q,
+                                             const GenNear<MODEL>& n, const Y2F& Y2, int a, int i,
+                                             int j, bool edges_x) {
+  using P = GenPair<MODEL>;
+  auto Y = [&](int k) { return P::get(n.y[k], a); };
+  auto J = [&](int k) { return P::get(n.j[k], a); };
+  const float c = q.y[a], I = q.I[a];
+  float d;
+  if (KIND == G_MASKED) {
+    // :154-185 (lap4 and the anisotropic term are not applied, as in the reference)
+    const float x = q.cxx * Y(0) - q.cxy * c + q.cxz * Y(1);
+    const float y = q.cyx * Y(2) - q.cyy * c + q.cyz * Y(3);
+    d = a == 0 ? x * g.rx + y * g.ry : x * g.rx * g.rscale + y * g.ry * g.rscale;
+  } else if (KIND == G_DIRICHLET) {
+    // :360-490: the field where the cell and the neighbour are tissue inside
+    // the domain, else the boundary value
+    auto B = [&](int k) { return ((q.flags >> (kGenSide + k)) & 1u) ? Y(k) : g.bval; };
+    const float x = B(0) - 2.0f * c + B(1), y = B(2) - 2.0f * c + B(3);
+    d = a == 0 ? x * g.rx + y * g.ry : x * g.rx * g.rscale + y * g.ry * g.rscale;
+    if (g.aniso) {
+      const float e = g.rxy * (B(4) + B(5) - B(6) - B(7));
+      d += a == 0 ? e : e * g.rscale;
+    }
+  } else {
+    // :188-199
+    const float W = Y(0), E = Y(1), N = Y(2), S = Y(3);
+    const float x = W - 2.0f * c + E, y = N - 2.0f * c + S;
+    d = a == 0 ? x * g.rx + y * g.ry : x * g.rx * g.rscale + y * g.ry * g.rscale;
+    if (LAP4) {
+      // :201-247; J = the neighbours' currents in this stage
+      const float z = (W - c + E) + (N - c + S);
+      const float diag = Y(4) + Y(6) + Y(7) + Y(5);
+      d += a == 0 ? -2.0f * g.q4 * z : -g.rscale * 2.0f * g.q4 * z;
+      d += a == 0 ? g.q4 * diag : g.rscale * g.q4 * diag;
+      d -= ((J(0) - 2.0f * I + J(1)) * g.fx4 + (J(2) - 2.0f * I + J(3)) * g.fy4);
+    }
+    if (KIND == G_ANISO || KIND == G_LAP4_ANISO) {
+      auto YA = [&](int b, int dx, int dy) {
+        return dx == 0 && dy == 0     ? c
+               : dx == -1 && dy == 0  ? W
+               : dx == 1 && dy == 0   ? E
+               : dx == 0 && dy == 1   ? N
+               : dx == 0 && dy == -1  ? S
+               : dx == -1 && dy == -1 ? Y(4)
+               : dx == 1 && dy == 1   ? Y(5)
+               : dx == 1 && dy == -1  ? Y(6)
+               : dx == -1 && dy == 1  ? Y(7)
+                                      : Y2(b, dx, dy);
+      };
+      d += g_aniso_neumann(g, YA, a, i, j, a == 0 ? 1.0f : g.rscale, edges_x);
+    }
+  }
+  return d;
 }
 
-// One Runge-Kutta stage (:114-503 for one rk4idx): increments d = F(y_s) of
-// every cell; rhs accumulates wsum*d (:501-502); the last stage writes
-// y0 + tc*rhs, zero in holes, and velTan = rhs/dt (:506-561).
-template <int MODEL>
-__global__ __launch_bounds__(256) void k_stage(GParams g, CFields y0, CFields dp, float ki,
-                                               float wsum, int first, int last, Fields dcur,
-                                               Fields rhs, Fields out, Fields vt,
-                                               const uint8_t* __restrict__ solid, ApdState apd,
-                                               int apd_on) {
+template <int MODEL, int KIND, bool APD>
+__global__ __launch_bounds__(kGenThreads) void k_general(
+    const GParams g, const GenRun r, CFields in, Fields out, Fields vt, float* __restrict__ prev,
+    const uint8_t* __restrict__ solid, const ApdState apd) {
   constexpr int NV = Model<MODEL>::NV;
-  const int i = blockIdx.x * 64 + threadIdx.x;
-  const int j = blockIdx.y * 4 + threadIdx.y;
-  if (i >= g.nx || j >= g.ny) return;
-  const int nx = g.nx, ny = g.ny, c = i + nx * j;
-  const StageField Y{y0, dp, ki};
-  const float u = Y(0, c), v = Y(1, c), w = NV > 2 ? Y(NV - 1, c) : 0.0f;
-  float Iu, Iv, Iw;
-  g_currents<MODEL>(g, u, v, w, i, j, Iu, Iv, Iw);
-  const bool vdiff = g.vdiff != 0;
-  float du = 0.0f, dv = 0.0f;
-  bool sc = true;
-  if (g.neumann) {
-    const int S = i + nx * mirror(j - 1, ny), N = i + nx * mirror(j + 1, ny);
-    const int W = mirror(i - 1, nx) + nx * j, E = mirror(i + 1, nx) + nx * j;
-    if (g.masked) {
-      // :154-185 (lap4 and the anisotropic term are not applied, as in the reference)
-      sc = solid[c] != 0;
-      const bool sw = solid[W] != 0, se = solid[E] != 0, sn = solid[N] != 0, ss = solid[S] != 0;
-      const float cxx = (sw && se) && (sw && sc) ? 1.0f : ((sw && sc) ? 2.0f : 0.0f);
-      const float cxy = sc ? ((sw || se) ? 2.0f : 0.0f) : 0.0f;
-      const float cxz = (sw && se) && (sc && se) ? 1.0f : ((sc && se) ? 2.0f : 0.0f);
-      const float cyx = (sn && ss) && (sn && sc) ? 1.0f : ((sn && sc) ? 2.0f : 0.0f);
-      const float cyy = sc ? ((sn || ss) ? 2.0f : 0.0f) : 0.0f;
-      const float cyz = (sn && ss) && (sc && ss) ? 1.0f : ((sc && ss) ? 2.0f : 0.0f);
-      du = (cxx * Y(0, W) - cxy * u + cxz * Y(0, E)) * g.rx + (cyx * Y(0, N) - cyy * u + cyz * Y(0, S)) * g.ry;
-      if (vdiff)
-        dv = (cxx * Y(1, W) - cxy * v + cxz * Y(1, E)) * g.rx * g.rscale
-           + (cyx * Y(1, N) - cyy * v + cyz * Y(1, S)) * g.ry * g.rscale;
-    } else {
-      // :188-199
-      du = (Y(0, W) - 2.0f * u + Y(0, E)) * g.rx + (Y(0, N) - 2.0f * u + Y(0, S)) * g.ry;
-      if (vdiff)
-        dv = (Y(1, W) - 2.0f * v + Y(1, E)) * g.rx * g.rscale + (Y(1, N) - 2.0f * v + Y(1, S)) * g.ry * g.rscale;
-      if (g.lap4) {
-        // :201-247; J of a neighbour = its current in this stage
-        int SW, SE, NW, NE;
-        g_diag(nx, ny, i, j, SW, SE, NW, NE);
-        float JW[3], JE[3], JN[3], JS[3];
-        const int iw = mirror(i - 1, nx), ie = mirror(i + 1, nx);
-        const int jn = mirror(j + 1, ny), js = mirror(j - 1, ny);
-        g_currents<MODEL>(g, Y(0, W), Y(1, W), NV > 2 ? Y(NV - 1, W) : 0.0f, iw, j, JW[0], JW[1], JW[2]);
-        g_currents<MODEL>(g, Y(0, E), Y(1, E), NV > 2 ? Y(NV - 1, E) : 0.0f, ie, j, JE[0], JE[1], JE[2]);
-        g_currents<MODEL>(g, Y(0, N), Y(1, N), NV > 2 ? Y(NV - 1, N) : 0.0f, i, jn, JN[0], JN[1], JN[2]);
-        g_currents<MODEL>(g, Y(0, S), Y(1, S), NV > 2 ? Y(NV - 1, S) : 0.0f, i, js, JS[0], JS[1], JS[2]);
-        du += -2.0f * g.q4 * ((Y(0, W) - u + Y(0, E)) + (Y(0, N) - u + Y(0, S)));
-        du += g.q4 * (Y(0, SW) + Y(0, SE) + Y(0, NW) + Y(0, NE));
-        du -= ((JW[0] - 2.0f * Iu + JE[0]) * g.fx4 + (JN[0] - 2.0f * Iu + JS[0]) * g.fy4);
-        if (vdiff) {
-          dv += -g.rscale * 2.0f * g.q4 * ((Y(1, W) - v + Y(1, E)) + (Y(1, N) - v + Y(1, S)));
-          dv += g.rscale * g.q4 * (Y(1, SW) + Y(1, SE) + Y(1, NW) + Y(1, NE));
-          dv -= ((JW[1] - 2.0f * Iv + JE[1]) * g.fx4 + (JN[1] - 2.0f * Iv + JS[1]) * g.fy4);
+  constexpr bool HOLES = KIND == G_MASKED || KIND == G_DIRICHLET;
+  using L = GenLds<MODEL, KIND>;
+  using P = GenPair<MODEL>;
+  __shared__ L lds;
+  const int tile = xcd_tile(blockIdx.x, r.ntiles);
+  const int ty = tile / r.tiles_x, tx = tile - ty * r.tiles_x;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nx = g.nx, ny = g.ny;
+  const int gx0 = tx * r.out_w - r.halo, gy0 = ty * r.out_h - r.halo;
+  const int gi = gx0 + lane;
+  const bool in_x = gi >= 0 && gi < nx;
+  // the region holds cells of a domain edge (or beyond it)
+  const bool edges_x = gx0 <= 0 || gx0 + 64 >= nx;
+  const bool edges = edges_x || gy0 <= 0 || gy0 + r.rows >= ny;
+  const bool vdiff = MODEL == M2V && g.vdiff != 0;
+  // this lane's cell of the wave's first row, two rows and columns before it,
+  // so every neighbour of every row lies at a constant offset >= 0
+  const int l0 = wave * kGenStride + lane;
+  auto off = [](int p, int dx, int dy) {
+    return (p * kGenWaves + kGenPad + dy) * kGenStride + kGenPad + dx;
+  };
+  GenCell q[kGenPer];
+
+  // The stage field (and currents) of row p's cell to LDS buffer b: at the
+  // cell and, with no-flux boundaries, at its mirror images outside the domain
+  // that lie in the region.
+  auto put = [&](int b, int p, int lr, int gj, const GenCell& c) __attribute__((always_inline)) {
+    const auto y = P::make(c.y[0], c.y[1]);
+    const auto J = P::make(c.I[0], c.I[1]);
+    auto at = [&](int dx, int dy) {
+      const int l = l0 + off(p, 0, 0) + dy * kGenStride + dx;
+      lds.y[b][l] = y;
+      if (L::LAP4) lds.j[L::LAP4 ? b : 0][L::LAP4 ? l : 0] = J;
+    };
+    at(0, 0);
+    if (KIND == G_DIRICHLET || !edges) return;
+    // a cell next to an edge cell is the mirror image of the one past the
+    // edge (helper_functions.cu:69-79)
+    const int dx = gi == 1 ? -2 : gi == nx - 2 ? 2 : 0;
+    const int dy = gj == 1 ? -2 : gj == ny - 2 ? 2 : 0;
+    const bool hx = dx != 0 && lane + dx >= 0 && lane + dx < 64;
+    const bool hy = dy != 0 && lr + dy >= 0 && lr + dy < r.rows;
+    if (hx) at(dx, 0);
+    if (hy) {
+      at(0, dy);
+      if (hx) at(dx, dy);
+    }
+  };
+  auto currents = [&](GenCell& c) __attribute__((always_inline)) {
+    g_currents<MODEL>(g, c.y[0], c.y[1], c.y[2], c.stim, c.I[0], c.I[1], c.I[2]);
+  };
+
+#pragma unroll
+  for (int p = 0; p < kGenPer; ++p) {
+    const int lr = wave + p * kGenWaves, gj = gy0 + lr;
+    GenCell& c = q[p];
+    c.flags = 0;
+    c.stim = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) c.y0[a] = c.rhs[a] = c.y[a] = c.I[a] = 0.0f;
+    if (lr < r.rows && gj >= 0 && gj < ny && in_x) {
+      const uint32_t idx = (uint32_t)gj * (uint32_t)nx + (uint32_t)gi;
+#pragma unroll
+      for (int a = 0; a < NV; ++a) c.y0[a] = c.y[a] = *at32(in.f[a], idx);
+      if (g.stim_on) {  // :54-61: radius^2 < 400 cells
+        const int di = gi - g.stim_x, dj = gj - g.stim_y;
+        if (di * di + dj * dj < 400) c.stim = 24.7f;
+      }
+      c.flags = kGenTissue;
+      if (lr >= r.halo && lr < r.halo + r.out_h && lane >= r.halo && lane < r.halo + r.out_w)
+        c.flags |= kGenOut;
+      if (KIND == G_MASKED) {
+        const bool sc = solid[idx] != 0;
+        const bool sw = solid[mirror(gi - 1, nx) + nx * gj] != 0;
+        const bool se = solid[mirror(gi + 1, nx) + nx * gj] != 0;
+        const bool sn = solid[gi + nx * mirror(gj + 1, ny)] != 0;
+        const bool ss = solid[gi + nx * mirror(gj - 1, ny)] != 0;
+        c.cxx = (sw && se) && (sw && sc) ? 1.0f : ((sw && sc) ? 2.0f : 0.0f);
+        c.cxy = sc ? ((sw || se) ? 2.0f : 0.0f) : 0.0f;
+        c.cxz = (sw && se) && (sc && se) ? 1.0f : ((sc && se) ? 2.0f : 0.0f);
+        c.cyx = (sn && ss) && (sn && sc) ? 1.0f : ((sn && sc) ? 2.0f : 0.0f);
+        c.cyy = sc ? ((sn || ss) ? 2.0f : 0.0f) : 0.0f;
+        c.cyz = (sn && ss) && (sc && ss) ? 1.0f : ((sc && ss) ? 2.0f : 0.0f);
+        if (!sc) c.flags &= ~kGenTissue;
+      }
+      if (KIND == G_DIRICHLET) {
+        const bool sc = !solid || solid[idx] != 0;
+        if (!sc) c.flags &= ~kGenTissue;
+        const int ox[8] = {-1, 1, 0, 0, -1, 1, 1, -1}, oy[8] = {0, 0, 1, -1, -1, 1, -1, 1};
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+          const int ni = gi + ox[n], nj = gj + oy[n];
+          const bool inside = ni >= 0 && ni < nx && nj >= 0 && nj < ny;
+          if (inside && sc && (!solid || solid[ni + nx * nj] != 0))
+            c.flags |= 1u << (kGenSide + n);
         }
       }
-      if (g.aniso) {
-        // :249-356
-        du += g_aniso_neumann(g, Y, 0, i, j, 1.0f);
-        if (vdiff) dv += g_aniso_neumann(g, Y, 1, i, j, g.rscale);
+      currents(c);
+      put(0, p, lr, gj, c);
+    }
+  }
+  __syncthreads();
+
+  const int T = r.K * r.order;
+  int st = 0, step = 0;
+  for (int t = 0; t < T; ++t) {
+    const int b = t & 1;
+    const bool last = st == r.order - 1, end = t == T - 1;
+    const float wsum = r.sw[st], ki = r.ki[st + 1];
+    const int lo = max(r.rad * (t + 1), -gy0), hi = min(r.rows - r.rad * (t + 1), ny - gy0);
+    const auto* yb = lds.y[b] + l0;
+    const auto* jb = lds.j[L::LAP4 ? b : 0] + (L::LAP4 ? l0 : 0);
+    // Row p + 1's neighbours are read from LDS before row p's arithmetic, so
+    // the LDS and the VALUs work at the same time (the reads are in bounds for
+    // rows that take no part, too): 18.8 -> 16.1 us a launch of 8 lap4 stages
+    // at 512 x 512.
+    GenNear<MODEL> near;
+    auto fetch = [&](int p) __attribute__((always_inline)) {
+      constexpr bool diag = L::LAP4 || KIND == G_ANISO || KIND == G_DIRICHLET;
+      const int ox[8] = {-1, 1, 0, 0, -1, 1, 1, -1}, oy[8] = {0, 0, 1, -1, -1, 1, -1, 1};
+      GenNear<MODEL> n = {};
+#pragma unroll
+      for (int k = 0; k < (diag ? 8 : 4); ++k) n.y[k] = yb[off(p, ox[k], oy[k])];
+      if (L::LAP4) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) n.j[k] = jb[L::LAP4 ? off(p, ox[k], oy[k]) : 0];
+      }
+      return n;
+    };
+    near = fetch(0);
+#pragma unroll
+    for (int p = 0; p < kGenPer; ++p) {
+      const GenNear<MODEL> n = near;
+      if (p + 1 < kGenPer) near = fetch(p + 1);
+      const int lr = wave + p * kGenWaves, gj = gy0 + lr;
+      if (lr < lo || lr >= hi) continue;
+      GenCell& c = q[p];
+      auto Y2 = [&](int a, int dx, int dy) { return P::get(yb[off(p, dx, dy)], a); };
+      const float u0 = c.y0[0];
+      // :498-499
+      float d[3];
+      d[0] = g_diffusion<MODEL, KIND, L::LAP4>(g, c, n, Y2, 0, gi, gj, edges_x) - g.dt * c.I[0];
+      d[1] = vdiff ? g_diffusion<MODEL, KIND, L::LAP4>(g, c, n, Y2, 1, gi, gj, edges_x) -
+                         g.dt * c.I[1]
+                   : 0.0f - g.dt * c.I[1];
+      d[2] = 0.0f - g.dt * c.I[2];
+      // :501-503; the last stage gives y0 + tc*rhs, zero in holes (:506-561)
+#pragma unroll
+      for (int a = 0; a < NV; ++a) c.rhs[a] = c.rhs[a] + wsum * d[a];
+      if (!last) {
+#pragma unroll
+        for (int a = 0; a < NV; ++a) c.y[a] = __builtin_fmaf(ki, d[a], c.y0[a]);
+      } else {
+        const bool sc = !HOLES || (c.flags & kGenTissue);
+#pragma unroll
+        for (int a = 0; a < NV; ++a) {
+          const float x = c.y0[a] + g.tc * c.rhs[a];
+          c.y0[a] = c.y[a] = sc ? x : 0.0f;
+        }
+        const bool owned = c.flags & kGenOut;
+        const uint32_t idx = (uint32_t)gj * (uint32_t)nx + (uint32_t)gi;
+        if (APD && owned && sc) {
+          float fr = apd.front[idx], bk = apd.back[idx], a1 = apd.apd1[idx], a2 = apd.apd2[idx];
+          uint32_t fi = apd.first[idx];
+          apd_cell(u0, c.y[0], apd.count0 + step + 1, apd.dt, apd.th, fr, bk, a1, a2, fi);
+          apd.front[idx] = fr;
+          apd.back[idx] = bk;
+          apd.apd1[idx] = a1;
+          apd.apd2[idx] = a2;
+          apd.first[idx] = (uint8_t)fi;
+        }
+        if (end && owned) {
+#pragma unroll
+          for (int a = 0; a < NV; ++a) {
+            *at32(out.f[a], idx) = c.y[a];
+            if (vt.f[0]) *at32(vt.f[a], idx) = sc ? c.rhs[a] / g.dt : 0.0f;
+          }
+          if (prev) *at32(prev, idx) = u0;
+        }
+#pragma unroll
+        for (int a = 0; a < NV; ++a) c.rhs[a] = 0.0f;
+      }
+      if (!end) {
+        currents(c);
+        if (in_x) put(b ^ 1, p, lr, gj, c);
       }
     }
-  } else {
-    // Dirichlet (:360-490)
-    sc = g.masked ? solid[c] != 0 : true;
-    du = (g_dir(g, Y, 0, solid, sc, i - 1, j) - 2.0f * u + g_dir(g, Y, 0, solid, sc, i + 1, j)) * g.rx
-       + (g_dir(g, Y, 0, solid, sc, i, j + 1) - 2.0f * u + g_dir(g, Y, 0, solid, sc, i, j - 1)) * g.ry;
-    if (vdiff)
-      dv = (g_dir(g, Y, 1, solid, sc, i - 1, j) - 2.0f * v + g_dir(g, Y, 1, solid, sc, i + 1, j)) * g.rx * g.rscale
-         + (g_dir(g, Y, 1, solid, sc, i, j + 1) - 2.0f * v + g_dir(g, Y, 1, solid, sc, i, j - 1)) * g.ry * g.rscale;
-    if (g.aniso) {
-      du += g.rxy * (g_dir(g, Y, 0, solid, sc, i - 1, j - 1) + g_dir(g, Y, 0, solid, sc, i + 1, j + 1)
-                     - g_dir(g, Y, 0, solid, sc, i + 1, j - 1) - g_dir(g, Y, 0, solid, sc, i - 1, j + 1));
-      if (vdiff)
-        dv += g.rxy * (g_dir(g, Y, 1, solid, sc, i - 1, j - 1) + g_dir(g, Y, 1, solid, sc, i + 1, j + 1)
-                       - g_dir(g, Y, 1, solid, sc, i + 1, j - 1) - g_dir(g, Y, 1, solid, sc, i - 1, j + 1)) * g.rscale;
-    }
-  }
-  // :498-499
-  float d[3];
-  d[0] = du - g.dt * Iu;
-  d[1] = dv - g.dt * Iv;
-  d[2] = -g.dt * Iw;
-#pragma unroll
-  for (int a = 0; a < NV; ++a) {
-    const float r = (first ? 0.0f : rhs.f[a][c]) + wsum * d[a];
+    if (!end) __syncthreads();
     if (last) {
-      const float x = y0.f[a][c] + g.tc * r;
-      out.f[a][c] = sc ? x : 0.0f;
-      if (vt.f[a]) vt.f[a][c] = sc ? r / g.dt : 0.0f;
+      st = 0;
+      ++step;
     } else {
-      rhs.f[a][c] = r;
-      dcur.f[a][c] = d[a];
+      ++st;
     }
-  }
-  if (last && apd_on && sc) {
-    const float u0 = y0.f[0][c];
-    const float un = out.f[0][c];
-    float fr = apd.front[c], bk = apd.back[c], a1 = apd.apd1[c], a2 = apd.apd2[c];
-    uint32_t fi = apd.first[c];
-    apd_cell(u0, un, apd.count0 + 1, apd.dt, apd.th, fr, bk, a1, a2, fi);
-    apd.front[c] = fr;
-    apd.back[c] = bk;
-    apd.apd1[c] = a1;
-    apd.apd2[c] = a2;
-    apd.first[c] = (uint8_t)fi;
   }
 }
 
-hipError_t launch_general_step(int model, const GParams& g, int order, CFields in, Fields out,
-                               Fields vt, const uint8_t* solid, float* const* scratch,
-                               hipStream_t s, const ApdState* apd) {
+// Cells a stage reads to each side.
+static int general_reach(const GParams& g) {
+  return g.neumann && !g.masked && g.aniso ? 2 : 1;
+}
+
+static int general_depth(const GParams& g, int order) {
+  return std::max(1, kGenHalo / (order * general_reach(g)));
+}
+
+// Steps to fuse (at most `steps`) and rows of a region on a device of `cus`
+// compute units: the pair with the least estimated time per step.  A launch
+// takes about 4 us before and after its stages and runs as many rounds as its
+// workgroups (16 waves, one a CU) fill; a row and stage costs c us on a CU.
+// More steps a launch pay its fixed part less often and recompute a wider
+// ring: RK4 with lap4 takes two steps a launch at 512 x 512 (17.3 against 2 x
+// 10.1 us, one round either way) and one at 1024 x 1024 (22.2 us, two rounds,
+// against 48.4, three).
+GenShape general_shape(int model, const GParams& g, int order, int steps, int cus) {
+  double c = model == M2V ? 0.025 : 0.05;
+  if (g.neumann && !g.masked) c += (g.lap4 ? 0.025 : 0.0) + (g.aniso ? 0.02 : 0.0);
+  const int rad = general_reach(g);
+  GenShape best{1, kGenRows};
+  double least = 1e300;
+  for (int K = 1; K <= std::min(steps, general_depth(g, order)); ++K) {
+    const int stages = K * order, halo = stages * rad, out_w = 64 - 2 * halo;
+    for (int rows = 8; rows <= kGenRows; rows += 4) {
+      const int out_h = rows - 2 * halo;
+      if (out_h < 1) continue;
+      const double tiles = (double)((g.nx + out_w - 1) / out_w) * ((g.ny + out_h - 1) / out_h);
+      double t = 0.5;
+      for (int s = 1; s <= stages; ++s) t += std::max(0.2, c * (rows - 2 * rad * s));
+      t = (4.0 + t * std::ceil(tiles / std::max(1, cus))) / K;
+      if (t < least) {
+        least = t;
+        best = GenShape{K, rows};
+      }
+    }
+  }
+  return best;
+}
+
+hipError_t launch_general(int model, const GParams& g, int order, GenShape shape, CFields in, Fields out,
+                          Fields vt, float* prev, const uint8_t* solid, hipStream_t s,
+                          const ApdState* apd) {
+  if (order != 1 && order != 2 && order != 4) return hipErrorInvalidValue;
+  const int K = shape.K;
+  if (K < 1 || K > general_depth(g, order) || shape.rows > kGenRows) return hipErrorInvalidValue;
   // :70-95, RK4 weights as the reference writes them
-  float ki[4] = {0.0f, 0.0f, 0.0f, 0.0f}, sw[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (order == 1) {
-    sw[0] = 1.0f;
-  } else if (order == 2) {
-    ki[1] = 0.5f;
-    sw[1] = 1.0f;
+  GenRun r = {};
+  r.K = K;
+  r.order = order;
+  r.sw[0] = 1.0f;
+  if (order == 2) {
+    r.ki[1] = 0.5f;
+    r.sw[0] = 0.0f;
+    r.sw[1] = 1.0f;
   } else if (order == 4) {
-    ki[1] = 0.5f;
-    ki[2] = 0.5f;
-    ki[3] = 1.0f;
-    sw[0] = 0.166666666666667f;
-    sw[1] = 0.333333333333333f;
-    sw[2] = 0.333333333333333f;
-    sw[3] = 0.166666666666667f;
-  } else {
-    return hipErrorInvalidValue;
+    r.ki[1] = r.ki[2] = 0.5f;
+    r.ki[3] = 1.0f;
+    r.sw[0] = r.sw[3] = 0.166666666666667f;
+    r.sw[1] = r.sw[2] = 0.333333333333333f;
   }
-  if (order > 1 && !scratch) return hipErrorInvalidValue;
-  // scratch: d ping-pong [0..2], [3..5]; rhs [6..8]
-  Fields dbuf[2] = {Fields{{nullptr, nullptr, nullptr}}, Fields{{nullptr, nullptr, nullptr}}};
-  Fields rhs{{nullptr, nullptr, nullptr}};
-  if (scratch) {
-    dbuf[0] = Fields{{scratch[0], scratch[1], scratch[2]}};
-    dbuf[1] = Fields{{scratch[3], scratch[4], scratch[5]}};
-    rhs = Fields{{scratch[6], scratch[7], scratch[8]}};
-  }
+  r.rad = general_reach(g);
+  r.halo = K * order * r.rad;
+  r.out_w = 64 - 2 * r.halo;
+  r.rows = shape.rows;
+  r.out_h = r.rows - 2 * r.halo;
+  if (r.out_w < 1 || r.out_h < 1) return hipErrorInvalidValue;
+  r.tiles_x = (g.nx + r.out_w - 1) / r.out_w;
+  r.ntiles = r.tiles_x * ((g.ny + r.out_h - 1) / r.out_h);
   const ApdState a = apd ? *apd : ApdState();
-  dim3 b(64, 4), gr((g.nx + 63) / 64, (g.ny + 3) / 4);
-  for (int st = 0; st < order; ++st) {
-    const Fields& dcur = dbuf[st & 1];
-    const Fields& dprev = dbuf[(st + 1) & 1];
-    CFields dp{{dprev.f[0], dprev.f[1], dprev.f[2]}};
-    if (st == 0) dp = in;  // ki[0] = 0: never read
-    const int first = st == 0, last = st == order - 1;
-    if (model == M2V)
-      hipLaunchKernelGGL(k_stage<M2V>, gr, b, 0, s, g, in, dp, ki[st], sw[st], first, last, dcur,
-                         rhs, out, vt, solid, a, apd ? 1 : 0);
-    else
-      hipLaunchKernelGGL(k_stage<MFK>, gr, b, 0, s, g, in, dp, ki[st], sw[st], first, last, dcur,
-                         rhs, out, vt, solid, a, apd ? 1 : 0);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(r.ntiles), dim3(kGenThreads), 0, s, g, r, in, out, vt, prev,
+                       solid, a);
+    return hipGetLastError();
+  };
+#define YH_GENERAL(KIND)                                                       \
+  return model == M2V ? (apd ? go(k_general<M2V, KIND, true>) : go(k_general<M2V, KIND, false>)) \
+                      : (apd ? go(k_general<MFK, KIND, true>) : go(k_general<MFK, KIND, false>))
+  if (!g.neumann) YH_GENERAL(G_DIRICHLET);
+  if (g.masked) YH_GENERAL(G_MASKED);
+  if (g.lap4 && g.aniso) YH_GENERAL(G_LAP4_ANISO);
+  if (g.lap4) YH_GENERAL(G_LAP4);
+  if (g.aniso) YH_GENERAL(G_ANISO);
+  YH_GENERAL(G_SQUARE);
+#undef YH_GENERAL
 }
 
 }  // namespace yh

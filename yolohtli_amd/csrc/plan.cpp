@@ -177,24 +177,25 @@ int plan_advance(yh_plan* pl, int nsteps, hipStream_t s) {
   int64_t done = pl->count;
   if (plan_general(pl)) {
     const int order = pl->p.timeIntOrder;
-    if (order > 1) {  // completes an allocation an earlier failure left partial
-      for (int q = 0; q < 9; ++q)
-        if (!pl->gscratch[q]) YH_HIP(hipMalloc(&pl->gscratch[q], pl->n * sizeof(float)));
-    }
     const GParams g = make_gparams(pl->p, pl->stim_on, pl->stim_x, pl->stim_y);
-    for (int q = 0; q < nsteps; ++q) {
+    if (!pl->prev_u) YH_HIP(hipMalloc(&pl->prev_u, pl->n * sizeof(float)));
+    while (remaining > 0) {
+      const GenShape shape = general_shape(pl->p.model, g, order, remaining, pl->cus);
+      const int K = shape.K;
       CFields ci;
       Fields co;
       fields(pl->cur, &ci, &co);
       apd.count0 = (int)done;
-      YH_HIP(launch_general_step(pl->p.model, g, order, ci, co, Fields{{nullptr, nullptr, nullptr}},
-                                 masked ? pl->solid_d : nullptr, order > 1 ? pl->gscratch : nullptr,
-                                 s, ap));
+      YH_HIP(launch_general(pl->p.model, g, order, shape, ci, co,
+                            Fields{{nullptr, nullptr, nullptr}},
+                            K == remaining ? pl->prev_u : nullptr,
+                            masked ? pl->solid_d : nullptr, s, ap));
       pl->cur ^= 1;
-      done += 1;
+      remaining -= K;
+      done += K;
     }
     pl->have_prev = true;
-    pl->past_prev_u = false;
+    pl->past_prev_u = true;
     pl->count += nsteps;
     return YH_OK;
   }
@@ -261,8 +262,6 @@ static void plan_free(yh_plan* pl) {
   for (void* q : apd)
     if (q) (void)hipFree(q);
   if (pl->sr) sr_free(pl->sr);
-  for (float* q : pl->gscratch)
-    if (q) (void)hipFree(q);
   void* cont[] = {pl->cont_pts, pl->cont_keys, pl->cont_count, pl->cont_area, pl->sapd};
   for (void* q : cont)
     if (q) (void)hipFree(q);
@@ -295,6 +294,9 @@ int yh_plan_create(const yh_params* p, yh_plan** out) {
   const size_t bytes = pl->n * sizeof(float);
   for (int b = 0; b < 2 && e == hipSuccess; ++b)
     for (int a = 0; a < pl->nv && e == hipSuccess; ++a) e = hipMalloc(&pl->buf[b][a], bytes);
+  // the general path keeps u of the step before the last on every call
+  if (e == hipSuccess && !standard_branch(*p) && p->timeIntOrder == 1)
+    e = hipMalloc(&pl->prev_u, bytes);
   if (e == hipSuccess) e = hipMalloc(&pl->tips_d, sizeof(yh_tip) * pl->tipcap);
   if (e == hipSuccess) e = hipMalloc(&pl->keys_d, sizeof(int) * pl->tipcap);
   if (e == hipSuccess) e = hipMalloc(&pl->tipcount_d, sizeof(int));

@@ -315,6 +315,7 @@ struct GParams {
   float mu, alpha, beta, gamma, delta, eps, theta;
   float u_c, u_v, u_csi, kk, tau_d, tau_r, tau_si, tau_0, tau_vp, tau_v1m, tau_v2m, tau_wp,
       tau_wm;
+  float tau_2si, r_d, r_r, r_2si, r_0, r_vp, r_v1m, r_v2m, r_wp, r_wm;  // 2 tau_si; reciprocals
   int stim_on, stim_x, stim_y;
 };
 GParams make_gparams(const yh_params& p, int stim_on, int stim_x, int stim_y);
@@ -324,11 +325,17 @@ GParams make_gparams(const yh_params& p, int stim_on, int stim_x, int stim_y);
 inline bool standard_branch(const yh_params& p) {
   return p.neumannBC && p.timeIntOrder == 1 && (p.solidSwitch || (!p.lap4 && !p.anisotropy));
 }
-// One step of the general path: `order` stage launches (1, 2 or 4); scratch
-// holds 9 device arrays of n floats (stage increments x2, rhs) when order > 1.
-hipError_t launch_general_step(int model, const GParams& g, int order, CFields in, Fields out,
-                               Fields vt, const uint8_t* solid, float* const* scratch,
-                               hipStream_t s, const ApdState* apd);
+// Steps one launch of the general path fuses and the rows of its regions.
+struct GenShape {
+  int K, rows;
+};
+GenShape general_shape(int model, const GParams& g, int order, int steps, int cus);
+// shape.K steps of the general path in one launch, from `in` to `out` (never
+// the same).  prev (may be null) receives u one step before the end, vt
+// (entries may be null) the last step's velocity; solid is null without a mask.
+hipError_t launch_general(int model, const GParams& g, int order, GenShape shape, CFields in,
+                          Fields out, Fields vt, float* prev, const uint8_t* solid,
+                          hipStream_t s, const ApdState* apd);
 
 // ------------------------------------------------------------- launchers
 hipError_t launch_codes(const uint8_t* solid, uint8_t* codes, int nx, int ny, hipStream_t s);
