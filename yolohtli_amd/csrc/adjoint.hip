@@ -44,9 +44,16 @@ struct AdjK {
 struct FkEval {
   float I, Gv, Gw;
   float dIdu, dIdv, dIdw, dGvdu, dGvdv, dGwdu, dGwdw;
-  float dI_dtau[4];  // tau_d, tau_r, tau_si, tau_0
-  float dGv_dtvp, dGw_dtwp;
+  float p, pc, Jfi, Jsi;  // what the time-constant derivatives are made of
 };
+
+// Correctly rounded 1/t: the hardware reciprocal (within 1 ulp) and one
+// Newton step by its exact residual (Markstein, IBM J. Res. Dev. 34(1), 1990;
+// equal to the quotient 1.0f/t for every significand), 3 instructions for 11.
+__device__ __forceinline__ float recip(float t) {
+  const float r = __builtin_amdgcn_rcpf(t);
+  return __builtin_fmaf(__builtin_fmaf(-t, r, 1.0f), r, r);
+}
 
 // s = sigmoid(2y) = 0.5*(1 + tanh y) and its complement sc = 1 - s, both
 // from a = exp(-2|y|) in (0, 1] with the hardware exp2 and reciprocal:
@@ -76,7 +83,7 @@ __device__ __forceinline__ void heav(float x, float iw, float tiw, float* h, flo
 // own, so the kernels that inline them agree bit for bit.  pc = 1 - p and
 // qc = 1 - q come from heav(); 1 + tanh(k(u - u_csi)) = 2 ss and
 // 1 - tanh^2 = 4 ss ssc with (ss, ssc) = sigmoid2(k(u - u_csi)).
-__device__ FkEval fk_eval(const AdjK& k, float u, float v, float w) {
+__device__ __forceinline__ FkEval fk_eval(const AdjK& k, float u, float v, float w) {
 #pragma clang fp contract(off)
   FkEval r;
   float p, pc, dp, q, qc, dq, ss, ssc;
@@ -96,7 +103,7 @@ __device__ FkEval fk_eval(const AdjK& k, float u, float v, float w) {
   r.dIdv = -p * f * k.itd;
   r.dIdw = -opth * k.ihtsi;
   const float tvm = qc * k.tv1m + q * k.tv2m;
-  const float itvm = 1.0f / tvm;
+  const float itvm = recip(tvm);
   const float dtvm = dq * (k.tv2m - k.tv1m);
   const float A = pc * (1.0f - v) * itvm - p * v * k.itvp;
   const float dAdu = -dp * (1.0f - v) * itvm - pc * (1.0f - v) * dtvm * (itvm * itvm) -
@@ -111,13 +118,25 @@ __device__ FkEval fk_eval(const AdjK& k, float u, float v, float w) {
   r.dGvdv = -dAdv;
   r.dGwdu = -dBdu;
   r.dGwdw = -dBdw;
-  r.dI_dtau[0] = -Jfi * k.itd;
-  r.dI_dtau[1] = -p * (k.itr * k.itr);
-  r.dI_dtau[2] = -2.0f * Jsi * k.ihtsi;
-  r.dI_dtau[3] = -u * pc * (k.it0 * k.it0);
-  r.dGv_dtvp = -p * v * (k.itvp * k.itvp);
-  r.dGw_dtwp = -p * w * (k.itwp * k.itwp);
+  r.p = p;
+  r.pc = pc;
+  r.Jfi = Jfi;
+  r.Jsi = Jsi;
   return r;
+}
+
+// The terms of dL/dtau (tau_d, tau_r, tau_si, tau_0, tau_v+, tau_w+) of one
+// cell and step, from mu, mv, mw = lambda of the step's result.
+__device__ __forceinline__ void fk_taus(const AdjK& k, const FkEval& r, float u, float v, float w,
+                                        float mu, float mv, float mw, float gt[6]) {
+#pragma clang fp contract(off)
+  const float tdt = k.tc * k.dt;
+  gt[0] = mu * (-tdt * (-r.Jfi * k.itd));
+  gt[1] = mu * (-tdt * (-r.p * (k.itr * k.itr)));
+  gt[2] = mu * (-tdt * (-2.0f * r.Jsi * k.ihtsi));
+  gt[3] = mu * (-tdt * (-u * r.pc * (k.it0 * k.it0)));
+  gt[4] = mv * (-tdt * (-r.p * v * (k.itvp * k.itvp)));
+  gt[5] = mw * (-tdt * (-r.p * w * (k.itwp * k.itwp)));
 }
 
 struct Coef4 {
@@ -153,22 +172,31 @@ __device__ __forceinline__ Coef4 coef_from_code(uint32_t b) {
 constexpr uint8_t kCodeAllOnes = 0x55;  // cW = cE = cN = cS = 1: no mask
 
 // ---------------------------------------------------------------- forward
-// One forward step of one cell from its state, its D, its four (mirror)
-// neighbours' u and D and its mask coefficients; shared by both forward
-// kernels, so they agree bit for bit.
-__device__ __forceinline__ void adj_fwd_cell(const AdjK& k, float u, float v, float w, float Dc,
-                                             float uW, float uE, float uN, float uS, float DW,
-                                             float DE, float DN, float DS, const Coef4& cf,
-                                             float& un, float& vn, float& wn) {
+// Diffusion weights of a cell, c * (D_c + D_n) / 2 per direction: constant
+// through the steps.
+struct AdjDif {
+  float W, E, N, S;
+};
+__device__ __forceinline__ AdjDif adj_dif(const Coef4& cf, float Dc, float DW, float DE, float DN,
+                                          float DS) {
 #pragma clang fp contract(off)
-  const float lap = k.rxh * (cf.W * 0.5f * (Dc + DW) * (uW - u) +
-                             cf.E * 0.5f * (Dc + DE) * (uE - u)) +
-                    k.ryh * (cf.N * 0.5f * (Dc + DN) * (uN - u) +
-                             cf.S * 0.5f * (Dc + DS) * (uS - u));
+  return AdjDif{cf.W * 0.5f * (Dc + DW), cf.E * 0.5f * (Dc + DE), cf.N * 0.5f * (Dc + DN),
+                cf.S * 0.5f * (Dc + DS)};
+}
+
+// One forward step of one cell from its state, its four (mirror) neighbours'
+// u and its diffusion weights; shared by both forward kernels, so they agree
+// bit for bit.
+__device__ __forceinline__ void adj_fwd_cell(const AdjK& k, float u, float v, float w, float uW,
+                                             float uE, float uN, float uS, const AdjDif& a,
+                                             bool tissue, float& un, float& vn, float& wn) {
+#pragma clang fp contract(off)
+  const float lap = k.rxh * (a.W * (uW - u) + a.E * (uE - u)) +
+                    k.ryh * (a.N * (uN - u) + a.S * (uS - u));
   const FkEval r = fk_eval(k, u, v, w);
-  un = cf.sc ? u + k.tc * (lap - k.dt * r.I) : 0.0f;
-  vn = cf.sc ? v + k.tc * (-k.dt * r.Gv) : 0.0f;
-  wn = cf.sc ? w + k.tc * (-k.dt * r.Gw) : 0.0f;
+  un = tissue ? u + k.tc * (lap - k.dt * r.I) : 0.0f;
+  vn = tissue ? v + k.tc * (-k.dt * r.Gv) : 0.0f;
+  wn = tissue ? w + k.tc * (-k.dt * r.Gw) : 0.0f;
 }
 
 __global__ __launch_bounds__(256) void k_adj_fwd(const AdjK k, CFields in, Fields out,
@@ -186,8 +214,8 @@ __global__ __launch_bounds__(256) void k_adj_fwd(const AdjK k, CFields in, Field
   const Coef4 cf = coef_of(codes, c);
   const float* U = in.f[0];
   float un, vn, wn;
-  adj_fwd_cell(k, U[c], in.f[1][c], in.f[2][c], D[c], U[W], U[E], U[N], U[S], D[W], D[E], D[N],
-               D[S], cf, un, vn, wn);
+  adj_fwd_cell(k, U[c], in.f[1][c], in.f[2][c], U[W], U[E], U[N], U[S],
+               adj_dif(cf, D[c], D[W], D[E], D[N], D[S]), cf.sc, un, vn, wn);
   out.f[0][c] = un;
   out.f[1][c] = vn;
   out.f[2][c] = wn;
@@ -197,96 +225,182 @@ __global__ __launch_bounds__(256) void k_adj_fwd(const AdjK k, CFields in, Field
   }
 }
 
-// K forward steps (K <= kAfKmax) of one kAfTX x kAfTY output tile through
-// LDS.  The tile's region is the output grown by K cells on each side and
-// clipped to the domain; mirror neighbours at the domain edge lie inside the
-// region, so in substep s only the cells s+1 away from region sides interior
-// to the domain lose an exact input and are skipped.  u is double-buffered
-// (neighbours read it); v and w are read by their own cell only and are
-// updated in place.  Outputs: with seg, the state after every substep into
-// seg slots slot0+1 .. slot0+K (the segment recompute); otherwise the final
-// state into out.  Sensor traces for every step with step % rec == 0.
-constexpr int kAfTX = 16, kAfTY = 16, kAfKmax = 8, kAfThreads = 1024;
-constexpr int kAfRN = (kAfTX + 2 * kAfKmax) * (kAfTY + 2 * kAfKmax);
+// ------------------------------------------------------------------ tiles
+// The tiled kernels run K <= kAdjKmax steps of an output tile of tw x th cells
+// (at most kAdjTile squared).  A cell at distance m from the tile (the larger
+// of its distances per axis, inside the domain) is needed exact after K - m
+// steps, so in step s (from 0) the cells with m <= K - 1 - s are computed.
+// One thread holds one cell for the whole launch, its state and coefficients
+// in registers; LDS carries only what neighbours read.  Threads are dealt out
+// in order of m, the tile first and then ring after ring, so the cells of a
+// step are the first threads and every later wave skips it whole: 8 steps of
+// a 16 x 16 tile take 73 wave-steps, against 92 with threads on a 32 x 32
+// square and 128 with every wave in every step.  Before, a step enumerated its
+// cells afresh with an integer division and modulus by run-time widths for
+// each, about as many instructions as the step itself.
+constexpr int kAdjTile = 16, kAdjKmax = 8, kAdjThreads = 1024;
+constexpr int kAdjStride = kAdjTile + 2 * kAdjKmax + 1;  // odd: columns spread over the banks
+constexpr int kAdjLds = kAdjStride * (kAdjTile + 2 * kAdjKmax);
+static_assert((kAdjTile + 2 * kAdjKmax) * (kAdjTile + 2 * kAdjKmax) <= kAdjThreads,
+              "one cell per thread");
 
-__global__ __launch_bounds__(kAfThreads) void k_adj_fwd_tiled(
+struct AdjTile {
+  int tiles_x, tw, th;
+};
+
+// Thread tid's cell: its coordinates and its ring m (K + 1: none, also where
+// the tile or its rings reach past the domain).
+struct AdjCell {
+  int x, y, m;
+};
+__device__ __forceinline__ AdjCell adj_cell(int tid, int ox0, int oy0, const AdjTile& t, int K,
+                                            int nx, int ny) {
+  int m = 0;
+  for (int q = 0; q <= K; ++q) m += tid >= (t.tw + 2 * q) * (t.th + 2 * q) ? 1 : 0;
+  int dx, dy;
+  if (m == 0) {
+    dy = tid / t.tw;
+    dx = tid - dy * t.tw;
+  } else {
+    // the ring's south row, north row, west and east column
+    const int W = t.tw + 2 * m, H = t.th + 2 * m - 2;
+    int p = tid - (W - 2) * H;
+    if (p < 2 * W) {
+      const bool north = p >= W;
+      dx = (north ? p - W : p) - m;
+      dy = north ? t.th + m - 1 : -m;
+    } else {
+      p -= 2 * W;
+      const bool east = p >= H;
+      dx = east ? t.tw + m - 1 : -m;
+      dy = (east ? p - H : p) - m + 1;
+    }
+  }
+  AdjCell c{ox0 + dx, oy0 + dy, m};
+  if (c.x < 0 || c.x >= nx || c.y < 0 || c.y >= ny) c.m = K + 1;
+  return c;
+}
+
+// A cell's place in LDS and its four neighbours' (mirrored at the domain edge,
+// helper_functions.cu:69-79).
+struct AdjAt {
+  int l, W, E, N, S;
+};
+__device__ __forceinline__ AdjAt adj_at(const AdjCell& c, int ox0, int oy0, int K, int nx,
+                                        int ny) {
+  const int l = (c.x - ox0 + K) + kAdjStride * (c.y - oy0 + K);
+  return AdjAt{l, c.x > 0 ? l - 1 : l + 1, c.x < nx - 1 ? l + 1 : l - 1,
+               c.y < ny - 1 ? l + kAdjStride : l - kAdjStride,
+               c.y > 0 ? l - kAdjStride : l + kAdjStride};
+}
+
+// K forward steps.  Outputs: with seg, the state after every step into seg
+// slots slot0+1 .. slot0+K (the segment recompute); otherwise the final state
+// into out.  Sensor traces for every step with step % rec == 0.
+template <bool MASKED>
+__global__ __launch_bounds__(kAdjThreads) void k_adj_fwd_tiled(
     const AdjK k, CFields in, Fields out, const float* __restrict__ D,
-    const uint8_t* __restrict__ codes, const int* __restrict__ smap, int K, int tiles_x,
-    int step0, int rec, float* __restrict__ traces, int ns, float* __restrict__ seg, size_t n,
-    int slot0) {
-  __shared__ float s_u[2][kAfRN];
-  __shared__ float s_v[kAfRN], s_w[kAfRN], s_D[kAfRN];
-  __shared__ uint8_t s_c[kAfRN];
-  __shared__ int s_sm[kAfRN];  // sensor slot of each region cell (-1: none), read once
+    const uint8_t* __restrict__ codes, const int* __restrict__ smap, int K, AdjTile t, int step0,
+    int rec, float* __restrict__ traces, int ns, float* __restrict__ seg, size_t n, int slot0) {
+  __shared__ float s_u[2][kAdjLds], s_D[kAdjLds];
   const int nx = k.nx, ny = k.ny;
-  const int tx = blockIdx.x % tiles_x, ty = blockIdx.x / tiles_x;
-  const int ox0 = tx * kAfTX, oy0 = ty * kAfTY;
-  const int ox1 = min(ox0 + kAfTX, nx), oy1 = min(oy0 + kAfTY, ny);
-  const int gx0 = max(ox0 - K, 0), gy0 = max(oy0 - K, 0);
-  const int gx1 = min(ox1 + K, nx), gy1 = min(oy1 + K, ny);
-  const int rw = gx1 - gx0, rn = rw * (gy1 - gy0);
-  for (int l = threadIdx.x; l < rn; l += kAfThreads) {
-    const size_t c = (size_t)(gx0 + l % rw) + (size_t)nx * (gy0 + l / rw);
-    s_u[0][l] = in.f[0][c];
-    s_v[l] = in.f[1][c];
-    s_w[l] = in.f[2][c];
-    s_D[l] = D[c];
-    s_c[l] = codes ? codes[c] : kCodeAllOnes;
-    s_sm[l] = traces ? smap[c] : -1;
+  const int ty = blockIdx.x / t.tiles_x, tx = blockIdx.x - ty * t.tiles_x;
+  const int ox0 = tx * t.tw, oy0 = ty * t.th;
+  const AdjCell q = adj_cell(threadIdx.x, ox0, oy0, t, K, nx, ny);
+  const AdjAt at = adj_at(q, ox0, oy0, K, nx, ny);
+  const size_t c = (size_t)q.x + (size_t)nx * q.y;
+  float u = 0.0f, v = 0.0f, w = 0.0f, Dc = 0.0f;
+  Coef4 cf{1.f, 1.f, 1.f, 1.f, true};
+  int sensor = -1;
+  if (q.m <= K) {
+    u = in.f[0][c];
+    v = in.f[1][c];
+    w = in.f[2][c];
+    Dc = D[c];
+    if (MASKED) cf = coef_from_code(codes[c]);
+    if (traces && q.m == 0) sensor = smap[c];
+    s_u[0][at.l] = u;
+    s_D[at.l] = Dc;
   }
   __syncthreads();
+  AdjDif a{};
+  if (q.m < K) a = adj_dif(cf, Dc, s_D[at.W], s_D[at.E], s_D[at.N], s_D[at.S]);
+  // the state after step step0 + s + 1, and the recorded steps to come: `left`
+  // steps to the next one, whose row is `row`
+  float* slot = seg ? seg + (size_t)(slot0 + 1) * 3 * n : nullptr;
+  int left = rec - step0 % rec;
+  float* row = traces ? traces + (size_t)(step0 / rec) * ns : nullptr;
   for (int s = 0; s < K; ++s) {
-    const int b = s & 1;
-    const int cx0 = gx0 > 0 ? gx0 + s + 1 : 0, cx1 = gx1 < nx ? gx1 - s - 1 : nx;
-    const int cy0 = gy0 > 0 ? gy0 + s + 1 : 0, cy1 = gy1 < ny ? gy1 - s - 1 : ny;
-    const int cw = cx1 - cx0, cn = cw * (cy1 - cy0);
-    const int step = step0 + s + 1;
-    float* row = (traces && step % rec == 0) ? traces + (size_t)(step / rec - 1) * ns : nullptr;
-    const float* U = s_u[b];
-    for (int q = threadIdx.x; q < cn; q += kAfThreads) {
-      const int gi = cx0 + q % cw, gj = cy0 + q / cw;
-      const int li = gi - gx0, lj = gj - gy0;
-      const int l = li + rw * lj;
-      const int lW = (mirror(gi - 1, nx) - gx0) + rw * lj;
-      const int lE = (mirror(gi + 1, nx) - gx0) + rw * lj;
-      const int lN = li + rw * (mirror(gj + 1, ny) - gy0);
-      const int lS = li + rw * (mirror(gj - 1, ny) - gy0);
+    const float* U = s_u[s & 1];
+    if (q.m < K - s) {
       float un, vn, wn;
-      adj_fwd_cell(k, U[l], s_v[l], s_w[l], s_D[l], U[lW], U[lE], U[lN], U[lS], s_D[lW],
-                   s_D[lE], s_D[lN], s_D[lS], coef_from_code(s_c[l]), un, vn, wn);
-      s_u[b ^ 1][l] = un;
-      s_v[l] = vn;
-      s_w[l] = wn;
-      if (gi >= ox0 && gi < ox1 && gj >= oy0 && gj < oy1) {
-        const size_t c = (size_t)gi + (size_t)nx * gj;
+      adj_fwd_cell(k, u, v, w, U[at.W], U[at.E], U[at.N], U[at.S], a, !MASKED || cf.sc, un, vn,
+                   wn);
+      u = un;
+      v = vn;
+      w = wn;
+      s_u[(s & 1) ^ 1][at.l] = u;
+      if (q.m == 0) {
         if (seg) {
-          float* base = seg + (size_t)(slot0 + s + 1) * 3 * n;
-          base[c] = un;
-          base[n + c] = vn;
-          base[2 * n + c] = wn;
+          slot[c] = u;
+          slot[n + c] = v;
+          slot[2 * n + c] = w;
         } else if (s == K - 1) {
-          out.f[0][c] = un;
-          out.f[1][c] = vn;
-          out.f[2][c] = wn;
+          out.f[0][c] = u;
+          out.f[1][c] = v;
+          out.f[2][c] = w;
         }
-        if (row) {
-          const int sm = s_sm[l];
-          if (sm >= 0) row[sm] = un;
-        }
+        if (left == 1 && sensor >= 0) row[sensor] = u;
       }
+    }
+    if (seg) slot += 3 * n;
+    if (--left == 0) {
+      left = rec;
+      if (traces) row += ns;
     }
     __syncthreads();
   }
 }
 
-static hipError_t launch_adj_fwd_tiled(const AdjK& k, CFields in, Fields out, const float* D,
-                                       const uint8_t* codes, const int* smap, int K, int step0,
-                                       int rec, float* traces, int ns, float* seg, size_t n,
-                                       int slot0, hipStream_t s) {
-  if (K < 1 || K > kAfKmax) return hipErrorInvalidValue;
-  const int tiles_x = (k.nx + kAfTX - 1) / kAfTX, tiles_y = (k.ny + kAfTY - 1) / kAfTY;
-  hipLaunchKernelGGL(k_adj_fwd_tiled, dim3(tiles_x * tiles_y), dim3(kAfThreads), 0, s, k, in,
-                     out, D, codes, smap, K, tiles_x, step0, rec, traces, ns, seg, n, slot0);
+// The output tile on a device of `cus` compute units, one workgroup a CU at a
+// time: the shape whose busiest CU computes the fewest cell-steps, rings
+// included (256 x 256: 16 x 16, 256 tiles; 128 x 128: 8 x 8, 256 tiles).
+static AdjTile adj_tile(int nx, int ny, int cus) {
+  const int shapes[4][2] = {{16, 16}, {16, 8}, {8, 8}, {8, 4}};
+  AdjTile best{};
+  double least = 1e300;
+  for (const auto& sh : shapes) {
+    const int tx = (nx + sh[0] - 1) / sh[0], ty = (ny + sh[1] - 1) / sh[1];
+    double work = 0.0;
+    for (int m = 0; m < kAdjKmax; ++m)  // waves over the four SIMDs of a CU, and a step's latency
+      work += 0.5 + std::ceil((sh[0] + 2 * m) * (sh[1] + 2 * m) / 256.0);
+    work *= std::ceil((double)tx * ty / std::max(1, cus));
+    if (work < least) {
+      least = work;
+      best = AdjTile{tx, sh[0], sh[1]};
+    }
+  }
+  return best;
+}
+static int adj_tiles(const AdjTile& t, int ny) { return t.tiles_x * ((ny + t.th - 1) / t.th); }
+
+// Threads of a launch: a cell each of the tile grown by K.
+static int adj_threads(const AdjTile& t, int K) {
+  return ((t.tw + 2 * K) * (t.th + 2 * K) + 63) / 64 * 64;
+}
+
+static hipError_t launch_adj_fwd_tiled(const AdjK& k, const AdjTile& t, CFields in, Fields out,
+                                       const float* D, const uint8_t* codes, const int* smap,
+                                       int K, int step0, int rec, float* traces, int ns,
+                                       float* seg, size_t n, int slot0, hipStream_t s) {
+  if (K < 1 || K > kAdjKmax) return hipErrorInvalidValue;
+  const dim3 g(adj_tiles(t, k.ny)), b(adj_threads(t, K));
+  if (codes)
+    hipLaunchKernelGGL(k_adj_fwd_tiled<true>, g, b, 0, s, k, in, out, D, codes, smap, K, t, step0,
+                       rec, traces, ns, seg, n, slot0);
+  else
+    hipLaunchKernelGGL(k_adj_fwd_tiled<false>, g, b, 0, s, k, in, out, D, codes, smap, K, t, step0,
+                       rec, traces, ns, seg, n, slot0);
   return hipGetLastError();
 }
 
@@ -344,10 +458,7 @@ __device__ __forceinline__ void adj_rev_cell(const AdjK& k, const Acc& A, int i,
   lv = -mu * tdt * r.dIdv + mv * (1.0f - tdt * r.dGvdv);
   lw = -mu * tdt * r.dIdw + mw * (1.0f - tdt * r.dGwdw);
   lu += src;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) gt[q] = mu * (-tdt * r.dI_dtau[q]);
-  gt[4] = mv * (-tdt * r.dGv_dtvp);
-  gt[5] = mw * (-tdt * r.dGw_dtwp);
+  fk_taus(k, r, u, v, w, mu, mv, mw, gt);
 }
 
 // Accessor over device fields (row stride nx, cell index c).
@@ -363,32 +474,49 @@ struct GlobalAcc {
   }
 };
 
-// The sum of gt over a workgroup of NT threads (FP64, fixed order), added to
-// the workgroup's slot.
+// v of the lane that DPP control CTRL names, 0 where it names none.
+template <int CTRL>
+__device__ __forceinline__ double dpp_double(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// Sum over the wave in lane 63, by shifts within rows of 16 lanes and
+// broadcasts of a row's last lane: VALU moves, no LDS round trips (with the
+// sums' old values read early, 15.2 -> 14.6 us a reverse launch against
+// ds_bpermute trees).
+__device__ __forceinline__ double wave_sum(double v) {
+  v += dpp_double<0x111>(v);  // row_shr:1
+  v += dpp_double<0x112>(v);  // row_shr:2
+  v += dpp_double<0x114>(v);  // row_shr:4
+  v += dpp_double<0x118>(v);  // row_shr:8
+  v += dpp_double<0x142>(v);  // row_bcast:15 (rows 1 and 3 take the row before)
+  v += dpp_double<0x143>(v);  // row_bcast:31 (rows 2 and 3 take the half before)
+  return v;
+}
+
+// The sums of gt over the first NT threads of a workgroup, those that hold any
+// (FP64, fixed order), added to the workgroup's slot, whose value before
+// (of threads 0 to 5) is `was`.
 template <int NT>
-__device__ __forceinline__ void adj_gtau_block(const double gt[6], double* slot) {
+__device__ __forceinline__ void adj_gtau_block(const double gt[6], double was, double* slot) {
   __shared__ double red[NT / 64][6];
+  const int waves = min(NT, (int)(blockDim.x * blockDim.y)) / 64;
   const int tid = threadIdx.y * blockDim.x + threadIdx.x;
   const int lane = tid & 63, wv = tid >> 6;
-  // the six shuffle trees interleaved level by level, so their latencies
-  // overlap; each value's adds keep their order
-  double v[6];
+  if (wv < waves) {
 #pragma unroll
-  for (int q = 0; q < 6; ++q) v[q] = gt[q];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-    for (int q = 0; q < 6; ++q) v[q] += __shfl_down(v[q], off, 64);
-  }
-  if (lane == 0) {
-#pragma unroll
-    for (int q = 0; q < 6; ++q) red[wv][q] = v[q];
+    for (int q = 0; q < 6; ++q) {
+      const double v = wave_sum(gt[q]);
+      if (lane == 63) red[wv][q] = v;
+    }
   }
   __syncthreads();
   if (tid < 6) {
     double s = 0.0;
-    for (int w = 0; w < NT / 64; ++w) s += red[w][tid];
-    slot[tid] += s;
+    for (int w = 0; w < waves; ++w) s += red[w][tid];
+    slot[tid] = was + s;
   }
 }
 
@@ -421,139 +549,197 @@ __global__ __launch_bounds__(256) void k_adj_rev(const AdjK k, CFields X, CField
 #pragma unroll
     for (int q = 0; q < 6; ++q) gtd[q] = (double)gt[q];
   }
-  adj_gtau_block<256>(gtd, gtau_part + (size_t)(blockIdx.y * gridDim.x + blockIdx.x) * 6);
+  double* slot = gtau_part + (size_t)(blockIdx.y * gridDim.x + blockIdx.x) * 6;
+  const int tid = threadIdx.y * blockDim.x + threadIdx.x;
+  adj_gtau_block<256>(gtd, tid < 6 ? slot[tid] : 0.0, slot);
 }
 
-// Accessor over an LDS region of row stride rw (cell index l).
-struct LdsAcc {
-  const float *Uf, *Df, *LUf;
-  const uint8_t* codes;
-  int l, rw;
-  __device__ float U(int di, int dj) const { return Uf[l + di + rw * dj]; }
-  __device__ float D(int di, int dj) const { return Df[l + di + rw * dj]; }
-  __device__ float LU(int di, int dj) const { return LUf[l + di + rw * dj]; }
-  __device__ uint32_t code(int di, int dj) const { return codes[l + di + rw * dj]; }
-};
-
-// K reverse steps (K <= kArKmax), n_top, n_top-1, ..., of one kArTX x kArTY
-// output tile through LDS; the region is the output grown by K and clipped
-// to the domain, as in the tiled forward (lambda has the same one-cell
-// dependence).  u of each step's state is staged in LDS (neighbours read
-// it); v and w of the cell come from the segment buffer.  lambda_u is
-// double-buffered, lambda_v and lambda_w are read by their own cell only and
-// updated in place.  dL/dD of the output cells accumulates over the K steps
-// in LDS (FP64) and is added once; dL/dtau per thread, then per workgroup.
-constexpr int kArTX = 16, kArTY = 16, kArKmax = 8, kArThreads = 1024;
-constexpr int kArRN = (kArTX + 2 * kArKmax) * (kArTY + 2 * kArKmax);
-
-__global__ __launch_bounds__(kArThreads) void k_adj_rev_tiled(
+// K reverse steps, n_top, n_top-1, ..., of one tile (see the tiles section; lambda has
+// the forward's one-cell dependence).  u of each step's state goes through LDS
+// (the neighbours of the tile's cells read it for dL/dD), lambda_u through a
+// double buffer.  A thread keeps its lambda_v, lambda_w, its row and column of
+// the transposed operator (constant through the steps), and, in the tile, its
+// dL/dD and dL/dtau sums (FP64).  u, v, w and the sensor source of a step are
+// loaded two steps ahead.  A step is bound by VALU issue: about 165
+// instructions a ring cell and 290 a tile cell, and 8 steps of a 16 x 16 tile
+// are 21 wave-steps on the busiest SIMD: 8 us of a 14.6 us launch at 256 x 256
+// (25.4 us with per-step index arithmetic; the forward 12.8 -> 9.2 us).
+template <bool MASKED>
+__global__ __launch_bounds__(kAdjThreads) void k_adj_rev_tiled(
     const AdjK k, const float* __restrict__ seg, const float* __restrict__ x0, size_t n,
-    int slot_top, int n_top, CFields lam_in,
-    Fields lam_out, const float* __restrict__ D, const uint8_t* __restrict__ codes,
-    const int* __restrict__ smap, const float* __restrict__ src, int rec, int ns,
-    double* __restrict__ gD, double* __restrict__ gtau_part, int K, int tiles_x) {
-  __shared__ float s_U[kArRN], s_D[kArRN], s_lu[2][kArRN], s_lv[kArRN], s_lw[kArRN];
-  __shared__ uint8_t s_c[kArRN];
-  __shared__ double s_gd[kArTX * kArTY];
+    int slot_top, int n_top, CFields lam_in, Fields lam_out, const float* __restrict__ D,
+    const uint8_t* __restrict__ codes, const int* __restrict__ smap,
+    const float* __restrict__ src, int rec, int ns, double* __restrict__ gD,
+    double* __restrict__ gtau_part, int K, AdjTile t) {
+#pragma clang fp contract(off)
+  __shared__ float s_U[2][kAdjLds], s_L[2][kAdjLds], s_D[kAdjLds];
+  __shared__ uint8_t s_c[MASKED ? kAdjLds : 1];
   const int nx = k.nx, ny = k.ny;
-  const int tx = blockIdx.x % tiles_x, ty = blockIdx.x / tiles_x;
-  const int ox0 = tx * kArTX, oy0 = ty * kArTY;
-  const int ox1 = min(ox0 + kArTX, nx), oy1 = min(oy0 + kArTY, ny);
-  const int gx0 = max(ox0 - K, 0), gy0 = max(oy0 - K, 0);
-  const int gx1 = min(ox1 + K, nx), gy1 = min(oy1 + K, ny);
-  const int rw = gx1 - gx0, rn = rw * (gy1 - gy0);
-  for (int l = threadIdx.x; l < rn; l += kArThreads) {
-    const size_t c = (size_t)(gx0 + l % rw) + (size_t)nx * (gy0 + l / rw);
-    s_D[l] = D[c];
-    s_c[l] = codes ? codes[c] : kCodeAllOnes;
-    s_lu[0][l] = lam_in.f[0][c];
-    s_lv[l] = lam_in.f[1][c];
-    s_lw[l] = lam_in.f[2][c];
-  }
-  for (int o = threadIdx.x; o < kArTX * kArTY; o += kArThreads) s_gd[o] = 0.0;
-  double gtd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  // A region has at most kArRN <= kArThreads cells, so thread t holds region
-  // cell t (u of the step's state) and computes the t-th cell of the step's
-  // shrinking region.  The values a step needs from global memory (u, the
-  // computed cell's v and w, its sensor source) are loaded one step ahead,
-  // during the previous step's arithmetic.
-  static_assert(kArRN <= kArThreads, "one region cell per thread");
-  const int tid = threadIdx.x;
+  const int ty = blockIdx.x / t.tiles_x, tx = blockIdx.x - ty * t.tiles_x;
+  const int ox0 = tx * t.tw, oy0 = ty * t.th;
+  const AdjCell q = adj_cell(threadIdx.x, ox0, oy0, t, K, nx, ny);
+  const AdjAt at = adj_at(q, ox0, oy0, K, nx, ny);
+  const size_t c = (size_t)q.x + (size_t)nx * q.y;
+  // tiles that hold cells next to an edge cell have mirror terms
+  const bool edges = ox0 - K <= 1 || oy0 - K <= 1 || ox0 + t.tw + K >= nx - 1 ||
+                     oy0 + t.th + K >= ny - 1;
+  const int sensor = src && q.m < K ? smap[c] : -1;
   struct Ahead {
     float u = 0.0f, v = 0.0f, w = 0.0f, src = 0.0f;
   };
   auto fetch = [&](int s) {
     Ahead a;
-    const float* X = slot_top - s == 0 ? x0 : seg + (size_t)(slot_top - s) * 3 * n;
-    if (tid < rn) a.u = X[(size_t)(gx0 + tid % rw) + (size_t)nx * (gy0 + tid / rw)];
-    const int cx0 = gx0 > 0 ? gx0 + s + 1 : 0, cx1 = gx1 < nx ? gx1 - s - 1 : nx;
-    const int cy0 = gy0 > 0 ? gy0 + s + 1 : 0, cy1 = gy1 < ny ? gy1 - s - 1 : ny;
-    const int cw = cx1 - cx0, cn = cw * (cy1 - cy0);
-    if (tid < cn) {
-      const size_t c = (size_t)(cx0 + tid % cw) + (size_t)nx * (cy0 + tid / cw);
+    if (s < K && q.m <= K - s) {
+      const float* X = slot_top - s == 0 ? x0 : seg + (size_t)(slot_top - s) * 3 * n;
+      a.u = X[c];
       a.v = X[n + c];
       a.w = X[2 * n + c];
       const int step = n_top - s;
-      if (src && step >= 1 && step % rec == 0) {
-        const int sm = smap[c];
-        if (sm >= 0) a.src = src[(size_t)(step / rec - 1) * ns + sm];
-      }
+      if (sensor >= 0 && step >= 1 && step % rec == 0)
+        a.src = src[(size_t)(step / rec - 1) * ns + sensor];
     }
     return a;
   };
-  Ahead next = fetch(0);
+  float Lu = 0.0f, Lv = 0.0f, Lw = 0.0f, Dc = 0.0f;
+  Coef4 cf{1.f, 1.f, 1.f, 1.f, true};
+  Ahead cur = fetch(0), next = fetch(1);
+  if (q.m <= K) {
+    Lu = lam_in.f[0][c];
+    Lv = lam_in.f[1][c];
+    Lw = lam_in.f[2][c];
+    Dc = D[c];
+    s_L[0][at.l] = Lu;
+    s_D[at.l] = Dc;
+    s_U[0][at.l] = cur.u;
+    if (MASKED) {
+      const uint32_t code = codes[c];
+      s_c[at.l] = (uint8_t)code;
+      cf = coef_from_code(code);
+    }
+  }
+  __syncthreads();
+  // own row: 1 - tc * sum of the weights.  Column: the weights with which the
+  // neighbours' updates read this cell, a = r c (D_c + D_n)/2, from the east,
+  // west, north, south neighbour, and x.. a second time from an edge cell,
+  // whose mirror neighbour this cell is.  h = c/2 for the dL/dD terms.
+  const float tc = k.tc;
+  float one = 0.0f, aE = 0.0f, aW = 0.0f, aN = 0.0f, aS = 0.0f, xE = 0.0f, xW = 0.0f, xN = 0.0f,
+        xS = 0.0f;
+  float hE = 0.0f, hW = 0.0f, hN = 0.0f, hS = 0.0f, yE = 0.0f, yW = 0.0f, yN = 0.0f, yS = 0.0f;
+  const float m = !MASKED || cf.sc ? 1.0f : 0.0f;
+  if (q.m < K) {
+    const float DW = s_D[at.W], DE = s_D[at.E], DN = s_D[at.N], DS = s_D[at.S];
+    float asum = 0.0f;
+    asum += k.rxh * cf.W * 0.5f * (Dc + DW);
+    asum += k.rxh * cf.E * 0.5f * (Dc + DE);
+    asum += k.ryh * cf.N * 0.5f * (Dc + DN);
+    asum += k.ryh * cf.S * 0.5f * (Dc + DS);
+    one = 1.0f - tc * asum;
+    Coef4 cE{1.f, 1.f, 1.f, 1.f, true}, cW = cE, cN = cE, cS = cE;
+    if (MASKED) {
+      cE = coef_from_code(s_c[at.E]);
+      cW = coef_from_code(s_c[at.W]);
+      cN = coef_from_code(s_c[at.N]);
+      cS = coef_from_code(s_c[at.S]);
+    }
+    auto weight = [&](bool there, float coef, float r, float Dn, float& a, float& h) {
+      a = there ? r * coef * 0.5f * (Dn + Dc) : 0.0f;
+      h = there ? coef * 0.5f : 0.0f;
+    };
+    weight(q.x + 1 < nx, cE.W, k.rxh, DE, aE, hE);
+    weight(q.x - 1 >= 0, cW.E, k.rxh, DW, aW, hW);
+    weight(q.y + 1 < ny, cN.S, k.ryh, DN, aN, hN);
+    weight(q.y - 1 >= 0, cS.N, k.ryh, DS, aS, hS);
+    weight(q.x == 1, cW.W, k.rxh, DW, xW, yW);
+    weight(q.x == nx - 2, cE.E, k.rxh, DE, xE, yE);
+    weight(q.y == 1, cS.S, k.ryh, DS, xS, yS);
+    weight(q.y == ny - 2, cN.N, k.ryh, DN, xN, yN);
+  }
+  // what the sums are added to at the end, read now
+  double* gt_slot = gtau_part + (size_t)blockIdx.x * 6;
+  const double gD_was = q.m == 0 ? gD[c] : 0.0;
+  const double gt_was = threadIdx.x < 6 ? gt_slot[threadIdx.x] : 0.0;
+  double gd = 0.0, gtd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   for (int s = 0; s < K; ++s) {
     const int b = s & 1;
-    const Ahead cur = next;
-    if (tid < rn) s_U[tid] = cur.u;
-    if (s + 1 < K) next = fetch(s + 1);
-    __syncthreads();
-    const int cx0 = gx0 > 0 ? gx0 + s + 1 : 0, cx1 = gx1 < nx ? gx1 - s - 1 : nx;
-    const int cy0 = gy0 > 0 ? gy0 + s + 1 : 0, cy1 = gy1 < ny ? gy1 - s - 1 : ny;
-    const int cw = cx1 - cx0, cn = cw * (cy1 - cy0);
-    if (tid < cn) {
-      const int gi = cx0 + tid % cw, gj = cy0 + tid / cw;
-      const int l = (gi - gx0) + rw * (gj - gy0);
-      LdsAcc A{s_U, s_D, s_lu[b], s_c, l, rw};
-      float lu, lv, lw, gt[6];
-      double gd;
-      adj_rev_cell(k, A, gi, gj, cur.v, cur.w, s_lv[l], s_lw[l], cur.src, lu, lv, lw, gd, gt);
-      s_lu[b ^ 1][l] = lu;
-      s_lv[l] = lv;
-      s_lw[l] = lw;
-      if (gi >= ox0 && gi < ox1 && gj >= oy0 && gj < oy1) {
-        s_gd[(gi - ox0) + kArTX * (gj - oy0)] += gd;
-#pragma unroll
-        for (int t = 0; t < 6; ++t) gtd[t] += (double)gt[t];
+    const Ahead then = fetch(s + 2);
+    if (q.m < K - s) {
+      const float* L = s_L[b];
+      const float LE = L[at.E], LW = L[at.W], LN = L[at.N], LS = L[at.S];
+      const float u = cur.u, v = cur.v, w = cur.w;
+      const float mu = m * Lu, mv = m * Lv, mw = m * Lw;
+      const float tE = tc * LE, tW = tc * LW, tN = tc * LN, tS = tc * LS;
+      float lin = tE * aE;
+      lin += tW * aW;
+      if (edges) {
+        lin += tW * xW;
+        lin += tE * xE;
       }
+      lin += tN * aN;
+      lin += tS * aS;
+      if (edges) {
+        lin += tS * xS;
+        lin += tN * xN;
+      }
+      const FkEval r = fk_eval(k, u, v, w);
+      const float tdt = tc * k.dt;
+      if (q.m == 0) {  // dL/dD and dL/dtau of the tile's cells
+        const float* U = s_U[b];
+        const float dE = U[at.E] - u, dW = U[at.W] - u, dN = U[at.N] - u, dS = U[at.S] - u;
+        const float tm = tc * mu, tx = tm * k.rxh, ty = tm * k.ryh;
+        gd += (double)(tx * (cf.W * 0.5f) * dW);
+        gd += (double)(tx * (cf.E * 0.5f) * dE);
+        gd += (double)(ty * (cf.N * 0.5f) * dN);
+        gd += (double)(ty * (cf.S * 0.5f) * dS);
+        gd -= (double)(tE * k.rxh * hE * dE);
+        gd -= (double)(tW * k.rxh * hW * dW);
+        gd -= (double)(tN * k.ryh * hN * dN);
+        gd -= (double)(tS * k.ryh * hS * dS);
+        if (edges) {
+          gd -= (double)(tW * k.rxh * yW * dW);
+          gd -= (double)(tE * k.rxh * yE * dE);
+          gd -= (double)(tS * k.ryh * yS * dS);
+          gd -= (double)(tN * k.ryh * yN * dN);
+        }
+        float gt[6];
+        fk_taus(k, r, u, v, w, mu, mv, mw, gt);
+#pragma unroll
+        for (int e = 0; e < 6; ++e) gtd[e] += (double)gt[e];
+      }
+      Lu = mu * (one - tdt * r.dIdu) + lin - mv * tdt * r.dGvdu - mw * tdt * r.dGwdu;
+      Lv = -mu * tdt * r.dIdv + mv * (1.0f - tdt * r.dGvdv);
+      Lw = -mu * tdt * r.dIdw + mw * (1.0f - tdt * r.dGwdw);
+      Lu += cur.src;
+      s_L[b ^ 1][at.l] = Lu;
     }
+    if (q.m <= 1) s_U[b ^ 1][at.l] = next.u;
+    cur = next;
+    next = then;
     __syncthreads();
   }
-  const float* LU = s_lu[K & 1];
-  const int ow = ox1 - ox0, on = ow * (oy1 - oy0);
-  for (int q = threadIdx.x; q < on; q += kArThreads) {
-    const int gi = ox0 + q % ow, gj = oy0 + q / ow;
-    const int l = (gi - gx0) + rw * (gj - gy0);
-    const size_t c = (size_t)gi + (size_t)nx * gj;
-    lam_out.f[0][c] = LU[l];
-    lam_out.f[1][c] = s_lv[l];
-    lam_out.f[2][c] = s_lw[l];
-    gD[c] += s_gd[(gi - ox0) + kArTX * (gj - oy0)];
+  if (q.m == 0) {
+    lam_out.f[0][c] = Lu;
+    lam_out.f[1][c] = Lv;
+    lam_out.f[2][c] = Lw;
+    gD[c] = gD_was + gd;
   }
-  adj_gtau_block<kArThreads>(gtd, gtau_part + (size_t)blockIdx.x * 6);
+  adj_gtau_block<kAdjTile * kAdjTile>(gtd, gt_was, gt_slot);
 }
 
-static hipError_t launch_adj_rev_tiled(const AdjK& k, const float* seg, const float* x0,
-                                       size_t n, int slot_top, int n_top, CFields li, Fields lo,
-                                       const float* D,
+static hipError_t launch_adj_rev_tiled(const AdjK& k, const AdjTile& t, const float* seg,
+                                       const float* x0, size_t n, int slot_top, int n_top,
+                                       CFields li, Fields lo, const float* D,
                                        const uint8_t* codes, const int* smap, const float* src,
                                        int rec, int ns, double* gD, double* gtau_part, int K,
                                        hipStream_t s) {
-  if (K < 1 || K > kArKmax) return hipErrorInvalidValue;
-  const int tiles_x = (k.nx + kArTX - 1) / kArTX, tiles_y = (k.ny + kArTY - 1) / kArTY;
-  hipLaunchKernelGGL(k_adj_rev_tiled, dim3(tiles_x * tiles_y), dim3(kArThreads), 0, s, k, seg, x0,
-                     n, slot_top, n_top, li, lo, D, codes, smap, src, rec, ns, gD, gtau_part, K,
-                     tiles_x);
+  if (K < 1 || K > kAdjKmax) return hipErrorInvalidValue;
+  const dim3 g(adj_tiles(t, k.ny)), b(adj_threads(t, K));
+  if (codes)
+    hipLaunchKernelGGL(k_adj_rev_tiled<true>, g, b, 0, s, k, seg, x0, n, slot_top, n_top, li, lo,
+                       D, codes, smap, src, rec, ns, gD, gtau_part, K, t);
+  else
+    hipLaunchKernelGGL(k_adj_rev_tiled<false>, g, b, 0, s, k, seg, x0, n, slot_top, n_top, li, lo,
+                       D, codes, smap, src, rec, ns, gD, gtau_part, K, t);
   return hipGetLastError();
 }
 
@@ -607,6 +793,7 @@ struct yh_adjoint {
   yh::AdjK k{};
   int fwdK = 8;  // steps per launch, forward and reverse: 1 = one-step kernels, else LDS-tiled
   int nparts = 0;  // dL/dtau workgroup slots: the larger of the two reverse grids
+  yh::AdjTile tile{};  // output tile of the tiled kernels
 };
 
 namespace yh {
@@ -711,8 +898,11 @@ int yh_adjoint_create(const yh_params* p, int nsteps, int rec_every, int ckpt_ev
   adj_k(a, tau6);
   const dim3 bg((p->nx + 63) / 64, (p->ny + 3) / 4);  // the 64 x 4 one-step blocks
   a->nblocks = bg.x * bg.y;
-  a->nparts = std::max(a->nblocks, ((p->nx + kArTX - 1) / kArTX) * ((p->ny + kArTY - 1) / kArTY));
-  hipError_t e = hipSuccess;
+  int dev = 0, cus = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  a->tile = adj_tile(p->nx, p->ny, cus);
+  a->nparts = std::max(a->nblocks, adj_tiles(a->tile, p->ny));
   auto M = [&](void** ptr, size_t bytes) {
     if (e == hipSuccess) e = hipMalloc(ptr, std::max<size_t>(bytes, 4));
   };
@@ -747,7 +937,7 @@ void yh_adjoint_destroy(yh_adjoint* a) {
 }
 
 int yh_adjoint_set_substeps(yh_adjoint* a, int k) {
-  if (!a || k < 1 || k > kAfKmax || k > kArKmax) return YH_EINVAL;
+  if (!a || k < 1 || k > kAdjKmax) return YH_EINVAL;
   a->fwdK = k;
   return YH_OK;
 }
@@ -813,7 +1003,7 @@ int yh_adjoint_forward(yh_adjoint* a, const float* d_D, const double tau6[6], vo
       hipLaunchKernelGGL(k_adj_fwd, bg, bb, 0, s, a->k, in, out, d_D, a->codes, a->smap, row);
       YH_HIP(hipGetLastError());
     } else {
-      YH_HIP(launch_adj_fwd_tiled(a->k, in, out, d_D, a->codes, a->smap, K, done, a->rec,
+      YH_HIP(launch_adj_fwd_tiled(a->k, a->tile, in, out, d_D, a->codes, a->smap, K, done, a->rec,
                                   a->traces, a->ns, nullptr, n, 0, s));
     }
     in = CFields{{out.f[0], out.f[1], out.f[2]}};
@@ -873,7 +1063,7 @@ int yh_adjoint_backward(yh_adjoint* a, void* stream, double* d_gD, double gtau[6
                            (float*)nullptr);
         YH_HIP(hipGetLastError());
       } else {  // slots t .. t+K-1
-        YH_HIP(launch_adj_fwd_tiled(a->k, in, out, a->D, a->codes, a->smap, K, s0 + t - 1,
+        YH_HIP(launch_adj_fwd_tiled(a->k, a->tile, in, out, a->D, a->codes, a->smap, K, s0 + t - 1,
                                     a->rec, nullptr, a->ns, a->seg, n, t - 1, s));
       }
       t += K;
@@ -895,7 +1085,7 @@ int yh_adjoint_backward(yh_adjoint* a, void* stream, double* d_gD, double gtau[6
         step -= 1;
       } else {  // steps step, step-1, ..., step-K+1 of this segment
         const int K = std::min(a->fwdK, t + 1);
-        YH_HIP(launch_adj_rev_tiled(a->k, a->seg, x0, n, t, step, li, lo, a->D, a->codes,
+        YH_HIP(launch_adj_rev_tiled(a->k, a->tile, a->seg, x0, n, t, step, li, lo, a->D, a->codes,
                                     a->smap, a->src, a->rec, a->ns, a->gD, a->gtau_part, K, s));
         step -= K;
       }
