@@ -344,8 +344,10 @@ int yh_batch_autotune(yh_batch* batch, int steps, void* stream, yh_kernel_cfg* b
 /* Gradient of loss = sum_{n % rec == 0} sum_s (u^n(sensor_s) - target)^2
  * through nsteps of the FK stepper with a spatial diffusion field D and the
  * tanh-smoothed Heaviside (params.heaviside_width > 0, model FK).  No
- * reference counterpart.  Checkpoints every ckpt_every steps; the reverse
- * sweep recomputes each segment.  Sensors are distinct cell indices. */
+ * reference counterpart.  Every state of the forward sweep is kept on the
+ * device where they take at most 4 GiB (and a quarter of its free memory);
+ * otherwise checkpoints every ckpt_every steps, from which the reverse sweep
+ * recomputes each segment.  Sensors are distinct cell indices. */
 typedef struct yh_adjoint yh_adjoint;
 int yh_adjoint_create(const yh_params* p, int nsteps, int rec_every, int ckpt_every,
                       const int* sensors, int nsensors, yh_adjoint** out);

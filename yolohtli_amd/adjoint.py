@@ -72,17 +72,20 @@ class SensorProblem:
 
     def forward(self, D, taus=None, stream=None):
         """D: contiguous float32 CUDA tensor of nx*ny cells.  Returns (loss, traces)."""
+        tr = np.empty((self.nrec, len(self.sensors)), np.float32)
+        return self._forward(D, taus, stream, tr), tr
+
+    def _forward(self, D, taus, stream, tr):
         taus = self.default_taus() if taus is None else np.asarray(taus, np.float64)
         if D.dtype.itemsize != 4 or not D.is_cuda or not D.is_contiguous():
             raise ValueError("D must be a contiguous float32 CUDA tensor")
-        tr = np.empty((self.nrec, len(self.sensors)), np.float32)
         loss = C.c_double()
         check(_protos().yh_adjoint_forward(self._h, D.data_ptr(), _ptr(np.ascontiguousarray(taus)),
                                            _stream_handle(stream), C.byref(loss), _ptr(tr)),
               "yh_adjoint_forward")
         self._gen += 1
         self._last = (D, taus.copy(), self._gen)
-        return loss.value, tr
+        return loss.value
 
     def backward(self, stream=None):
         """Gradient of the last forward's loss: (gD float64 CUDA tensor, gtau[6])."""
@@ -105,7 +108,7 @@ def _make_function():
         def forward(ctx, D, taus, problem):
             Dc = D.detach().contiguous().to(torch.float32)
             tv = taus.detach().to("cpu", torch.float64).numpy()
-            loss, _ = problem.forward(Dc, tv)
+            loss = problem._forward(Dc, tv, None, None)  # the traces stay on the device
             ctx.problem = problem
             ctx.gen = problem._gen
             ctx.Dc = Dc
@@ -117,7 +120,7 @@ def _make_function():
         def backward(ctx, gL):
             pr = ctx.problem
             if pr._gen != ctx.gen:  # another forward ran since: recompute this one
-                pr.forward(ctx.Dc, ctx.tv)
+                pr._forward(ctx.Dc, ctx.tv, None, None)
             gD, gt = pr.backward()
             g = gL.to(torch.float64)
             gD = (g * gD).to(ctx.Ddtype).view(ctx.Dshape)

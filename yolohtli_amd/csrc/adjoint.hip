@@ -14,9 +14,9 @@
 // lambda^{n+1}, gtau += (dF/dtau)^T lambda^{n+1}.  The transpose of the
 // mirrored, masked operator is applied in gather form: cell j collects the
 // coefficient of every (cell c, direction) whose neighbour is j, including the
-// two mirror images at each edge.  The forward keeps a checkpoint every
-// `ckpt` steps; each segment is recomputed into a buffer before its reverse
-// sweep.  gD and gtau accumulate in FP64 (gtau per workgroup, in a fixed
+// two mirror images at each edge.  The forward keeps every state where they
+// fit in 4 GiB; a longer run keeps a checkpoint every `ckpt` steps, and each
+// segment is recomputed into a buffer before its reverse sweep.  gD and gtau accumulate in FP64 (gtau per workgroup, in a fixed
 // order, so results are deterministic).
 #include <hip/hip_runtime.h>
 
@@ -295,8 +295,7 @@ __device__ __forceinline__ AdjAt adj_at(const AdjCell& c, int ox0, int oy0, int 
 }
 
 // K forward steps.  Outputs: with seg, the state after every step into seg
-// slots slot0+1 .. slot0+K (the segment recompute); otherwise the final state
-// into out.  Sensor traces for every step with step % rec == 0.
+// slots slot0+1 .. slot0+K; otherwise the final state into out.  Sensor traces for every step with step % rec == 0.
 template <bool MASKED>
 __global__ __launch_bounds__(kAdjThreads) void k_adj_fwd_tiled(
     const AdjK k, CFields in, Fields out, const float* __restrict__ D,
@@ -759,6 +758,27 @@ __global__ void k_adj_init(Fields lam, size_t n, const int* __restrict__ smap,
   }
 }
 
+// src = 2 (trace - target), the source of the reverse sweep, and the loss sum
+// (trace - target)^2 in FP64: per thread, then per wave, then per workgroup in
+// a fixed order, one partial a workgroup.
+constexpr int kLossBlocks = 64;
+__global__ __launch_bounds__(256) void k_adj_loss(const float* __restrict__ traces,
+                                                  const float* __restrict__ targets,
+                                                  float* __restrict__ src, size_t m,
+                                                  double* __restrict__ part) {
+  __shared__ double red[4];
+  double sum = 0.0;
+  for (size_t q = blockIdx.x * (size_t)256 + threadIdx.x; q < m; q += (size_t)kLossBlocks * 256) {
+    const double d = (double)traces[q] - (double)targets[q];
+    sum += d * d;
+    src[q] = (float)(2.0 * d);
+  }
+  sum = wave_sum(sum);
+  if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
 __global__ void k_fill_d(double* p, size_t n, double v) {
   for (size_t c = blockIdx.x * (size_t)blockDim.x + threadIdx.x; c < n;
        c += (size_t)gridDim.x * blockDim.x)
@@ -787,13 +807,16 @@ struct yh_adjoint {
   double* gD = nullptr;
   double* gtau_part = nullptr;
   int nblocks = 0;
-  std::vector<float> h_traces, h_targets;
+  double* loss_part = nullptr;  // kLossBlocks
   bool have_targets = false, forward_done = false;
   const float* D = nullptr;
   yh::AdjK k{};
   int fwdK = 8;  // steps per launch, forward and reverse: 1 = one-step kernels, else LDS-tiled
   int nparts = 0;  // dL/dtau workgroup slots: the larger of the two reverse grids
   yh::AdjTile tile{};  // output tile of the tiled kernels
+  // every state X^0 .. X^nsteps is kept (seg slots 0 .. nsteps), so the reverse
+  // sweep recomputes nothing; otherwise checkpoints every ckpt steps
+  bool keep = false;
 };
 
 namespace yh {
@@ -808,7 +831,7 @@ static void adj_free(yh_adjoint* a) {
   for (int q = 0; q < 3; ++q)
     if (a->X0[q]) (void)hipFree(a->X0[q]);
   void* ptrs[] = {a->ck, a->seg, a->smap, a->solid, a->codes, a->traces, a->targets, a->src,
-                  a->gD, a->gtau_part};
+                  a->gD, a->gtau_part, a->loss_part};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   delete a;
@@ -848,6 +871,9 @@ static void adj_k(yh_adjoint* a, const double tau6[6]) {
   k.itwp = (float)(1.0 / tau6[5]);
   k.itwm = (float)(1.0 / f.tau_wm);
 }
+
+// Most device memory a problem takes to keep every state of its forward sweep.
+constexpr size_t kAdjKeep = (size_t)4 << 30;
 
 static inline float* slot(float* base, size_t n, int s, int var) {
   return base + ((size_t)s * 3 + var) * n;
@@ -912,13 +938,30 @@ int yh_adjoint_create(const yh_params* p, int nsteps, int rec_every, int ckpt_ev
       M((void**)&a->lam[b][q], n * 4);
     }
   for (int q = 0; q < 3; ++q) M((void**)&a->X0[q], n * 4);
-  M((void**)&a->ck, (size_t)a->nckpt * 3 * n * 4);
-  M((void**)&a->seg, (size_t)(a->ckpt + 1) * 3 * n * 4);
+  // All states where they take at most kAdjKeep and a quarter of what is free
+  // on the device: recomputing each segment is a second forward sweep (2.4 of
+  // 9.0 ms per gradient at 256 x 256 x 2000, whose states are 1.6 GB of 288).
+  // If they cannot be had, the checkpoints the caller asked for.
+  const size_t all = (size_t)(nsteps + 1) * 3 * n * 4;
+  size_t avail = 0, total = 0;
+  if (e == hipSuccess && all <= kAdjKeep && hipMemGetInfo(&avail, &total) == hipSuccess &&
+      all <= avail / 4) {
+    a->keep = hipMalloc(&a->seg, all) == hipSuccess;
+    if (!a->keep) {
+      a->seg = nullptr;
+      (void)hipGetLastError();
+    }
+  }
+  if (!a->keep) {
+    M((void**)&a->ck, (size_t)a->nckpt * 3 * n * 4);
+    M((void**)&a->seg, (size_t)(a->ckpt + 1) * 3 * n * 4);
+  }
   M((void**)&a->smap, n * 4);
   M((void**)&a->traces, (size_t)a->nrec * a->ns * 4);
   M((void**)&a->targets, (size_t)a->nrec * a->ns * 4);
   M((void**)&a->src, (size_t)a->nrec * a->ns * 4);
   M((void**)&a->gD, n * 8);
+  M((void**)&a->loss_part, kLossBlocks * 8);
   M((void**)&a->gtau_part, (size_t)a->nparts * 6 * 8);
   if (e == hipSuccess) e = hipMemcpy(a->smap, smap.data(), n * 4, hipMemcpyHostToDevice);
   for (int q = 0; q < 3 && e == hipSuccess; ++q) e = hipMemset(a->X0[q], 0, n * 4);
@@ -966,7 +1009,6 @@ int yh_adjoint_set_initial(yh_adjoint* a, const float* u, const float* v, const 
 int yh_adjoint_set_targets(yh_adjoint* a, const float* targets) {
   if (!a || !targets) return YH_EINVAL;
   const size_t m = (size_t)a->nrec * a->ns;
-  a->h_targets.assign(targets, targets + m);
   YH_HIP(hipMemcpy(a->targets, targets, m * 4, hipMemcpyHostToDevice));
   a->have_targets = true;
   return YH_OK;
@@ -983,20 +1025,22 @@ int yh_adjoint_forward(yh_adjoint* a, const float* d_D, const double tau6[6], vo
   a->D = d_D;
   const size_t n = a->n;
   dim3 bb(64, 4), bg((a->p.nx + 63) / 64, (a->p.ny + 3) / 4);
-  // checkpoint 0 = X^0; a launch that ends on a later checkpoint step writes
-  // its state into that checkpoint, which the next launch reads
+  // X^0 to its slot.  With every state kept, launches write the state after
+  // each step into its slot; otherwise a launch that ends on a checkpoint step
+  // writes its state into that checkpoint, which the next launch reads.
+  float* x0 = a->keep ? a->seg : a->ck;
   for (int q = 0; q < 3; ++q)
-    YH_HIP(hipMemcpyAsync(slot(a->ck, n, 0, q), a->X0[q], n * 4, hipMemcpyDeviceToDevice, s));
-  CFields in{{slot(a->ck, n, 0, 0), slot(a->ck, n, 0, 1), slot(a->ck, n, 0, 2)}};
+    YH_HIP(hipMemcpyAsync(slot(x0, n, 0, q), a->X0[q], n * 4, hipMemcpyDeviceToDevice, s));
+  CFields in{{slot(x0, n, 0, 0), slot(x0, n, 0, 1), slot(x0, n, 0, 2)}};
   int nb = 0;  // the work buffer the next launch writes (never the one it reads)
   for (int done = 0; done < a->nsteps;) {
-    // launches end on every checkpoint step
-    const int K = std::min({a->fwdK, a->nsteps - done, (done / a->ckpt + 1) * a->ckpt - done});
+    int K = std::min(a->fwdK, a->nsteps - done);
+    if (!a->keep) K = std::min(K, (done / a->ckpt + 1) * a->ckpt - done);  // end on checkpoints
     const int end = done + K;
-    const bool to_ck = end % a->ckpt == 0 && end < a->nsteps;
-    const int ci = end / a->ckpt;
-    Fields out = to_ck ? Fields{{slot(a->ck, n, ci, 0), slot(a->ck, n, ci, 1), slot(a->ck, n, ci, 2)}}
-                       : Fields{{a->X[nb][0], a->X[nb][1], a->X[nb][2]}};
+    const bool to_ck = !a->keep && end % a->ckpt == 0 && end < a->nsteps;
+    float* to = a->keep ? slot(a->seg, n, end, 0) : to_ck ? slot(a->ck, n, end / a->ckpt, 0) : nullptr;
+    const Fields out = to ? Fields{{to, to + n, to + 2 * n}}
+                          : Fields{{a->X[nb][0], a->X[nb][1], a->X[nb][2]}};
     if (a->fwdK == 1) {
       const int step = done + 1;
       float* row = (step % a->rec == 0) ? a->traces + (size_t)(step / a->rec - 1) * a->ns : nullptr;
@@ -1004,28 +1048,26 @@ int yh_adjoint_forward(yh_adjoint* a, const float* d_D, const double tau6[6], vo
       YH_HIP(hipGetLastError());
     } else {
       YH_HIP(launch_adj_fwd_tiled(a->k, a->tile, in, out, d_D, a->codes, a->smap, K, done, a->rec,
-                                  a->traces, a->ns, nullptr, n, 0, s));
+                                  a->traces, a->ns, a->keep ? a->seg : nullptr, n, done, s));
     }
     in = CFields{{out.f[0], out.f[1], out.f[2]}};
-    if (!to_ck) nb ^= 1;
+    if (!to) nb ^= 1;
     done = end;
   }
   const size_t m = (size_t)a->nrec * a->ns;
-  a->h_traces.resize(m);
-  YH_HIP(hipMemcpyAsync(a->h_traces.data(), a->traces, m * 4, hipMemcpyDeviceToHost, s));
-  YH_HIP(hipStreamSynchronize(s));
-  if (traces) std::memcpy(traces, a->h_traces.data(), m * 4);
-  double L = 0.0;
+  double part[kLossBlocks] = {};
   if (a->have_targets) {
-    std::vector<float> src(m);
-    for (size_t q = 0; q < m; ++q) {
-      const double dlt = (double)a->h_traces[q] - (double)a->h_targets[q];
-      L += dlt * dlt;
-      src[q] = (float)(2.0 * dlt);
-    }
-    YH_HIP(hipMemcpyAsync(a->src, src.data(), m * 4, hipMemcpyHostToDevice, s));
-    YH_HIP(hipStreamSynchronize(s));
+    // on the device: the host's loop over the traces and their way there and
+    // back took 0.3 ms at 2000 records of 64 sensors
+    hipLaunchKernelGGL(k_adj_loss, dim3(kLossBlocks), dim3(256), 0, s, a->traces, a->targets,
+                       a->src, m, a->loss_part);
+    YH_HIP(hipGetLastError());
+    YH_HIP(hipMemcpyAsync(part, a->loss_part, sizeof part, hipMemcpyDeviceToHost, s));
   }
+  if (traces) YH_HIP(hipMemcpyAsync(traces, a->traces, m * 4, hipMemcpyDeviceToHost, s));
+  YH_HIP(hipStreamSynchronize(s));
+  double L = 0.0;
+  for (double q : part) L += q;
   if (loss) *loss = L;
   a->forward_done = true;
   return YH_OK;
@@ -1046,13 +1088,14 @@ int yh_adjoint_backward(yh_adjoint* a, void* stream, double* d_gD, double gtau[6
   Fields l0{{a->lam[0][0], a->lam[0][1], a->lam[0][2]}};
   hipLaunchKernelGGL(k_adj_init, dim3(256), dim3(256), 0, s, l0, n, (const int*)a->smap, srcN);
   YH_HIP(hipGetLastError());
-  for (int seg = a->nckpt - 1; seg >= 0; --seg) {
-    const int s0 = seg * a->ckpt;
-    const int s1 = std::min(N, s0 + a->ckpt);  // reverse steps n = s1-1 .. s0
-    // recompute X^{s0+1} .. X^{s1-1} into seg slots 1 .. s1-s0-1; X^{s0} is
-    // read from its checkpoint (slot 0 stands for it)
-    float* x0 = slot(a->ck, n, seg, 0);  // the checkpoint's three fields, n apart
-    for (int t = 1; t < s1 - s0;) {
+  const int span = a->keep ? N : a->ckpt;
+  for (int seg = (N + span - 1) / span - 1; seg >= 0; --seg) {
+    const int s0 = seg * span;
+    const int s1 = std::min(N, s0 + span);  // reverse steps n = s1-1 .. s0
+    // X^{s0}: its slot, or its checkpoint (slot 0 of the segment stands for it)
+    float* x0 = slot(a->keep ? a->seg : a->ck, n, seg, 0);
+    // with checkpoints, recompute X^{s0+1} .. X^{s1-1} into seg slots 1 .. s1-s0-1
+    for (int t = 1; !a->keep && t < s1 - s0;) {
       CFields in = t == 1 ? CFields{{x0, x0 + n, x0 + 2 * n}}
                           : CFields{{slot(a->seg, n, t - 1, 0), slot(a->seg, n, t - 1, 1),
                                      slot(a->seg, n, t - 1, 2)}};
