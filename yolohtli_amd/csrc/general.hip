@@ -471,16 +471,7 @@ __global__ __launch_bounds__(kGenThreads) void k_general(
         }
         const bool owned = c.flags & kGenOut;
         const uint32_t idx = (uint32_t)gj * (uint32_t)nx + (uint32_t)gi;
-        if (APD && owned && sc) {
-          float fr = apd.front[idx], bk = apd.back[idx], a1 = apd.apd1[idx], a2 = apd.apd2[idx];
-          uint32_t fi = apd.first[idx];
-          apd_cell(u0, c.y[0], apd.count0 + step + 1, apd.dt, apd.th, fr, bk, a1, a2, fi);
-          apd.front[idx] = fr;
-          apd.back[idx] = bk;
-          apd.apd1[idx] = a1;
-          apd.apd2[idx] = a2;
-          apd.first[idx] = (uint8_t)fi;
-        }
+        if (APD && owned && sc) apd_cell(apd, idx, u0, c.y[0], apd.count0 + step + 1);
         if (end && owned) {
 #pragma unroll
           for (int a = 0; a < NV; ++a) {

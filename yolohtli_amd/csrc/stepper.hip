@@ -101,16 +101,7 @@ __global__ __launch_bounds__(256) void k_direct_codes(const KParams k, CFields i
   const bool sc = cell_update_codes<MODEL>(k, in.f, codes, i, j, xo, inc);
 #pragma unroll
   for (int a = 0; a < M::NV; ++a) out.f[a][c] = xo[a];
-  if (APD && sc) {
-    float fr = apd.front[c], bk = apd.back[c], d1 = apd.apd1[c], d2 = apd.apd2[c];
-    uint32_t fs = apd.first[c];
-    apd_cell(in.f[0][c], xo[0], apd.count0 + 1, apd.dt, apd.th, fr, bk, d1, d2, fs);
-    apd.front[c] = fr;
-    apd.back[c] = bk;
-    apd.apd1[c] = d1;
-    apd.apd2[c] = d2;
-    apd.first[c] = (uint8_t)fs;
-  }
+  if (APD && sc) apd_cell(apd, (uint32_t)c, in.f[0][c], xo[0], apd.count0 + 1);
 }
 
 hipError_t launch_direct(int model, const KParams& k, CFields in, Fields out, Fields vt,
@@ -201,14 +192,17 @@ static hipError_t launch_tiled_m(int rows, int waves, int cols, int K, const KPa
   const ApdState a = apd ? *apd : ApdState();
   if (apd) {
     if (prev) return hipErrorInvalidValue;
+#define YH_TILE_APD_I(RR, WW, I) \
+  launch_tiled_t<MODEL, MASKED, RR, WW, 1, true, false, I>(K, k, in, out, codes, s, a, nullptr, occ)
 #define YH_TILE_APD(RR, WW)                    \
   if (rows == RR && waves == WW && cols == 1) \
-    return launch_tiled_t<MODEL, MASKED, RR, WW, 1, true>(K, k, in, out, codes, s, a, nullptr, occ);
+    return k.iso ? YH_TILE_APD_I(RR, WW, 1) : YH_TILE_APD_I(RR, WW, -1);
     YH_TILE_APD(4, 8)
     YH_TILE_APD(8, 8)
     YH_TILE_APD(4, 16)
     YH_TILE_APD(8, 16)
 #undef YH_TILE_APD
+#undef YH_TILE_APD_I
     return hipErrorInvalidValue;
   }
   // the shapes the automatic choice takes (7 x 16 and the 8 x 16 its

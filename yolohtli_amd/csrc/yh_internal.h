@@ -77,25 +77,37 @@ struct ApdState {
   int count0 = 0;    // step count before the launch
 };
 
-// One sAPD update (spaceAPD.cu:328-358, stimulus off) for a cell going from
-// uo to un at step `count`.
-__device__ __forceinline__ void apd_cell(float uo, float un, int count, float dt, float th,
-                                         float& front, float& back, float& apd1, float& apd2,
-                                         uint32_t& first) {
-  if ((un > th) && (uo < th)) front = dt * ((float)count - (un - th) / (un - uo));
-  if ((un < th) && (uo > th)) back = dt * ((float)count - (un - th) / (un - uo));
-  if ((back > 0.0f) && (front > 0.0f) && (first == 0u)) {
-    apd1 = back - front;
-    front = 0.0f;
-    back = 0.0f;
-    first = 1u;
+// Whether u crosses th from uo to un.
+__device__ __forceinline__ bool apd_crosses(float uo, float un, float th) {
+  return (un > th && uo < th) || (un < th && uo > th);
+}
+// The sAPD update (spaceAPD.cu:328-358, stimulus off) of a cell whose u crosses
+// th from uo to un at step `count`; without a crossing nothing changes, since
+// a duration is formed as soon as front and back are both set.  Returns
+// whether this completed the duration d.
+__device__ __forceinline__ bool apd_crossing(float uo, float un, int count, float dt, float th,
+                                             float& front, float& back, float& d) {
+  const float t = dt * ((float)count - (un - th) / (un - uo));
+  if (un > th) front = t;
+  else back = t;
+  d = back - front;
+  if (!((back > 0.0f) && (front > 0.0f))) return false;
+  front = 0.0f;
+  back = 0.0f;
+  return true;
+}
+// The update of cell idx in memory: durations go to apd1 and apd2 in turn.
+__device__ __forceinline__ void apd_cell(const ApdState& a, uint32_t idx, float uo, float un,
+                                         int count) {
+  if (!apd_crosses(uo, un, a.th)) return;
+  float front = a.front[idx], back = a.back[idx], d;
+  if (apd_crossing(uo, un, count, a.dt, a.th, front, back, d)) {
+    const uint8_t first = a.first[idx];
+    (first ? a.apd2 : a.apd1)[idx] = d;
+    a.first[idx] = first ? 0 : 1;
   }
-  if ((back > 0.0f) && (front > 0.0f) && (first != 0u)) {
-    apd2 = back - front;
-    front = 0.0f;
-    back = 0.0f;
-    first = 0u;
-  }
+  a.front[idx] = front;
+  a.back[idx] = back;
 }
 
 // ----------------------------------------------------------------- models
