@@ -24,8 +24,8 @@ HIPFLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function", "-Wno-unused-command-line-argument",
 ]
-SOURCES = ["api.cpp", "plan.cpp", "autotune.cpp", "stepper.hip", "sr.hip", "batch.hip",
-           "adjoint.hip", "io.cpp", "general.hip", "contour.hip", "noalloc.hip"]
+SOURCES = ["tiled_fk.hip", "tiled_2v.hip", "batch.hip", "api.cpp", "plan.cpp", "autotune.cpp",
+           "stepper.hip", "sr.hip", "adjoint.hip", "io.cpp", "general.hip", "contour.hip", "noalloc.hip"]
 
 
 def _compile(src):

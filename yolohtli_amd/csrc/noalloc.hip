@@ -91,31 +91,39 @@ int yh_step_noalloc(const yh_params* p, float* const out[3], const float* const 
   if (masked) YH_HIP(launch_codes(solid, codes, p->nx, p->ny, s));
   KParams k;
   make_kparams(*p, d, &k);
-  // the kernel a plan left on YH_KERNEL_AUTO runs, with the plan's store
-  // policy per launch (neither the remainder merge nor the store policy
-  // changes a value: the result does not depend on where launches split,
-  // so it equals yh_step's bit for bit)
-  const bool pairs = tiled_per_cu(p->model, masked, k, 4, 16, 1, false) >= 2;
+  // the launches of a plan left on YH_KERNEL_AUTO, with its store policy
+  // (neither the split, the remainder merge it may use nor the store policy
+  // changes a value: the result does not depend on where launches split, so it
+  // equals yh_step's bit for bit)
+  const bool pairs = tiled_per_cu(p->model, masked, k, 4, 16, 1, false, false) >= 2;
   const yh_kernel_cfg c = auto_cfg(p->nx, p->ny, cus, pairs);
-  const int per_cu = tiled_per_cu(p->model, masked, k, c.rows, c.waves, c.cols, false);
-  const int K = c.substeps;
-  const int launches = (nsteps + K - 1) / K;
+  AutoTable t;
+  auto_table(p->model, masked, k, cus, false, &t);
+  const bool split = auto_wins(t, p->model, masked, k, cus, c, false, nsteps);
+  auto next = [&](int remaining) {
+    yh_kernel_cfg l = split ? auto_next(t, remaining) : c;
+    l.substeps = std::min(l.substeps, remaining);
+    return l;
+  };
+  int launches = 0;
+  for (int r = nsteps; r > 0; r -= next(r).substeps) ++launches;
   // launch i writes `out` when launches - 1 - i is even, else the scratch
   // state, so the last one writes `out` and no launch reads what it writes
   const float* src[3] = {in[0], in[1], nv == 3 ? in[2] : nullptr};
   int remaining = nsteps;
   for (int i = 0; i < launches; ++i) {
     float* const* dst = ((launches - 1 - i) % 2 == 0) ? out : mid;
-    const int steps = std::min(K, remaining);
+    const yh_kernel_cfg l = next(remaining);
     CFields ci{{src[0], src[1], src[2]}};
     Fields co{{dst[0], dst[1], nv == 3 ? dst[2] : nullptr}};
     KParams kl = k;
     kl.wt = tiled_write_through(
-        tiled_tile_count(p->nx, p->ny, c.rows, c.waves, c.cols, steps), cus, per_cu);
-    YH_HIP(launch_tiled(p->model, masked, c.rows, c.waves, c.cols, steps, kl, ci, co,
+        tiled_tile_count(p->nx, p->ny, l.rows, l.waves, l.cols, l.substeps), cus,
+        tiled_per_cu(p->model, masked, k, l.rows, l.waves, l.cols, false, false));
+    YH_HIP(launch_tiled(p->model, masked, l.rows, l.waves, l.cols, l.substeps, kl, ci, co,
                         masked ? codes : nullptr, s));
     for (int a = 0; a < 3; ++a) src[a] = co.f[a];
-    remaining -= steps;
+    remaining -= l.substeps;
   }
   return YH_OK;
 }

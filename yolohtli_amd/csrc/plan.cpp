@@ -62,34 +62,36 @@ yh_kernel_cfg auto_cfg(int nx, int ny, int cus, bool pairs) {
 }
 
 // Workgroups of the tiled kernel of this shape (model, mask, the isotropy
-// of k, with or without the previous-u output) that one CU holds at once
-// (its occupancy), cached per instantiation in a fixed table, so neither
-// the query nor the cache allocates (the no-allocation entry point uses it).
+// of k, with or without the previous-u output or the APD update) that one CU
+// holds at once (its occupancy), cached per instantiation in a fixed table, so
+// neither the query nor the cache allocates (the no-allocation entry point
+// uses it).
 int tiled_per_cu(int model, bool masked, const KParams& k, int rows, int waves, int cols,
-                 bool prev) {
+                 bool prev, bool apd) {
   struct Entry {
-    int key[7];
+    int key[8];
     int n;
   };
   static std::mutex mu;
   static Entry table[256];
   static int used = 0;
-  const int key[7] = {model, masked ? 1 : 0, k.iso, rows, waves, cols, prev ? 1 : 0};
+  const int key[8] = {model, masked ? 1 : 0, k.iso, rows, waves, cols, prev ? 1 : 0, apd ? 1 : 0};
   {
     std::lock_guard<std::mutex> g(mu);
     for (int e = 0; e < used; ++e)
-      if (std::equal(key, key + 7, table[e].key)) return table[e].n;
+      if (std::equal(key, key + 8, table[e].key)) return table[e].n;
   }
   static float dummy;  // selects the previous-u instantiation; never written in a query
+  const ApdState none;  // selects the APD instantiation
   int n = 0;
   if (launch_tiled(model, masked, rows, waves, cols, 1, k, CFields{{nullptr, nullptr, nullptr}},
-                   Fields{{nullptr, nullptr, nullptr}}, nullptr, nullptr, nullptr,
+                   Fields{{nullptr, nullptr, nullptr}}, nullptr, nullptr, apd ? &none : nullptr,
                    prev ? &dummy : nullptr, &n) != hipSuccess ||
       n < 1)
     n = 1;
   std::lock_guard<std::mutex> g(mu);
   if (used < 256) {  // every instantiation fits; past that, query again
-    std::copy(key, key + 7, table[used].key);
+    std::copy(key, key + 8, table[used].key);
     table[used].n = n;
     ++used;
   }
@@ -97,7 +99,90 @@ int tiled_per_cu(int model, bool masked, const KParams& k, int rows, int waves, 
 }
 
 static int tiled_per_cu(const yh_plan* pl, int rows, int waves, int cols, bool prev) {
-  return tiled_per_cu(pl->p.model, pl->p.solidSwitch != 0, pl->k, rows, waves, cols, prev);
+  return tiled_per_cu(pl->p.model, pl->p.solidSwitch != 0, pl->k, rows, waves, cols, prev, false);
+}
+
+// ------------------------------------------------------- launches of a call
+// Estimated time (us) of one launch of K substeps on a rows x waves shape of
+// one column per lane, `per_cu` workgroups of which fit on a CU.  The busiest
+// CU runs L workgroups in b batches.  A batch takes the serial chain of a
+// wave, K substeps of a barrier and `rows` rows each; a workgroup adds the
+// issue of its rows still computed (the region shrinks by two rows a substep)
+// and the loads and stores of all its rows.  Alone on a CU a workgroup does
+// not overlap them with another's, and issues less densely.  The constants are
+// least-squares fits to 1600 (shape, depth, grid) timings of each kernel
+// family, grids from 64 x 64 to 2048 x 2048 with ragged and elongated ones
+// among them, weighed towards the shapes near the best (within 8%).
+static double tiled_time(int model, bool masked, int nx, int ny, int rows, int waves, int K,
+                         int cus, int per_cu) {
+  static const double fit[2][2][5] = {
+      // substep, row of a wave, issue, load and store, issue alone
+      {{0.192, 0.0094, 0.0113, 0.0086, 0.0015}, {0.149, 0.0476, 0.0091, 0.0170, 0.0010}},  // 2V
+      {{0.051, 0.0514, 0.0085, 0.0201, 0.0011}, {0.030, 0.0443, 0.0086, 0.0300, 0.0025}}};  // FK
+  const double* c = fit[model == M2V ? 0 : 1][masked ? 1 : 0];
+  const int64_t tiles = tile_count(nx, ny, rows, waves, 1, K);
+  const int64_t L = (tiles + cus - 1) / cus, b = (L + per_cu - 1) / per_cu;
+  const int H = rows * waves;
+  const double computed = (double)K * H - (double)K * (K + 1);
+  const double issue = c[2] + (std::min<int64_t>(L, per_cu) == 1 ? c[4] : 0.0);
+  return 2.7 + b * K * (c[0] + c[1] * rows) + L * (computed * issue + H * c[3]);
+}
+
+// The launches of a YH_KERNEL_AUTO call.  A cell's value does not depend on
+// the shape, the depth or where launches split, so a call may mix them: the
+// table holds the best shape of every depth, the depth with the least time
+// per step, and for the last steps of a call the split with the least time.
+void auto_table(int model, bool masked, const KParams& k, int cus, bool apd, AutoTable* t) {
+  static const int shapes[6][2] = {{4, 8}, {8, 8}, {4, 16}, {8, 16}, {5, 16}, {7, 16}};
+  const int nx = k.nx, ny = k.ny;
+  t->depth = std::max(1, std::min(AutoTable::kDepth, std::min(nx, ny) - 1));
+  t->best = 1;
+  for (int K = 1; K <= t->depth; ++K) {
+    t->cost[K] = 1e300;
+    for (const auto& sh : shapes) {
+      if (2 * K >= sh[0] * sh[1]) continue;
+      if (apd && !tiled_apd_supported(sh[0], sh[1], 1)) continue;
+      const double us = tiled_time(model, masked, nx, ny, sh[0], sh[1], K, std::max(1, cus),
+                                   tiled_per_cu(model, masked, k, sh[0], sh[1], 1, false, apd));
+      if (us < t->cost[K]) {
+        t->cost[K] = us;
+        t->shape[K] = yh_kernel_cfg{YH_KERNEL_TILED, K, sh[0], sh[1], 1};
+      }
+    }
+    if (t->cost[K] * t->best < t->cost[t->best] * K) t->best = K;
+  }
+  t->time[0] = 0.0;
+  for (int n = 1; n <= AutoTable::kEnd; ++n) {
+    t->time[n] = 1e300;
+    for (int K = 1; K <= std::min(n, t->depth); ++K)
+      if (t->cost[K] + t->time[n - K] < t->time[n]) {
+        t->time[n] = t->cost[K] + t->time[n - K];
+        t->first[n] = K;
+      }
+  }
+  t->ready = true;
+}
+
+const yh_kernel_cfg& auto_next(const AutoTable& t, int remaining) {
+  return t.shape[remaining > AutoTable::kEnd ? t.best : t.first[remaining]];
+}
+
+// Whether a call of n steps takes the table's launches rather than launches of
+// the fixed configuration c (auto_cfg): only for an estimated gain of 3%, the
+// estimate's spread near the best.  In the timings above that is never slower
+// and 13% faster in the mean; 20-40% on ragged grids whose tiles of the fixed
+// shape would fill a last round badly (1300 x 1300 masked FK: 2.76 against
+// 3.89 us a step), 10-25% below 400 x 400 (4 x 8 regions at K=12).
+bool auto_wins(const AutoTable& t, int model, bool masked, const KParams& k, int cus,
+               const yh_kernel_cfg& c, bool apd, int n) {
+  const int many = n > AutoTable::kEnd ? (n - AutoTable::kEnd + t.best - 1) / t.best : 0;
+  const double split = many * t.cost[t.best] + t.time[n - many * t.best];
+  const int per_cu = tiled_per_cu(model, masked, k, c.rows, c.waves, c.cols, false, apd);
+  const int K = c.substeps, r = n % K;
+  auto us = [&](int d) {
+    return tiled_time(model, masked, k.nx, k.ny, c.rows, c.waves, d, std::max(1, cus), per_cu);
+  };
+  return split < 0.97 * ((n / K) * us(K) + (r ? us(r) : 0.0));
 }
 
 yh_kernel_cfg resolve_cfg(const yh_plan* pl) {
@@ -206,7 +291,28 @@ int plan_advance(yh_plan* pl, int nsteps, hipStream_t s) {
       tiled && pl->keep_prev && !ap && tiled_prev_supported(c.rows, c.waves, c.cols);
   const int tail = (pl->keep_prev && !prev_fused) ? 1 : 0;
   if (prev_fused && !pl->prev_u) YH_HIP(hipMalloc(&pl->prev_u, pl->n * sizeof(float)));
-  if (tiled) {
+  bool split = false;  // the launches of the AUTO table
+  if (tiled && pl->cfg.variant == YH_KERNEL_AUTO && remaining > tail) {
+    AutoTable& t = pl->table[ap ? 1 : 0];
+    if (!t.ready) auto_table(pl->p.model, masked, pl->k, pl->cus, ap != nullptr, &t);
+    split = auto_wins(t, pl->p.model, masked, pl->k, pl->cus, c, ap != nullptr, remaining - tail);
+    while (split && remaining > tail) {
+      const yh_kernel_cfg& l = auto_next(t, remaining - tail);
+      CFields ci;
+      Fields co;
+      fields(pl->cur, &ci, &co);
+      apd.count0 = (int)done;
+      float* prev = (prev_fused && l.substeps == remaining) ? pl->prev_u : nullptr;
+      KParams kl = pl->k;
+      kl.wt = !ap && write_through(pl, l.rows, l.waves, l.cols, l.substeps, prev != nullptr);
+      YH_HIP(launch_tiled(pl->p.model, masked, l.rows, l.waves, l.cols, l.substeps, kl, ci, co,
+                          masked ? pl->codes_d : nullptr, s, ap, prev));
+      pl->cur ^= 1;
+      remaining -= l.substeps;
+      done += l.substeps;
+    }
+  }
+  if (tiled && !split) {
     const int body = remaining - tail, r = body % c.substeps;
     const bool merge = !ap && r > 0 && body > c.substeps && merge_ok(pl, c, r, prev_fused);
     while (remaining > tail) {

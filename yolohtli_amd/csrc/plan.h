@@ -7,6 +7,21 @@
 
 struct yh_sr;  // symmetry-reduction session state (sr.hip)
 
+namespace yh {
+// The launches of a YH_KERNEL_AUTO call (plan.cpp): the best shape of every
+// depth, the depth with the least time per step, and the split of up to kEnd
+// last steps with the least time.
+struct AutoTable {
+  static constexpr int kDepth = 16, kEnd = 48;
+  bool ready = false;
+  int depth = 1, best = 1;
+  double cost[kDepth + 1];
+  yh_kernel_cfg shape[kDepth + 1];
+  double time[kEnd + 1];
+  int first[kEnd + 1];
+};
+}  // namespace yh
+
 struct yh_plan {
   yh_params p;
   yh_derived d;
@@ -29,6 +44,7 @@ struct yh_plan {
   int tipcap = 0;
   int* flag_d = nullptr;
   yh_kernel_cfg cfg{YH_KERNEL_AUTO, 4, 8, 8, 1};
+  yh::AutoTable table[2];  // without and with the APD update
   int64_t count = 0;
   bool keep_prev = true;
   bool apd_on = false;
@@ -56,7 +72,14 @@ yh_kernel_cfg auto_cfg(int nx, int ny, int cus, bool pairs = false);
 // Workgroups of the tiled kernel of this shape one CU holds at once
 // (cached; allocates nothing).
 int tiled_per_cu(int model, bool masked, const KParams& k, int rows, int waves, int cols,
-                 bool prev);
+                 bool prev, bool apd);
+// The launches of an AUTO call on a device of `cus` compute units, the next
+// one with `remaining` steps to go, and whether a call of n steps takes them
+// rather than launches of configuration c.
+void auto_table(int model, bool masked, const KParams& k, int cus, bool apd, AutoTable* t);
+const yh_kernel_cfg& auto_next(const AutoTable& t, int remaining);
+bool auto_wins(const AutoTable& t, int model, bool masked, const KParams& k, int cus,
+               const yh_kernel_cfg& c, bool apd, int n);
 // Tiles of one launch of K substeps on a rows x waves x cols shape.
 int64_t tiled_tile_count(int nx, int ny, int rows, int waves, int cols, int K);
 // Whether a tiled launch of `tiles` workgroups, `per_cu` per CU at most,

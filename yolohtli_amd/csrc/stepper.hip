@@ -21,7 +21,6 @@
 #include <algorithm>
 
 #include "direct.h"
-#include "tile.h"
 #include "yh_internal.h"
 
 namespace yh {
@@ -132,20 +131,6 @@ hipError_t launch_direct_codes(int model, const KParams& k, CFields in, Fields o
 }
 
 // ------------------------------------------------------------------- tiled
-template <int MODEL, bool MASKED, int R, int NW, int CW, bool APD, bool PREV, int ISO = -1,
-          bool WT = false>
-__global__ __launch_bounds__(64 * NW) void k_tiled(const KParams k, CFields in, Fields out,
-                                                   const uint8_t* __restrict__ codes, int K,
-                                                   int tiles_x, int ntiles, const ApdState apd,
-                                                   float* __restrict__ prev) {
-  __shared__ TileLds<MODEL, NW, CW> lds;
-  const int tile = xcd_tile(blockIdx.x, ntiles);
-  const int ty = tile / tiles_x;
-  tile_advance<MODEL, MASKED, R, NW, CW, APD, PREV, ISO, WT>(k, in, out, codes, K,
-                                                             tile - ty * tiles_x, ty, lds, apd,
-                                                             prev);
-}
-
 bool tiled_supported(int rows, int waves, int cols) {
   const bool rw = (rows == 4 && (waves == 4 || waves == 8 || waves == 16)) ||
                   (rows == 8 && (waves == 4 || waves == 8 || waves == 16)) ||
@@ -167,104 +152,11 @@ bool tiled_prev_supported(int rows, int waves, int cols) {
          (cols == 1 && (rows == 7 || rows == 5) && waves == 16);
 }
 
-template <int MODEL, bool MASKED, int R, int NW, int CW, bool APD, bool PREV = false,
-          int ISO = -1, bool WT = false>
-static hipError_t launch_tiled_t(int K, const KParams& k, CFields in, Fields out,
-                                 const uint8_t* codes, hipStream_t s, const ApdState& apd,
-                                 float* prev = nullptr, int* occ = nullptr) {
-  if (occ)  // the workgroups of this instantiation one CU holds at once; no launch
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        occ, k_tiled<MODEL, MASKED, R, NW, CW, APD, PREV, ISO, WT>, 64 * NW, 0);
-  const int wout = 64 * CW - 2 * K, hout = NW * R - 2 * K;
-  if (K < 1 || wout <= 0 || hout <= 0) return hipErrorInvalidValue;
-  const int tiles_x = (k.nx + wout - 1) / wout;
-  const int tiles_y = (k.ny + hout - 1) / hout;
-  const int ntiles = tiles_x * tiles_y;
-  hipLaunchKernelGGL((k_tiled<MODEL, MASKED, R, NW, CW, APD, PREV, ISO, WT>), dim3(ntiles),
-                     dim3(64 * NW), 0, s, k, in, out, codes, K, tiles_x, ntiles, apd, prev);
-  return hipGetLastError();
-}
-
+// tiled.h, compiled in one file per model
 template <int MODEL, bool MASKED>
-static hipError_t launch_tiled_m(int rows, int waves, int cols, int K, const KParams& k,
-                                 CFields in, Fields out, const uint8_t* codes, hipStream_t s,
-                                 const ApdState* apd, float* prev, int* occ) {
-  const ApdState a = apd ? *apd : ApdState();
-  if (apd) {
-    if (prev) return hipErrorInvalidValue;
-#define YH_TILE_APD_I(RR, WW, I) \
-  launch_tiled_t<MODEL, MASKED, RR, WW, 1, true, false, I>(K, k, in, out, codes, s, a, nullptr, occ)
-#define YH_TILE_APD(RR, WW)                    \
-  if (rows == RR && waves == WW && cols == 1) \
-    return k.iso ? YH_TILE_APD_I(RR, WW, 1) : YH_TILE_APD_I(RR, WW, -1);
-    YH_TILE_APD(4, 8)
-    YH_TILE_APD(8, 8)
-    YH_TILE_APD(4, 16)
-    YH_TILE_APD(8, 16)
-#undef YH_TILE_APD
-#undef YH_TILE_APD_I
-    return hipErrorInvalidValue;
-  }
-  // the shapes the automatic choice takes (7 x 16 and the 8 x 16 its
-  // remainders merge into on 1024^2, 8 x 8 on grids with more tiles than CUs,
-  // 4 x 16 on grids with fewer, and the 5 x 16 its remainders merge into)
-  // also come with isotropic diffusion fixed at compile time, and with
-  // write-through stores (k.wt) for launches of two workgroups per CU
-  if (k.iso && cols == 1) {
-#define YH_TILE_ISO_W(RR, WW, W)                                              \
-  return prev ? launch_tiled_t<MODEL, MASKED, RR, WW, 1, false, true, 1, W>(   \
-                    K, k, in, out, codes, s, a, prev, occ)                    \
-              : launch_tiled_t<MODEL, MASKED, RR, WW, 1, false, false, 1, W>(  \
-                    K, k, in, out, codes, s, a, nullptr, occ);
-#define YH_TILE_ISO(RR, WW)               \
-  if (rows == RR && waves == WW) {        \
-    if (k.wt) YH_TILE_ISO_W(RR, WW, true) \
-    YH_TILE_ISO_W(RR, WW, false)          \
-  }
-    YH_TILE_ISO(7, 16)
-    YH_TILE_ISO(8, 16)
-    YH_TILE_ISO(8, 8)
-    YH_TILE_ISO(4, 16)
-    YH_TILE_ISO(5, 16)
-#undef YH_TILE_ISO
-#undef YH_TILE_ISO_W
-  }
-  if (prev) {
-#define YH_TILE_PREV(RR, WW)                   \
-  if (rows == RR && waves == WW && cols == 1) \
-    return launch_tiled_t<MODEL, MASKED, RR, WW, 1, false, true>(K, k, in, out, codes, s, a, prev, \
-                                                                 occ);
-    YH_TILE_PREV(4, 8)
-    YH_TILE_PREV(8, 8)
-    YH_TILE_PREV(4, 16)
-    YH_TILE_PREV(8, 16)
-    YH_TILE_PREV(7, 16)
-    YH_TILE_PREV(5, 16)
-#undef YH_TILE_PREV
-    return hipErrorInvalidValue;
-  }
-#define YH_TILE_CASE(RR, WW, CC)                 \
-  if (rows == RR && waves == WW && cols == CC) \
-    return launch_tiled_t<MODEL, MASKED, RR, WW, CC, false>(K, k, in, out, codes, s, a, nullptr, \
-                                                            occ);
-  YH_TILE_CASE(4, 4, 1)
-  YH_TILE_CASE(8, 4, 1)
-  YH_TILE_CASE(16, 4, 1)
-  YH_TILE_CASE(4, 8, 1)
-  YH_TILE_CASE(8, 8, 1)
-  YH_TILE_CASE(16, 8, 1)
-  YH_TILE_CASE(4, 16, 1)
-  YH_TILE_CASE(8, 16, 1)
-  YH_TILE_CASE(7, 16, 1)
-  YH_TILE_CASE(5, 16, 1)
-  YH_TILE_CASE(4, 4, 2)
-  YH_TILE_CASE(8, 4, 2)
-  YH_TILE_CASE(4, 8, 2)
-  YH_TILE_CASE(8, 8, 2)
-  YH_TILE_CASE(4, 16, 2)
-#undef YH_TILE_CASE
-  return hipErrorInvalidValue;
-}
+hipError_t launch_tiled_m(int rows, int waves, int cols, int K, const KParams& k, CFields in,
+                          Fields out, const uint8_t* codes, hipStream_t s, const ApdState* apd,
+                          float* prev, int* occ);
 
 hipError_t launch_tiled(int model, bool masked, int rows, int waves, int cols, int K,
                         const KParams& k, CFields in, Fields out, const uint8_t* codes,
