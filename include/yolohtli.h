@@ -316,8 +316,10 @@ int yh_solve_matrix(const double phi[3], const double I[12], double c[3]);
  * tissue by k steps from a (tissue, tile) work list; yh_batch_step replays a
  * captured hipGraph of the launches when graphs are on (default).  The
  * kernel starts as k = 6 on 8 rows x 8 waves, one workgroup per item, with k
- * capped at the smallest tissue's min(nx, ny) - 1; yh_batch_autotune times
- * the alternatives. */
+ * capped at the smallest tissue's min(nx, ny) - 1; until yh_batch_set_kernel
+ * or yh_batch_autotune, calls run with other shapes and depths where an
+ * estimate of their time is lower (the results are the same bit for bit);
+ * yh_batch_autotune times the alternatives. */
 typedef struct yh_batch yh_batch;
 int yh_batch_create(const yh_params* per_tissue, int ntissues, yh_batch** out);
 void yh_batch_destroy(yh_batch* batch);

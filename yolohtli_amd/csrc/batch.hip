@@ -41,10 +41,15 @@ __global__ __launch_bounds__(64 * NW) void k_batch(const BatchTissue* __restrict
   __shared__ TileLds<MODEL, NW, CW> lds;
   const int G = gridDim.x;
   int x = blockIdx.x & 7, local = blockIdx.x >> 3;
-  // XCD x handles items [lo, hi) with its workgroups b = x, x+8, x+16, ...
+  // XCD x handles items [lo, hi) with its workgroups b = x, x+8, x+16, ...;
+  // the XCDs with one workgroup more (the first G mod 8) also take the items
+  // left over, so with a workgroup per item none runs two (bounds at
+  // nitems*x/8 gave some a second item, and the launch twice the time, for
+  // most item counts)
   int per_x = (G + 7 - x) >> 3;
-  int lo = (int)(((long long)nitems * x) >> 3);
-  int hi = (int)(((long long)nitems * (x + 1)) >> 3);
+  const int q = nitems >> 3, rem = nitems & 7;
+  int lo = x * q + (x < rem ? x : rem);
+  int hi = lo + q + (x < rem ? 1 : 0);
   if (G < 8) {  // too few workgroups to give every XCD one: plain striding
     local = blockIdx.x;
     per_x = G;
@@ -107,12 +112,12 @@ static int max_resident(int* out) {
                : FN<M, MK, RR, WW, CC, -1>(__VA_ARGS__);
 
 #define YH_BATCH_SHAPES(M, MK, FN, ...)            \
-  YH_BATCH_ONE(M, MK, 4, 8, 1, FN, __VA_ARGS__)   \
+  YH_BATCH_ISO(M, MK, 4, 8, 1, FN, __VA_ARGS__)   \
   YH_BATCH_ISO(M, MK, 8, 8, 1, FN, __VA_ARGS__)   \
-  YH_BATCH_ONE(M, MK, 4, 16, 1, FN, __VA_ARGS__)  \
-  YH_BATCH_ONE(M, MK, 8, 16, 1, FN, __VA_ARGS__)  \
+  YH_BATCH_ISO(M, MK, 4, 16, 1, FN, __VA_ARGS__)  \
+  YH_BATCH_ISO(M, MK, 8, 16, 1, FN, __VA_ARGS__)  \
   YH_BATCH_ONE(M, MK, 16, 8, 1, FN, __VA_ARGS__)  \
-  YH_BATCH_ONE(M, MK, 7, 16, 1, FN, __VA_ARGS__)  \
+  YH_BATCH_ISO(M, MK, 7, 16, 1, FN, __VA_ARGS__)  \
   YH_BATCH_ONE(M, MK, 4, 8, 2, FN, __VA_ARGS__)   \
   YH_BATCH_ONE(M, MK, 8, 8, 2, FN, __VA_ARGS__)   \
   YH_BATCH_ONE(M, MK, 4, 16, 2, FN, __VA_ARGS__)
@@ -159,6 +164,11 @@ struct yh_batch {
   // at most min(nx, ny) - 1 substeps)
   yh_kernel_cfg cfg{YH_KERNEL_TILED, 6, 8, 8, 1};
   int persistent = 0;
+  // until a kernel is set or tuned, calls may take other shapes and depths
+  // (the same results) where an estimate of their time is lower
+  bool chosen = false;
+  yh::AutoTable table;
+  double cfg_us[8];  // the same estimate of cfg's launches of 0 .. 6 steps
   bool use_graph = true;
   int64_t count = 0;
   // per-K work lists: K -> (tissue table, items, nitems)
@@ -192,10 +202,11 @@ static void batch_clear_graphs(yh_batch* b) {
   b->graph_objs.clear();
 }
 
-static int batch_worklist(yh_batch* b, int K, yh_batch::WL** out) {
+static int batch_worklist(yh_batch* b, const yh_kernel_cfg& c, yh_batch::WL** out) {
+  const int K = c.substeps;
   auto it = b->wl.find(K);
-  if (it != b->wl.end() && it->second.cfg.rows == b->cfg.rows &&
-      it->second.cfg.waves == b->cfg.waves && it->second.cfg.cols == b->cfg.cols) {
+  if (it != b->wl.end() && it->second.cfg.rows == c.rows && it->second.cfg.waves == c.waves &&
+      it->second.cfg.cols == c.cols) {
     *out = &it->second;
     return YH_OK;
   }
@@ -206,7 +217,7 @@ static int batch_worklist(yh_batch* b, int K, yh_batch::WL** out) {
     (void)hipFree(it->second.items);
     b->wl.erase(it);
   }
-  const int wout = 64 * b->cfg.cols - 2 * K, hout = b->cfg.rows * b->cfg.waves - 2 * K;
+  const int wout = 64 * c.cols - 2 * K, hout = c.rows * c.waves - 2 * K;
   if (wout <= 0 || hout <= 0) return YH_EINVAL;
   std::vector<BatchTissue> tab(b->nt);
   std::vector<int2> items;
@@ -219,7 +230,7 @@ static int batch_worklist(yh_batch* b, int K, yh_batch::WL** out) {
     for (int q = 0; q < tab[t].tiles_x * tiles_y; ++q) items.push_back(make_int2(t, q));
   }
   yh_batch::WL w;
-  w.cfg = b->cfg;
+  w.cfg = c;
   w.nitems = (int)items.size();
   hipError_t e = hipMalloc(&w.tissues, sizeof(BatchTissue) * b->nt);
   if (e == hipSuccess) e = hipMalloc(&w.items, sizeof(int2) * items.size());
@@ -237,17 +248,74 @@ static int batch_worklist(yh_batch* b, int K, yh_batch::WL** out) {
   return YH_OK;
 }
 
-// Enqueue nsteps as launches of K = cfg.substeps (the last one shorter).
-static int batch_enqueue(yh_batch* b, int nsteps, hipStream_t s) {
-  const yh_kernel_cfg c = b->cfg;
+// Estimated time (us) of a launch, as the plan's tiled_time (plan.cpp) over the
+// tiles of all tissues: the constants are fits to 960 timings of each kernel
+// family on batches of 2 to 100 tissues of sides 64 to 768.
+static double batch_time(const yh_batch* b, int rows, int waves, int K, int cus, int resident) {
+  static const double fit[2][2][4] = {
+      // substep, row of a wave, issue, load and store
+      {{0.175, 0.0134, 0.0111, 0.0067}, {0.205, 0.0, 0.0126, 0.0112}},   // 2V
+      {{0.0, 0.0178, 0.0127, 0.0129}, {0.064, 0.0, 0.0150, 0.0187}}};    // FK
+  const double* c = fit[b->model == M2V ? 0 : 1][b->masked ? 1 : 0];
+  const int wout = 64 - 2 * K, H = rows * waves, hout = H - 2 * K;
+  int64_t tiles = 0;
+  for (const yh_params& p : b->p)
+    tiles += (int64_t)((p.nx + wout - 1) / wout) * ((p.ny + hout - 1) / hout);
+  const int64_t per_cu = std::max(1, resident / cus);
+  const int64_t L = (tiles + cus - 1) / cus, q = (L + per_cu - 1) / per_cu;
+  const double computed = (double)K * H - (double)K * (K + 1);
+  return 4.2 + q * K * (c[0] + c[1] * rows) + L * (computed * c[2] + H * c[3]);
+}
+
+// Whether a call of n steps takes the table's launches rather than cfg's: while
+// no kernel was chosen, for an estimated gain of 3% (in the timings above never
+// more than 1.3% slower, 18% faster in the mean; a batch of a few small tissues
+// twice as fast, since cfg was picked on 256).
+static int batch_auto(yh_batch* b, int n, bool* wins) {
+  *wins = false;
+  if (b->chosen) return YH_OK;
+  const int K0 = b->cfg.substeps;
+  if (!b->table.ready) {
+    int dev = 0, cus = 0, rc = YH_OK, side = 1 << 30;
+    YH_HIP(hipGetDevice(&dev));
+    YH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    auto us = [&](int rows, int waves, int K) {
+      int res = 0;
+      if (!batch_shape_ok(rows, waves, 1)) return -1.0;
+      const int e = batch_resident(b->model, b->masked, b->iso, rows, waves, 1, &res);
+      if (e) rc = e;
+      return batch_time(b, rows, waves, K, std::max(1, cus), res);
+    };
+    for (const yh_params& p : b->p) side = std::min({side, p.nx, p.ny});
+    b->table.fill(side - 1, us);
+    for (int K = 1; K <= K0; ++K) b->cfg_us[K] = us(b->cfg.rows, b->cfg.waves, K);
+    b->cfg_us[0] = 0.0;
+    if (rc) {
+      b->table.ready = false;
+      return rc;
+    }
+  }
+  *wins = b->table.of(n) < 0.97 * ((n / K0) * b->cfg_us[K0] + b->cfg_us[n % K0]);
+  return YH_OK;
+}
+
+// The launch with `remaining` steps to go.
+static yh_kernel_cfg batch_next(const yh_batch* b, bool table, int remaining) {
+  yh_kernel_cfg c = table ? b->table.next(remaining) : b->cfg;
+  c.substeps = std::min(c.substeps, remaining);
+  return c;
+}
+
+// Enqueue nsteps.
+static int batch_enqueue(yh_batch* b, int nsteps, bool table, hipStream_t s) {
   int remaining = nsteps;
   while (remaining > 0) {
-    const int K = std::min(c.substeps, remaining);
+    const yh_kernel_cfg c = batch_next(b, table, remaining);
     yh_batch::WL* w = nullptr;
-    int rc = batch_worklist(b, K, &w);
+    int rc = batch_worklist(b, c, &w);
     if (rc) return rc;
     int grid = w->nitems;
-    if (b->persistent) {
+    if (b->persistent && !table) {
       int res = 0;
       rc = batch_resident(b->model, b->masked, b->iso, c.rows, c.waves, c.cols, &res);
       if (rc) return rc;
@@ -257,9 +325,10 @@ static int batch_enqueue(yh_batch* b, int nsteps, hipStream_t s) {
     CFields in{{b->buf[bi][0], b->buf[bi][1], b->buf[bi][2]}};
     Fields out{{b->buf[bi ^ 1][0], b->buf[bi ^ 1][1], b->buf[bi ^ 1][2]}};
     YH_HIP(launch_batch(b->model, b->masked, b->iso, c.rows, c.waves, c.cols, grid, w->tissues,
-                        w->items, w->nitems, in, out, b->masked ? b->codes_d : nullptr, K, s));
+                        w->items, w->nitems, in, out, b->masked ? b->codes_d : nullptr,
+                        c.substeps, s));
     b->cur ^= 1;
-    remaining -= K;
+    remaining -= c.substeps;
   }
   return YH_OK;
 }
@@ -406,6 +475,7 @@ int yh_batch_set_kernel(yh_batch* b, const yh_kernel_cfg* cfg, int persistent) {
     if (cfg->substeps > std::min(b->p[t].nx, b->p[t].ny) - 1) return YH_EINVAL;
   b->cfg = *cfg;
   b->persistent = persistent ? 1 : 0;
+  b->chosen = true;
   return YH_OK;
 }
 
@@ -422,31 +492,39 @@ int yh_batch_step(yh_batch* b, int nsteps, void* stream) {
     for (int t = 0; t < b->nt; ++t)
       if (!b->mask_set[t]) return YH_ESTATE;
   hipStream_t s = (hipStream_t)stream;
+  bool table = false;
+  int rc = batch_auto(b, nsteps, &table);
+  if (rc) return rc;
   if (!b->use_graph) {
-    int rc = batch_enqueue(b, nsteps, s);
+    rc = batch_enqueue(b, nsteps, table, s);
     if (rc) return rc;
     b->count += nsteps;
     return YH_OK;
   }
-  const auto key = std::make_tuple(nsteps, b->cur, b->cfg.substeps, b->cfg.rows, b->cfg.waves,
-                                   b->cfg.cols, b->persistent);
+  const auto key =
+      table ? std::make_tuple(nsteps, b->cur, 0, 0, 0, 0, 0)
+            : std::make_tuple(nsteps, b->cur, b->cfg.substeps, b->cfg.rows, b->cfg.waves,
+                              b->cfg.cols, b->persistent);
   auto it = b->graphs.find(key);
-  const int nlaunch = (nsteps + b->cfg.substeps - 1) / b->cfg.substeps;
+  int nlaunch = 0;
+  for (int rem = nsteps; rem > 0; rem -= batch_next(b, table, rem).substeps) ++nlaunch;
   if (it == b->graphs.end()) {
     // build the work lists outside the capture (they allocate)
-    for (int rem = nsteps; rem > 0; rem -= b->cfg.substeps) {
+    for (int rem = nsteps; rem > 0;) {
+      const yh_kernel_cfg c = batch_next(b, table, rem);
       yh_batch::WL* w = nullptr;
-      int rc = batch_worklist(b, std::min(b->cfg.substeps, rem), &w);
+      rc = batch_worklist(b, c, &w);
       if (rc) return rc;
+      rem -= c.substeps;
     }
     int res = 0;
-    int rc = batch_resident(b->model, b->masked, b->iso, b->cfg.rows, b->cfg.waves, b->cfg.cols,
+    rc = batch_resident(b->model, b->masked, b->iso, b->cfg.rows, b->cfg.waves, b->cfg.cols,
                             &res);
     if (rc) return rc;
     if (!b->cap_stream) YH_HIP(hipStreamCreateWithFlags(&b->cap_stream, hipStreamNonBlocking));
     const int cur0 = b->cur;
     YH_HIP(hipStreamBeginCapture(b->cap_stream, hipStreamCaptureModeThreadLocal));
-    rc = batch_enqueue(b, nsteps, b->cap_stream);
+    rc = batch_enqueue(b, nsteps, table, b->cap_stream);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(b->cap_stream, &g);
     b->cur = cur0;  // capture only recorded the launches
@@ -527,10 +605,10 @@ int yh_batch_autotune(yh_batch* b, int steps, void* stream, yh_kernel_cfg* best,
         b->cfg = yh_kernel_cfg{YH_KERNEL_TILED, K, sh[0], sh[1], sh[2]};
         b->persistent = pers;
         const int n = std::max(K, (steps / K) * K);
-        rc = batch_enqueue(b, K, s);
+        rc = batch_enqueue(b, K, false, s);
         if (rc) break;
         if (hipEventRecord(e0, s) != hipSuccess) { rc = YH_EHIP; break; }
-        rc = batch_enqueue(b, n, s);
+        rc = batch_enqueue(b, n, false, s);
         if (rc) break;
         if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess) {
           rc = YH_EHIP;
@@ -564,6 +642,7 @@ int yh_batch_autotune(yh_batch* b, int steps, void* stream, yh_kernel_cfg* best,
   }
   b->cfg = bestc;
   b->persistent = bestp;
+  b->chosen = true;
   if (best) *best = bestc;
   if (best_ms) *best_ms = bestt;
   return YH_OK;

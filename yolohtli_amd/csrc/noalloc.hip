@@ -101,7 +101,7 @@ int yh_step_noalloc(const yh_params* p, float* const out[3], const float* const 
   auto_table(p->model, masked, k, cus, false, &t);
   const bool split = auto_wins(t, p->model, masked, k, cus, c, false, nsteps);
   auto next = [&](int remaining) {
-    yh_kernel_cfg l = split ? auto_next(t, remaining) : c;
+    yh_kernel_cfg l = split ? t.next(remaining) : c;
     l.substeps = std::min(l.substeps, remaining);
     return l;
   };

@@ -133,38 +133,11 @@ static double tiled_time(int model, bool masked, int nx, int ny, int rows, int w
 // table holds the best shape of every depth, the depth with the least time
 // per step, and for the last steps of a call the split with the least time.
 void auto_table(int model, bool masked, const KParams& k, int cus, bool apd, AutoTable* t) {
-  static const int shapes[6][2] = {{4, 8}, {8, 8}, {4, 16}, {8, 16}, {5, 16}, {7, 16}};
-  const int nx = k.nx, ny = k.ny;
-  t->depth = std::max(1, std::min(AutoTable::kDepth, std::min(nx, ny) - 1));
-  t->best = 1;
-  for (int K = 1; K <= t->depth; ++K) {
-    t->cost[K] = 1e300;
-    for (const auto& sh : shapes) {
-      if (2 * K >= sh[0] * sh[1]) continue;
-      if (apd && !tiled_apd_supported(sh[0], sh[1], 1)) continue;
-      const double us = tiled_time(model, masked, nx, ny, sh[0], sh[1], K, std::max(1, cus),
-                                   tiled_per_cu(model, masked, k, sh[0], sh[1], 1, false, apd));
-      if (us < t->cost[K]) {
-        t->cost[K] = us;
-        t->shape[K] = yh_kernel_cfg{YH_KERNEL_TILED, K, sh[0], sh[1], 1};
-      }
-    }
-    if (t->cost[K] * t->best < t->cost[t->best] * K) t->best = K;
-  }
-  t->time[0] = 0.0;
-  for (int n = 1; n <= AutoTable::kEnd; ++n) {
-    t->time[n] = 1e300;
-    for (int K = 1; K <= std::min(n, t->depth); ++K)
-      if (t->cost[K] + t->time[n - K] < t->time[n]) {
-        t->time[n] = t->cost[K] + t->time[n - K];
-        t->first[n] = K;
-      }
-  }
-  t->ready = true;
-}
-
-const yh_kernel_cfg& auto_next(const AutoTable& t, int remaining) {
-  return t.shape[remaining > AutoTable::kEnd ? t.best : t.first[remaining]];
+  t->fill(std::min(k.nx, k.ny) - 1, [&](int rows, int waves, int K) {
+    if (apd && !tiled_apd_supported(rows, waves, 1)) return -1.0;
+    return tiled_time(model, masked, k.nx, k.ny, rows, waves, K, std::max(1, cus),
+                      tiled_per_cu(model, masked, k, rows, waves, 1, false, apd));
+  });
 }
 
 // Whether a call of n steps takes the table's launches rather than launches of
@@ -175,14 +148,12 @@ const yh_kernel_cfg& auto_next(const AutoTable& t, int remaining) {
 // 3.89 us a step), 10-25% below 400 x 400 (4 x 8 regions at K=12).
 bool auto_wins(const AutoTable& t, int model, bool masked, const KParams& k, int cus,
                const yh_kernel_cfg& c, bool apd, int n) {
-  const int many = n > AutoTable::kEnd ? (n - AutoTable::kEnd + t.best - 1) / t.best : 0;
-  const double split = many * t.cost[t.best] + t.time[n - many * t.best];
   const int per_cu = tiled_per_cu(model, masked, k, c.rows, c.waves, c.cols, false, apd);
   const int K = c.substeps, r = n % K;
   auto us = [&](int d) {
     return tiled_time(model, masked, k.nx, k.ny, c.rows, c.waves, d, std::max(1, cus), per_cu);
   };
-  return split < 0.97 * ((n / K) * us(K) + (r ? us(r) : 0.0));
+  return t.of(n) < 0.97 * ((n / K) * us(K) + (r ? us(r) : 0.0));
 }
 
 yh_kernel_cfg resolve_cfg(const yh_plan* pl) {
@@ -297,7 +268,7 @@ int plan_advance(yh_plan* pl, int nsteps, hipStream_t s) {
     if (!t.ready) auto_table(pl->p.model, masked, pl->k, pl->cus, ap != nullptr, &t);
     split = auto_wins(t, pl->p.model, masked, pl->k, pl->cus, c, ap != nullptr, remaining - tail);
     while (split && remaining > tail) {
-      const yh_kernel_cfg& l = auto_next(t, remaining - tail);
+      const yh_kernel_cfg& l = t.next(remaining - tail);
       CFields ci;
       Fields co;
       fields(pl->cur, &ci, &co);

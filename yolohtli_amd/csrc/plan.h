@@ -19,6 +19,45 @@ struct AutoTable {
   yh_kernel_cfg shape[kDepth + 1];
   double time[kEnd + 1];
   int first[kEnd + 1];
+
+  // us(rows, waves, K): estimated time of a launch, < 0 for a shape that is not
+  // to be taken.
+  template <class Time>
+  void fill(int max_depth, Time us) {
+    static const int shapes[6][2] = {{4, 8}, {8, 8}, {4, 16}, {8, 16}, {5, 16}, {7, 16}};
+    depth = max_depth < 1 ? 1 : max_depth > kDepth ? kDepth : max_depth;
+    best = 1;
+    for (int K = 1; K <= depth; ++K) {
+      cost[K] = 1e300;
+      for (const auto& sh : shapes) {
+        if (2 * K >= sh[0] * sh[1]) continue;
+        const double t = us(sh[0], sh[1], K);
+        if (t < 0.0 || t >= cost[K]) continue;
+        cost[K] = t;
+        shape[K] = yh_kernel_cfg{YH_KERNEL_TILED, K, sh[0], sh[1], 1};
+      }
+      if (cost[K] * best < cost[best] * K) best = K;
+    }
+    time[0] = 0.0;
+    for (int n = 1; n <= kEnd; ++n) {
+      time[n] = 1e300;
+      for (int K = 1; K <= n && K <= depth; ++K)
+        if (cost[K] + time[n - K] < time[n]) {
+          time[n] = cost[K] + time[n - K];
+          first[n] = K;
+        }
+    }
+    ready = true;
+  }
+  // The next launch with `remaining` steps to go.
+  const yh_kernel_cfg& next(int remaining) const {
+    return shape[remaining > kEnd ? best : first[remaining]];
+  }
+  // Estimated time of n steps.
+  double of(int n) const {
+    const int many = n > kEnd ? (n - kEnd + best - 1) / best : 0;
+    return many * cost[best] + time[n - many * best];
+  }
 };
 }  // namespace yh
 
@@ -73,11 +112,9 @@ yh_kernel_cfg auto_cfg(int nx, int ny, int cus, bool pairs = false);
 // (cached; allocates nothing).
 int tiled_per_cu(int model, bool masked, const KParams& k, int rows, int waves, int cols,
                  bool prev, bool apd);
-// The launches of an AUTO call on a device of `cus` compute units, the next
-// one with `remaining` steps to go, and whether a call of n steps takes them
-// rather than launches of configuration c.
+// The launches of an AUTO call on a device of `cus` compute units, and whether
+// a call of n steps takes them rather than launches of configuration c.
 void auto_table(int model, bool masked, const KParams& k, int cus, bool apd, AutoTable* t);
-const yh_kernel_cfg& auto_next(const AutoTable& t, int remaining);
 bool auto_wins(const AutoTable& t, int model, bool masked, const KParams& k, int cus,
                const yh_kernel_cfg& c, bool apd, int n);
 // Tiles of one launch of K substeps on a rows x waves x cols shape.
