@@ -140,7 +140,7 @@ __global__ __launch_bounds__(kRtBX* kRtBY) void k_sr_rdtips(const KParams k, con
   const float* pr = X.f[0];
   // physicalTime = dt*count (main.cu:885)
   const float t = (float)(g.dt * (double)st->count);
-  tip_solve(i, j, nx, MASKED, Uth, pr[c], pr[sx], pr[sxy], pr[sy], s_u[l0], s_u[lx], s_u[lxy],
+  tip_solve(i, j, nx, Uth, pr[c], pr[sx], pr[sxy], pr[sy], s_u[l0], s_u[lx], s_u[lxy],
             s_u[ly], t, tips, keys, count, kSrTipCap);
 }
 
@@ -792,7 +792,7 @@ __global__ __launch_bounds__(kBfThreads) void k_bf_rd(const KParams k, SrGeom g,
     const bool ex = gi < nx - 1, ey = gj < ny - 1;
     const int lx = ex ? L + 1 : L, ly = ey ? L + LW : L, lxy = (ex && ey) ? L + LW + 1 : L;
     const float* pr = s_f[0];
-    tip_solve(gi, gj, nx, MASKED, Uth, pr[L], pr[lx], pr[lxy], pr[ly], s_ro[L], s_ro[lx],
+    tip_solve(gi, gj, nx, Uth, pr[L], pr[lx], pr[lxy], pr[ly], s_ro[L], s_ro[lx],
               s_ro[lxy], s_ro[ly], t, sa.next_tips, sa.next_keys, sa.next_count, kSrTipCap);
   }
 }

