@@ -26,6 +26,7 @@
 #include <new>
 #include <vector>
 
+#include "lanes.h"
 #include "plan.h"
 
 namespace yh {
@@ -473,31 +474,10 @@ struct GlobalAcc {
   }
 };
 
-// v of the lane that DPP control CTRL names, 0 where it names none.
-template <int CTRL>
-__device__ __forceinline__ double dpp_double(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-// Sum over the wave in lane 63, by shifts within rows of 16 lanes and
-// broadcasts of a row's last lane: VALU moves, no LDS round trips (with the
-// sums' old values read early, 15.2 -> 14.6 us a reverse launch against
-// ds_bpermute trees).
-__device__ __forceinline__ double wave_sum(double v) {
-  v += dpp_double<0x111>(v);  // row_shr:1
-  v += dpp_double<0x112>(v);  // row_shr:2
-  v += dpp_double<0x114>(v);  // row_shr:4
-  v += dpp_double<0x118>(v);  // row_shr:8
-  v += dpp_double<0x142>(v);  // row_bcast:15 (rows 1 and 3 take the row before)
-  v += dpp_double<0x143>(v);  // row_bcast:31 (rows 2 and 3 take the half before)
-  return v;
-}
-
 // The sums of gt over the first NT threads of a workgroup, those that hold any
 // (FP64, fixed order), added to the workgroup's slot, whose value before
-// (of threads 0 to 5) is `was`.
+// (of threads 0 to 5) is `was` (read early, and the sums by VALU moves: 15.2 ->
+// 14.6 us a reverse launch against ds_bpermute trees and a late read).
 template <int NT>
 __device__ __forceinline__ void adj_gtau_block(const double gt[6], double was, double* slot) {
   __shared__ double red[NT / 64][6];
@@ -508,7 +488,7 @@ __device__ __forceinline__ void adj_gtau_block(const double gt[6], double was, d
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
       const double v = wave_sum(gt[q]);
-      if (lane == 63) red[wv][q] = v;
+      if (lane == 0) red[wv][q] = v;
     }
   }
   __syncthreads();
@@ -774,7 +754,7 @@ __global__ __launch_bounds__(256) void k_adj_loss(const float* __restrict__ trac
     src[q] = (float)(2.0 * d);
   }
   sum = wave_sum(sum);
-  if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = sum;
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sum;
   __syncthreads();
   if (threadIdx.x == 0) part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }

@@ -11,13 +11,14 @@
 //                   symmetryReduction.cu:95-107), then over the disk's
 //                   bounding box: slices, template and velTan in FP64, the
 //                   12 disk inner products as per-workgroup partial sums
-//                   (slice_kernel + trapz_kernel fused: no slice arrays)
+//                   (slice_kernel + trapz_kernel fused: no slice arrays);
+//                   one wave appends the step's tips to the log
 //   3 k_bf_fused    every workgroup reduces the partials in one fixed order
 //                   and solves solve_matrix (symmetryReduction.cu:386-418)
 //                   itself, so all agree bit for bit; then BFECC of Xo into X
 //                   (advFDBFECC.cu:18-165), the three dependent phases through
 //                   an LDS tile with a 3-cell halo.  Workgroup 0 commits the
-//                   step: c, phi += dt*c, centre, count, the tips to the log.
+//                   step: c, phi += dt*c, centre, count.
 // By default a steady step is two launches: k_sr_slices, then k_bf_rd, which
 // is k_bf_fused on a 5-cell halo followed by the next step's RD and tip test
 // (what k_sr_rdtips would compute, bit for bit) on the same tile; the first
@@ -41,6 +42,7 @@
 #include <vector>
 
 #include "direct.h"
+#include "lanes.h"
 #include "plan.h"
 
 namespace yh {
@@ -63,24 +65,36 @@ struct SrGeom {
   double dtx, dty;  // dt/hx, dt/hy (advection Courant factors)
 };
 
-// Buffers of one step: the state slots, the step's tips, the partials, the
-// plan's tip log and the (c, phi) history.
+// What the slices launch finds of a step's tips: the disk centre and the count.
+struct SrStep {
+  int cx, cy, found, pad;
+};
+
+// The tips of a step and the plan's tip log.
+struct SrTips {
+  const yh_tip* tips;
+  const int* keys;
+  const int* count;
+  yh_tip* log_tips;
+  int* log_keys;
+  int* log_count;
+  int logcap;
+  SrStep* step;
+};
+
+// Buffers of one step's BFECC launch: the state slots, the partials, the
+// (c, phi) history and the next step's tips (k_bf_rd).
 struct SrArgs {
   const SrDev* st_in;
   SrDev* st_out;
+  const SrStep* step;
   const double* partials;
   int nparts;
   int record;  // push (c, phi) before the solve into hist
   double* hist;
   long long histcap;
-  const yh_tip* step_tips;
-  const int* step_keys;
-  int* step_count;
-  yh_tip* log_tips;
-  int* log_keys;
-  int* log_count;
-  int logcap;
-  yh_tip* next_tips;  // the next step's tips (k_bf_rd)
+  int* step_count;  // cleared for the step after next
+  yh_tip* next_tips;
   int* next_keys;
   int* next_count;
 };
@@ -145,12 +159,14 @@ __global__ __launch_bounds__(kRtBX* kRtBY) void k_sr_rdtips(const KParams k, con
 }
 
 // ---------------------------------------------------------------- centre
-// Disk centre of this step, the same in every wave that asks: tipx0 at
+// Disk centre of this step, the same in every wave: tipx0 at
 // count 0 (symmetryReduction.cu:98-100), else the last tip of this step in
 // (cell, root) order (:102-103), else the previous centre.  Keys are unique,
 // so the wave maximum names one slot.
+// cnt: the tips found.
 __device__ __forceinline__ void sr_centre(const SrGeom& g, const SrDev* st, const yh_tip* tips,
-                                          const int* keys, const int* count, int& cx, int& cy) {
+                                          const int* keys, const int* count, int& cx, int& cy,
+                                          int& cnt) {
   const int lane = __lane_id();
   // the step count, the tip count, the first 64 keys and their tips are read
   // together (slots past the tip count are ignored), so the centre costs one
@@ -158,7 +174,7 @@ __device__ __forceinline__ void sr_centre(const SrGeom& g, const SrDev* st, cons
   const long long step = st->count;
   const int k0 = keys[lane];
   const yh_tip t0 = tips[lane];
-  const int cnt = *count;
+  cnt = *count;
   if (step == 0) {
     cx = __float2int_rn(st->tip0x - (float)(g.nx / 2));
     cy = __float2int_rn(st->tip0y - (float)(g.ny / 2));
@@ -208,13 +224,26 @@ __device__ __forceinline__ void sr_centre(const SrGeom& g, const SrDev* st, cons
 template <int MODEL, bool MASKED>
 __global__ __launch_bounds__(kSliceBX* kSliceBY) void k_sr_slices(
     const KParams k, const SrGeom g, int R, CFields X, const uint8_t* __restrict__ codes,
-    const SrDev* __restrict__ st, const yh_tip* __restrict__ step_tips,
-    const int* __restrict__ step_keys, const int* __restrict__ step_count,
-    double* __restrict__ partials) {
+    const SrDev* __restrict__ st, const SrTips tp, int log, double* __restrict__ partials) {
   using M = Model<MODEL>;
   constexpr int NV = M::NV;
-  int cx, cy;
-  sr_centre(g, st, step_tips, step_keys, step_count, cx, cy);
+  int cx, cy, found;
+  sr_centre(g, st, tp.tips, tp.keys, tp.count, cx, cy, found);
+  // one wave of one workgroup also moves the tips to the log: its slots are
+  // asked for here and filled at the end, so the way to memory and back runs
+  // beside the slices (in the BFECC launch it held workgroup 0 up twice before
+  // the solve).  The tips are read again there: kept in a struct since the
+  // centre they went to LDS at an address from the dispatch packet, whose read
+  // from host memory made the launch 10 us longer
+  const int tid = threadIdx.y * kSliceBX + threadIdx.x;
+  const int lane = tid & 63, wv = tid >> 6;
+  const bool mover = log && blockIdx.x == 0 && blockIdx.y == 0 &&
+                     wv == kSliceBX * kSliceBY / 64 - 1;
+  int base = 0;
+  if (mover && lane == 0) {
+    base = *tp.log_count;
+    *tp.step = SrStep{cx, cy, found, 0};
+  }
   const int i = g.nx / 2 + cx - R + blockIdx.x * kSliceBX + threadIdx.x;
   const int j = g.ny / 2 + cy - R + blockIdx.y * kSliceBY + threadIdx.y;
   double acc[12];
@@ -281,30 +310,24 @@ __global__ __launch_bounds__(kSliceBX* kSliceBY) void k_sr_slices(
   }
   // block reduction: wave shuffles, then across the 4 waves through LDS
   __shared__ double red[kSliceBX * kSliceBY / 64][12];
-  const int tid = threadIdx.y * kSliceBX + threadIdx.x;
-  const int lane = tid & 63, wv = tid >> 6;
   // Sums over the wave's 64 lanes with the pairs of a shfl_down tree (at
   // each level lane i's partial meets lane i + off's, so every sum equals
-  // that tree's bit for bit: IEEE addition commutes) but fewer exchanges:
-  // at the first level the lower half of the wave keeps values 0-5 and the
-  // upper half 6-11, at the second each quarter keeps three, so 6 + 3 +
-  // 4 x 3 exchanges instead of 6 x 12.  Values 3r..3r+2 end in lane 16r.
-  const bool up32 = (lane & 32) != 0, up16 = (lane & 16) != 0;
-  double h[6], t[3];
+  // that tree's bit for bit: IEEE addition commutes).  A swap of lane halves
+  // adds two values at once: after the first level the lower half of the wave
+  // holds values 0-5 and the upper half 6-11, after the second each row three.
+  // Values 3r..3r+2 end in lane 16r.
+  double t[6];
 #pragma unroll
   for (int p = 0; p < 6; ++p) {
-    const double give = up32 ? acc[p] : acc[6 + p];
-    h[p] = (up32 ? acc[6 + p] : acc[p]) + __shfl_xor(give, 32, 64);
+    double a = acc[p], b = acc[6 + p];
+    swap_lanes<false>(a, b);
+    t[p] = a + b;
   }
 #pragma unroll
   for (int p = 0; p < 3; ++p) {
-    const double give = up16 ? h[p] : h[3 + p];
-    t[p] = (up16 ? h[3 + p] : h[p]) + __shfl_xor(give, 16, 64);
-  }
-#pragma unroll
-  for (int off = 8; off > 0; off >>= 1) {
-#pragma unroll
-    for (int p = 0; p < 3; ++p) t[p] += __shfl_xor(t[p], off, 64);
+    double a = t[p], b = t[3 + p];
+    swap_lanes<true>(a, b);
+    t[p] = row_sum(a + b);
   }
   if ((lane & 15) == 0) {
 #pragma unroll
@@ -316,12 +339,25 @@ __global__ __launch_bounds__(kSliceBX* kSliceBY) void k_sr_slices(
     for (int w = 0; w < kSliceBX * kSliceBY / 64; ++w) s += red[w][tid];
     partials[(size_t)tid * gridDim.x * gridDim.y + blockIdx.y * gridDim.x + blockIdx.x] = s;
   }
+  if (mover) {
+    base = __builtin_amdgcn_readfirstlane(base);
+    if (lane == 0) *tp.log_count = base + found;
+    const int n = min(found, kSrTipCap);
+    for (int q = lane; q < n; q += 64) {
+      const yh_tip tip = tp.tips[q];
+      const int key = tp.keys[q];
+      if (base + q < tp.logcap) {
+        tp.log_tips[base + q] = tip;
+        tp.log_keys[base + q] = key;
+      }
+    }
+  }
 }
 
 // ----------------------------------------------------------------- solve
 // Column q of the partials (stored column-major, [12][nparts]) summed by one
-// wave in a fixed order (lane-strided, then a shuffle tree), so the integrals do not depend on scheduling and
-// every wave that sums a column gets the same bits.  The total is in lane 0.
+// wave in a fixed order (lane-strided, then the pairs of a shuffle tree), so the integrals do not depend on
+// scheduling and every wave that sums a column gets the same bits.  The total is in lane 0.
 __device__ __forceinline__ double sr_column_sum(const double* partials, int nparts, int q) {
   const int lane = __lane_id();
   double s = 0.0;
@@ -339,22 +375,20 @@ __device__ __forceinline__ double sr_column_sum(const double* partials, int npar
     for (int u = 0; u < 4; ++u)
       if (b0 + lane + 64 * u < nparts) s += v[u];
   }
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  return s;
+  return wave_sum(s);
 }
 
-// One thread: the integrals sums*hx*hy, solve_matrix
-// (symmetryReduction.cu:386-418), the advection parameters of Cxy_field
-// (:45-56) with the new c and the current phi, and, when advance, the Euler
-// update phi += dt*c (reduceSymStart stays set, main.cu:935-941) and the
-// step count.
-__device__ void sr_solve(const SrGeom& g, const double* sums, SrDev& o, bool advance, double sp,
-                         double cp) {
+// One thread: solve_matrix (symmetryReduction.cu:386-418) on the integrals
+// sums*hx*hy, and the advection parameters of Cxy_field (:45-56) with the new c
+// and the current phi (its sine and cosine sp, cp).
+struct SrSolved {
+  double c[3], ac2, axc, ayc;
+};
+__device__ __forceinline__ SrSolved sr_solve(const SrGeom& g, const double* sums, double sp,
+                                             double cp) {
   double I[12];
-  for (int p = 0; p < 12; ++p) {
-    I[p] = sums[p] * (g.hx * g.hy);
-    o.I[p] = I[p];
-  }
+#pragma unroll
+  for (int p = 0; p < 12; ++p) I[p] = sums[p] * (g.hx * g.hy);
   const double a1 = I[0] * cp + I[1] * sp, a2 = I[1] * cp - I[0] * sp, a3 = I[2];
   const double b1 = I[3] * cp + I[4] * sp, b2 = I[4] * cp - I[3] * sp, b3 = I[5];
   const double C1 = I[6] * cp + I[7] * sp, C2 = I[7] * cp - I[6] * sp, C3 = I[8];
@@ -365,15 +399,23 @@ __device__ void sr_solve(const SrGeom& g, const double* sums, SrDev& o, bool adv
   const double x3 = d3pp / c3pp;
   const double x2 = (d2p - b3p * x3) / b2p;
   const double x1 = (d1 - a2 * x2 - a3 * x3) / a1;
-  if (!(isfinite(x1) && isfinite(x2) && isfinite(x3))) o.status |= 1;
-  o.c[0] = x1;
-  o.c[1] = x2;
-  o.c[2] = x3;
+  return SrSolved{{x1, x2, x3}, x3, -x1 * cp + x2 * sp, -x1 * sp - x2 * cp};
+}
+// The state after a solve and, when advance, the Euler update phi += dt*c
+// (reduceSymStart stays set, main.cu:935-941) and the step count.
+__device__ __forceinline__ void sr_apply(const SrGeom& g, const double* sums, const SrSolved& x,
+                                         SrDev& o, bool advance) {
+#pragma unroll
+  for (int p = 0; p < 12; ++p) o.I[p] = sums[p] * (g.hx * g.hy);
+  if (!(isfinite(x.c[0]) && isfinite(x.c[1]) && isfinite(x.c[2]))) o.status |= 1;
+#pragma unroll
+  for (int p = 0; p < 3; ++p) o.c[p] = x.c[p];
   o.aphi = o.phi[2];
-  o.ac2 = x3;
-  o.axc = -x1 * cp + x2 * sp;
-  o.ayc = -x1 * sp - x2 * cp;
+  o.ac2 = x.ac2;
+  o.axc = x.axc;
+  o.ayc = x.ayc;
   if (advance) {
+#pragma unroll
     for (int p = 0; p < 3; ++p) o.phi[p] = o.phi[p] + o.c[p] * g.dt;
     o.count += 1;
   }
@@ -385,6 +427,7 @@ __device__ void sr_solve(const SrGeom& g, const double* sums, SrDev& o, bool adv
 __device__ __forceinline__ void sr_record(const SrDev& o, double* hist, long long histcap) {
   if (!hist || o.count >= histcap) return;
   double* h = hist + (size_t)o.count * 6;
+#pragma unroll
   for (int p = 0; p < 3; ++p) {
     h[p] = o.c[p];
     h[3 + p] = o.phi[p];
@@ -402,12 +445,11 @@ __global__ __launch_bounds__(768) void k_sr_solve_pre(SrGeom g, SrDev* st, const
   if (__lane_id() == 0) Is[q] = s;
   __syncthreads();
   if (threadIdx.x != 0) return;
-  SrDev o = *st;
+  SrDev& o = *st;
   sr_record(o, hist, histcap);
   double sp, cp;
   sincos(o.phi[2], &sp, &cp);
-  sr_solve(g, Is, o, false, sp, cp);
-  *st = o;
+  sr_apply(g, Is, sr_solve(g, Is, sp, cp), o, false);
 }
 
 // ----------------------------------------------------------------- BFECC
@@ -470,8 +512,8 @@ __device__ __forceinline__ BfIdx bf_index(uint32_t f, int c, int stride) {
 // neighbour.
 constexpr int kBfTX = 64, kBfTY = 16, kBfHalo = 3, kBfThreads = 1024;
 // The fused step (k_bf_rd) also takes the RD step of the new state on the
-// tile grown by one cell and the tip test on the tile, which needs the new
-// state on the tile grown by two: a halo of 3 + 2.
+// tile and the cells east and north of it and the tip test on the tile, which
+// needs the new state on the tile grown by up to two: a halo of 3 + 2.
 constexpr int kBfHaloRd = 5;
 template <int HALO>
 struct BfTile {
@@ -495,14 +537,18 @@ struct BfCells {
   static constexpr int IT = (N1 + kBfThreads - 1) / kBfThreads;
 };
 
-// Per-thread state of its cells: flags (bit 7: inside the domain, bits 5-6:
-// the advection's signs), |c| dt/h per axis, and per variable the input q,
-// the forward step uf and the corrected field ue of the cell itself.
+// Per-thread state of its cells: place and flags, |c| dt/h per axis, the LDS
+// places of the neighbours the upwind rules take (constant through the phases:
+// phases 1 and 3 read one per axis, phase 2 the two ends of a difference), and
+// per variable the input q, the forward step uf and the corrected field ue of
+// the cell itself.
 template <int NV, int HALO>
 struct BfOwn {
   static constexpr int IT = BfCells<HALO>::IT;
-  uint32_t fl[IT];
+  int at[IT];        // the cell
+  uint32_t fl[IT];   // bf_flags, bit 7: inside the domain, bits 8..: rings in from the region's edge
   float rx[IT], ry[IT];
+  int x1[IT], y1[IT], x2[IT], x3[IT], y2[IT], y3[IT];
   float q[IT][NV], f[IT][NV], e[IT][NV];
 };
 
@@ -513,48 +559,44 @@ template <int PH, int NV, int HALO = kBfHalo, bool KEEP = false>
 __device__ __forceinline__ void bf_phase(int tid, float tc, float (*s_q)[BfTile<HALO>::LN],
                                          float (*s_f)[BfTile<HALO>::LN], BfOwn<NV, HALO>& o,
                                          Fields out, int i0, int j0, int nx) {
-  constexpr int LW = BfTile<HALO>::LW, LH = BfTile<HALO>::LH;
-  constexpr int W1 = BfCells<HALO>::W1, N1 = BfCells<HALO>::N1, IT = BfCells<HALO>::IT;
+  constexpr int W1 = BfCells<HALO>::W1, IT = BfCells<HALO>::IT;
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
-    const int l = tid + it * kBfThreads;
-    const int li = 1 + l % W1, lj = 1 + l / W1;
-    const bool in_region = l < N1 && li >= PH && li < LW - PH && lj >= PH && lj < LH - PH;
     const uint32_t fl = o.fl[it];
-    if (in_region && (fl & 128u)) {  // inside the domain
-      const int L = li + LW * lj;
-      const BfIdx x = bf_index(fl, L, LW);
+    // inside the domain and in the phase's region
+    if ((fl & 128u) && (PH == 1 || (fl >> 8) >= (uint32_t)PH)) {
+      const int L = o.at[it];
       const float Rx = o.rx[it], Ry = o.ry[it];
-      const bool px = fl & 32u, py = fl & 64u;
 #pragma unroll
       for (int a = 0; a < NV; ++a) {
         if (PH == 1) {  // forward step (advFDBFECC.cu:128-131)
-          const float* q = s_q[a];
           const float qL = o.q[it][a];
-          const float FDx = px ? qL - q[x.W] : qL - q[x.E];
-          const float FDy = py ? qL - q[x.S] : qL - q[x.N];
+          const float FDx = qL - s_q[a][o.x1[it]];
+          const float FDy = qL - s_q[a][o.y1[it]];
           const float uf = qL - tc * (Rx * FDx + Ry * FDy);
           s_f[a][L] = uf;
           o.f[it][a] = uf;
         } else if (PH == 2) {  // backward step and error correction (:134-139)
           const float* f = s_f[a];
-          const float FDx = px ? f[x.iE] - f[x.E2] : f[x.iW] - f[x.W2];
-          const float FDy = py ? f[x.iN] - f[x.N2] : f[x.iS] - f[x.S2];
+          const float FDx = f[o.x2[it]] - f[o.x3[it]];
+          const float FDy = f[o.y2[it]] - f[o.y3[it]];
           const float ub = o.f[it][a] - tc * (Rx * FDx + Ry * FDy);
           const float g0 = o.q[it][a];
           const float ue = g0 - 0.5f * (ub - g0);
           s_q[a][L] = ue;  // over the input: only cell L read it there
           o.e[it][a] = ue;
         } else {  // forward step from the corrected field (:141-144)
-          const float* e = s_q[a];
           const float eL = o.e[it][a];
-          const float FDx = px ? eL - e[x.W] : eL - e[x.E];
-          const float FDy = py ? eL - e[x.S] : eL - e[x.N];
+          const float FDx = eL - s_q[a][o.x1[it]];
+          const float FDy = eL - s_q[a][o.y1[it]];
           const float r = eL - tc * (Rx * FDx + Ry * FDy);
           const float m = (fl & 1u) ? r : 0.0f;
           if (KEEP) s_f[a][L] = m;  // uf is dead after phase 2
-          if (li >= HALO && li < HALO + kBfTX && lj >= HALO && lj < HALO + kBfTY)
+          if ((fl >> 8) >= (uint32_t)HALO) {
+            const int l = tid + it * kBfThreads;
+            const int lj = 1 + l / W1, li = 1 + l - (lj - 1) * W1;
             store_through(out.f[a], (uint32_t)((i0 + li) + nx * (j0 + lj)), m);
+          }
         }
       }
     }
@@ -564,23 +606,22 @@ __device__ __forceinline__ void bf_phase(int tid, float tc, float (*s_q)[BfTile<
 // The solve and the three BFECC phases of one step on a tile with a halo of
 // HALO cells: s_q holds the state advected, then the corrected field ue;
 // s_f the forward step uf (with KEEP, then phase 3's output).  A thread's
-// cells carry their flags bf_flags | px << 5 | py << 6 | inside << 7 in
-// registers (BfOwn).
+// cells carry their flags, neighbours and values in registers (BfOwn).
 // Returns the step count of the state it advanced (from LDS).
 template <bool MASKED, int NV, int HALO, bool KEEP>
 __device__ __forceinline__ long long bf_advect(const SrGeom& g, const SrArgs& sa, CFields in,
                                           Fields out, const uint8_t* __restrict__ solid,
                                           float (*s_q)[BfTile<HALO>::LN],
                                           float (*s_f)[BfTile<HALO>::LN]) {
-  constexpr int LW = BfTile<HALO>::LW, LN = BfTile<HALO>::LN;
+  constexpr int LW = BfTile<HALO>::LW, LH = BfTile<HALO>::LH, LN = BfTile<HALO>::LN;
   constexpr int W1 = BfCells<HALO>::W1, N1 = BfCells<HALO>::N1, IC = BfCells<HALO>::IT;
   __shared__ double s_I[12];
-  __shared__ double s_adv[3];  // ac2, axc, ayc
-  __shared__ int s_cx, s_cy, s_found, s_base;
+  __shared__ SrSolved s_x;    // the solve
+  __shared__ SrStep s_step;   // the step's centre and tip count
   __shared__ SrDev s_st;      // this step's SR state
   __shared__ double s_sc[2];  // sine and cosine of its angle phi[2]
   static_assert(sizeof(SrDev) % 8 == 0 && sizeof(SrDev) / 8 <= 64, "SrDev copy by one wave");
-  static_assert(kBfThreads / 64 >= 14, "waves 12 and 13 fetch the state");
+  static_assert(kBfThreads / 64 >= 15, "waves 12 to 14 fetch the state");
   const int tid = threadIdx.x;
   const int lane = tid & 63, wv = tid >> 6;
   const int nx = g.nx, ny = g.ny;
@@ -611,9 +652,12 @@ __device__ __forceinline__ long long bf_advect(const SrGeom& g, const SrArgs& sa
 #pragma unroll
   for (int it = 0; it < IC; ++it) {
     const int l = tid + it * kBfThreads;
-    const int gi = i0 + 1 + l % W1, gj = j0 + 1 + l / W1;
+    const int li = 1 + l % W1, lj = 1 + l / W1;
+    const int gi = i0 + li, gj = j0 + lj;
     const bool ok = l < N1 && gi >= 0 && gi < nx && gj >= 0 && gj < ny;
-    o.fl[it] = ok ? (bf_flags<MASKED>(gi, gj, nx, ny, solid) | 128u) : 0u;
+    const int rings = min(min(li, LW - 1 - li), min(lj, LH - 1 - lj));
+    o.at[it] = li + LW * lj;
+    o.fl[it] = ok ? (bf_flags<MASKED>(gi, gj, nx, ny, solid) | 128u | ((uint32_t)rings << 8)) : 0u;
   }
   for (int q = wv; q < 12; q += kBfThreads / 64) {
     const double v = sr_column_sum(sa.partials, sa.nparts, q);
@@ -630,6 +674,8 @@ __device__ __forceinline__ long long bf_advect(const SrGeom& g, const SrArgs& sa
     sincos(sa.st_in->phi[2], &sp, &cp);
     s_sc[0] = sp;
     s_sc[1] = cp;
+  } else if (wv == 14 && lane == 0) {
+    s_step = *sa.step;
   }
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
@@ -642,72 +688,41 @@ __device__ __forceinline__ long long bf_advect(const SrGeom& g, const SrArgs& sa
       }
     }
   }
-  if (commit && wv == 0) {
-    int cx, cy;
-    sr_centre(g, sa.st_in, sa.step_tips, sa.step_keys, sa.step_count, cx, cy);
-    if (lane == 0) {
-      const int found = *sa.step_count;
-      s_cx = cx;
-      s_cy = cy;
-      s_found = found;
-      s_base = atomicAdd(sa.log_count, found);
-    }
-  }
   __syncthreads();
-  // 2 the solve, in every workgroup from the same sums; workgroup 0 writes
-  //   the next state slot and moves this step's tips to the log
-  if (tid == 0) {
-    SrDev o = s_st;
-    if (commit && sa.record) sr_record(o, sa.hist, sa.histcap);
-    sr_solve(g, s_I, o, true, s_sc[0], s_sc[1]);
-    s_adv[0] = o.ac2;
-    s_adv[1] = o.axc;
-    s_adv[2] = o.ayc;
-    if (commit) {
-      o.cx = s_cx;
-      o.cy = s_cy;
-      o.ntips = s_found;
-      *sa.st_out = o;
-    }
-  }
-  if (commit) {
-    const int n = min(s_found, kSrTipCap);
-    for (int q = tid; q < n; q += kBfThreads) {
-      const int slot = s_base + q;
-      if (slot < sa.logcap) {
-        sa.log_tips[slot] = sa.step_tips[q];
-        sa.log_keys[slot] = sa.step_keys[q];
-      }
-    }
-  }
+  // 2 the solve, in every workgroup from the same sums
+  if (tid == 0) s_x = sr_solve(g, s_I, s_sc[0], s_sc[1]);
   __syncthreads();
-  if (commit && tid == 0) *sa.step_count = 0;
   // 3 advection coefficients of this thread's cells (Cxy_field_kernel,
-  //   symmetryReduction.cu:45-56, negated as at advFDBFECC.cu:30-31) and
-  //   their input values; phase 1 reads nothing else another thread wrote
-  //   after the barrier above
-  const double ac2 = s_adv[0], axc = s_adv[1], ayc = s_adv[2];
+  //   symmetryReduction.cu:45-56, negated as at advFDBFECC.cu:30-31), the
+  //   neighbours their signs select and their input values; phase 1 reads
+  //   nothing else another thread wrote after the barrier above
+  const double ac2 = s_x.ac2, axc = s_x.axc, ayc = s_x.ayc;
 #pragma unroll
   for (int it = 0; it < IC; ++it) {
     const int l = tid + it * kBfThreads;
     const int li = 1 + l % W1, lj = 1 + l / W1;
-    uint32_t fl = o.fl[it];
-    float rx = 0.0f, ry = 0.0f;
+    const uint32_t fl = o.fl[it];
+    const int L = o.at[it];
+    o.rx[it] = o.ry[it] = 0.0f;
     if (fl & 128u) {
       const int gi = i0 + li, gj = j0 + lj;
       double ax = g.hy * (double)gj * ac2 + axc;
       double ay = -g.hx * (double)gi * ac2 + ayc;
       if (MASKED && !(fl & 1u)) ax = ay = 0.0;  // Cxy_field_kernel :50-51
       const double cx = -ax, cy = -ay;          // advFDBFECC.cu:30-31
-      rx = (float)(fabs(cx) * g.dtx);
-      ry = (float)(fabs(cy) * g.dty);
-      fl |= (cx > 0.0 ? 32u : 0u) | (cy > 0.0 ? 64u : 0u);
+      o.rx[it] = (float)(fabs(cx) * g.dtx);
+      o.ry[it] = (float)(fabs(cy) * g.dty);
+      const bool px = cx > 0.0, py = cy > 0.0;
+      const BfIdx x = bf_index(fl, L, LW);
+      o.x1[it] = px ? x.W : x.E;
+      o.y1[it] = py ? x.S : x.N;
+      o.x2[it] = px ? x.iE : x.iW;
+      o.x3[it] = px ? x.E2 : x.W2;
+      o.y2[it] = py ? x.iN : x.iS;
+      o.y3[it] = py ? x.N2 : x.S2;
 #pragma unroll
-      for (int a = 0; a < NV; ++a) o.q[it][a] = s_q[a][li + LW * lj];
+      for (int a = 0; a < NV; ++a) o.q[it][a] = s_q[a][L];
     }
-    o.rx[it] = rx;
-    o.ry[it] = ry;
-    o.fl[it] = fl;
   }
   const float tc = (float)g.tc;
   bf_phase<1, NV, HALO>(tid, tc, s_q, s_f, o, out, i0, j0, nx);
@@ -715,6 +730,17 @@ __device__ __forceinline__ long long bf_advect(const SrGeom& g, const SrArgs& sa
   bf_phase<2, NV, HALO>(tid, tc, s_q, s_f, o, out, i0, j0, nx);
   __syncthreads();
   bf_phase<3, NV, HALO, KEEP>(tid, tc, s_q, s_f, o, out, i0, j0, nx);
+  // 4 workgroup 0 writes the next state slot
+  if (commit && tid == 0) {
+    SrDev n = s_st;
+    if (sa.record) sr_record(n, sa.hist, sa.histcap);
+    sr_apply(g, s_I, s_x, n, true);
+    n.cx = s_step.cx;
+    n.cy = s_step.cy;
+    n.ntips = s_step.found;
+    *sa.st_out = n;
+    *sa.step_count = 0;
+  }
   return s_st.count;
 }
 
@@ -730,11 +756,18 @@ __global__ __launch_bounds__(kBfThreads) void k_bf_fused(SrGeom g, SrArgs sa, CF
 // halo of kBfHaloRd, keeping the new state of the tile grown by two cells in
 // LDS), then the RD step and the tip test of the next step, which
 // k_sr_rdtips would otherwise take in a launch of its own:
-//   RD of the new state on the tile grown by one, with cell_update (the
-//   arithmetic of k_sr_rdtips, bit for bit), its output of the tile to
-//   xo_out and its u to LDS;
+//   RD of the new state on the tile and the cells east and north of it, with
+//   cell_update (the arithmetic of k_sr_rdtips, bit for bit), its output of
+//   the tile to xo_out and its u to LDS;
 //   the tips of the tile between the new state (g_present) and its RD output
 //   (g_past) into the next step's tip buffer, stamped with the next count.
+// What bounds a step is its chain of dependent parts, 256 workgroups of 16
+// waves at 512 x 512: a launch, the columns, the solve, three phases and RD
+// with a barrier between them.  So a thread works out the places of its cells'
+// neighbours once rather than in every phase, the tips leave the chain for
+// k_sr_slices, the column sums add by lane moves instead of trips through LDS,
+// and RD takes one cell a thread and then the ring (FK at 512 x 512: this
+// kernel 10.0 -> 8.1 us, k_sr_slices 5.8 -> 5.0, a step 15.3 -> 12.7).
 template <int MODEL, bool MASKED>
 __global__ __launch_bounds__(kBfThreads) void k_bf_rd(const KParams k, SrGeom g, SrArgs sa,
                                                        CFields in, Fields out, Fields xo_out,
@@ -753,14 +786,19 @@ __global__ __launch_bounds__(kBfThreads) void k_bf_rd(const KParams k, SrGeom g,
   const int nx = g.nx, ny = g.ny;
   const int i0 = blockIdx.x * kBfTX - H, j0 = blockIdx.y * kBfTY - H;
   const float* f[3] = {s_f[0], s_f[1], s_f[NV - 1]};
-  constexpr int RW = kBfTX + 2, RN = RW * (kBfTY + 2);
-  for (int l = tid; l < RN; l += kBfThreads) {
-    const int li = H - 1 + l % RW, lj = H - 1 + l / RW;
+  // the tile's cells, one a thread, then those east and north of it, whose
+  // new u the tip test of the tile's cells reads
+  static_assert(kBfTX * kBfTY == kBfThreads, "one cell of the tile per thread");
+  constexpr int RING = kBfTX + 1 + kBfTY;
+  for (int l = tid; l < kBfThreads + RING; l += kBfThreads) {
+    const int r = l - kBfThreads;
+    const int li = H + (r < 0 ? l % kBfTX : min(r, kBfTX));
+    const int lj = H + (r < 0 ? l / kBfTX : r <= kBfTX ? kBfTY : r - kBfTX - 1);
     const int gi = i0 + li, gj = j0 + lj;
-    if (gi < 0 || gi >= nx || gj < 0 || gj >= ny) continue;
+    if (gi >= nx || gj >= ny) continue;
     const int L = li + LW * lj;
-    const int Lw = (mirror(gi - 1, nx) - i0) + LW * lj, Le = (mirror(gi + 1, nx) - i0) + LW * lj;
-    const int Ln = li + LW * (mirror(gj + 1, ny) - j0), Ls = li + LW * (mirror(gj - 1, ny) - j0);
+    const int Lw = gi > 0 ? L - 1 : L + 1, Le = gi < nx - 1 ? L + 1 : L - 1;
+    const int Ln = gj < ny - 1 ? L + LW : L - LW, Ls = gj > 0 ? L - LW : L + LW;
     float cW = 1.f, cE = 1.f, cN = 1.f, cS = 1.f;
     bool sc = true;
     if (MASKED) {  // cell_update_codes
@@ -775,7 +813,7 @@ __global__ __launch_bounds__(kBfThreads) void k_bf_rd(const KParams k, SrGeom g,
     float xo[3], inc[3];
     cell_update<MODEL>(k, f, L, Lw, Le, Ln, Ls, cW, cE, cN, cS, sc, xo, inc);
     s_ro[L] = xo[0];
-    if (li >= H && li < H + kBfTX && lj >= H && lj < H + kBfTY) {
+    if (r < 0) {
 #pragma unroll
       for (int a = 0; a < NV; ++a) store_through(xo_out.f[a], (uint32_t)(gi + nx * gj), xo[a]);
     }
@@ -810,6 +848,7 @@ struct yh_sr {
   yh_tip* step_tips = nullptr;
   int* step_keys = nullptr;
   int* step_count = nullptr;
+  yh::SrStep* step = nullptr;  // this step's centre and tip count
   float* xo2[3] = {nullptr, nullptr, nullptr};  // RD output of odd steps (two launches)
   bool pending = false;      // the RD output and tips of step `count` are computed ...
   long long epoch = -1;      // ... from the state of this plan state epoch
@@ -848,6 +887,7 @@ void sr_free(yh_sr* sr) {
   if (sr->step_tips) (void)hipFree(sr->step_tips);
   if (sr->step_keys) (void)hipFree(sr->step_keys);
   if (sr->step_count) (void)hipFree(sr->step_count);
+  if (sr->step) (void)hipFree(sr->step);
   for (float* q : sr->xo2)
     if (q) (void)hipFree(q);
   if (sr->hist) (void)hipFree(sr->hist);
@@ -883,10 +923,9 @@ static int disk_reach(int r2) {
 
 template <int MODEL, bool MASKED>
 static void sr_launch_slices(const yh_plan* pl, const SrGeom& g, int R, CFields X, const SrDev* st,
-                             const yh_tip* tips, const int* keys, const int* cnt, dim3 sg,
-                             dim3 sb, hipStream_t s) {
+                             const SrTips& tp, int log, dim3 sg, dim3 sb, hipStream_t s) {
   hipLaunchKernelGGL((k_sr_slices<MODEL, MASKED>), sg, sb, 0, s, pl->k, g, R, X, pl->codes_d, st,
-                     tips, keys, cnt, pl->sr->partials);
+                     tp, log, pl->sr->partials);
 }
 
 // Clears a step's tip count with a kernel (capturable, unlike a memset).
@@ -940,13 +979,15 @@ static int sr_enqueue(yh_plan* pl, bool first, bool need_rd, int slot, hipStream
   // 2 slices + inner products over the moving disk's box (at count 0 first
   //   the preliminary pass and its solve, in place)
   dim3 sb(kSliceBX, kSliceBY), sg((box + kSliceBX - 1) / kSliceBX, (box + kSliceBY - 1) / kSliceBY);
-  for (int pass = first ? 0 : 1; pass < 2; ++pass) {
+  const SrTips tp{tips,          keys,         cnt, pl->tips_d, pl->keys_d, pl->tipcount_d,
+                  pl->tipcap, sr->step};
+  for (int pass = first ? 0 : 1; pass < 2; ++pass) {  // the second logs the tips
     if (model == M2V) {
-      if (masked) sr_launch_slices<M2V, true>(pl, g, R, X, st_in, tips, keys, cnt, sg, sb, s);
-      else sr_launch_slices<M2V, false>(pl, g, R, X, st_in, tips, keys, cnt, sg, sb, s);
+      if (masked) sr_launch_slices<M2V, true>(pl, g, R, X, st_in, tp, pass, sg, sb, s);
+      else sr_launch_slices<M2V, false>(pl, g, R, X, st_in, tp, pass, sg, sb, s);
     } else {
-      if (masked) sr_launch_slices<MFK, true>(pl, g, R, X, st_in, tips, keys, cnt, sg, sb, s);
-      else sr_launch_slices<MFK, false>(pl, g, R, X, st_in, tips, keys, cnt, sg, sb, s);
+      if (masked) sr_launch_slices<MFK, true>(pl, g, R, X, st_in, tp, pass, sg, sb, s);
+      else sr_launch_slices<MFK, false>(pl, g, R, X, st_in, tp, pass, sg, sb, s);
     }
     YH_HIP(hipGetLastError());
     if (pass == 0) {
@@ -965,13 +1006,8 @@ static int sr_enqueue(yh_plan* pl, bool first, bool need_rd, int slot, hipStream
   sa.record = first ? 0 : 1;  // at count 0 the preliminary solve recorded
   sa.hist = sr->hist;
   sa.histcap = sr->histcap;
-  sa.step_tips = tips;
-  sa.step_keys = keys;
+  sa.step = sr->step;
   sa.step_count = cnt;
-  sa.log_tips = pl->tips_d;
-  sa.log_keys = pl->keys_d;
-  sa.log_count = pl->tipcount_d;
-  sa.logcap = pl->tipcap;
   sa.next_tips = sr->step_tips + (size_t)(tb ^ 1) * kSrTipCap;
   sa.next_keys = sr->step_keys + (size_t)(tb ^ 1) * kSrTipCap;
   sa.next_count = sr->step_count + (tb ^ 1);
@@ -1025,6 +1061,7 @@ int yh_sr_begin(yh_plan* pl, float tip0x, float tip0y, void* stream) {
   if (!sr->step_tips) YH_HIP(hipMalloc(&sr->step_tips, 2 * sizeof(yh_tip) * kSrTipCap));
   if (!sr->step_keys) YH_HIP(hipMalloc(&sr->step_keys, 2 * sizeof(int) * kSrTipCap));
   if (!sr->step_count) YH_HIP(hipMalloc(&sr->step_count, 2 * sizeof(int)));
+  if (!sr->step) YH_HIP(hipMalloc(&sr->step, sizeof(SrStep)));
   for (int a = 0; a < pl->nv; ++a)
     if (!sr->xo2[a]) YH_HIP(hipMalloc(&sr->xo2[a], pl->n * sizeof(float)));
   SrDev h[2];
