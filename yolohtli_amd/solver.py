@@ -9,6 +9,7 @@ Errors raise ``YhError`` carrying the C error code; nothing here computes on
 the CPU.
 """
 import ctypes as C
+import sys
 
 import numpy as np
 
@@ -16,6 +17,7 @@ from . import abi_types as T
 from ._lib import check, lib
 
 BASE_SEED = 20261202
+_Ptr3 = C.c_void_p * 3  # fields u, v, w; those a model lacks stay null
 
 
 def _ptr(a):
@@ -74,7 +76,18 @@ def _dev_ptr(t):
 
 
 def _stream_handle(stream):
+    """The handle of `stream`, by default torch's current stream.
+
+    Once torch has initialised the device its raw handle is asked for: 0.4 us
+    against 3.4 us for the availability test and a Stream object, of the 10.2 us
+    that one 512 x 512 step took, 3.9 of them its launch."""
     if stream is None:
+        torch = sys.modules.get("torch")
+        try:
+            if torch is not None and torch.cuda.is_initialized():
+                return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        except AttributeError:  # not every torch has these
+            pass
         try:
             import torch
             if torch.cuda.is_available():
@@ -90,12 +103,9 @@ def reactionDiffusion_wrapper(p, gOut, gIn, velTan=None, solid=None, stream=None
     """One time step on caller-owned device fields (lists of tensors u,v[,w]);
     stimLockMouse/point: the mouse stimulus of reactionDiffusion.cu:54-61."""
     nv = T.nvars(p)
-    arr = C.c_void_p * 3
-    out = arr(*([_dev_ptr(x) for x in gOut[:nv]] + [None] * (3 - nv)))
-    inp = arr(*([_dev_ptr(x) for x in gIn[:nv]] + [None] * (3 - nv)))
-    vt = None
-    if velTan is not None:
-        vt = arr(*([_dev_ptr(x) for x in velTan[:nv]] + [None] * (3 - nv)))
+    out = _Ptr3(*[_dev_ptr(x) for x in gOut[:nv]])
+    inp = _Ptr3(*[_dev_ptr(x) for x in gIn[:nv]])
+    vt = None if velTan is None else _Ptr3(*[_dev_ptr(x) for x in velTan[:nv]])
     check(lib().yh_rd_step_dev_ex(C.byref(p), out, inp, vt, _dev_ptr(solid),
                                   int(bool(stimLockMouse)), int(point[0]), int(point[1]),
                                   _stream_handle(stream)), "yh_rd_step_dev_ex")
