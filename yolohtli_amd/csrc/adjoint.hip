@@ -28,24 +28,28 @@
 
 #include "lanes.h"
 #include "plan.h"
+#include "tile.h"
 
 namespace yh {
 
 struct AdjK {
   int nx, ny;
-  float rxh, ryh;  // dt/hx^2, dt/hy^2
-  float dt, tc;
-  float hw;        // Heaviside width
-  float td, tr, tsi, t0, tvp, tv1m, tv2m, twp, twm, uc, uv, ucsi, kk;
-  // reciprocals, rounded once on the host from FP64: 1/hw, 2/hw, 1/tau_d,
-  // 1/tau_r, 0.5/tau_si, 1/tau_0, 1/tau_v+, 1/tau_w-, 1/tau_w+
-  float ihw, tihw, itd, itr, ihtsi, it0, itvp, itwm, itwp;
+  float rxt, ryt;  // tc dt / (2 hx^2), tc dt / (2 hy^2)
+  float tdt;       // tc dt
+  float uc, uv, ucsi, uc1;  // uc1 = 1 + u_c
+  float tv1m, tv2m, dtv;    // tau_v1-, tau_v2-, tau_v2- - tau_v1-
+  // rounded once on the host from FP64: 2/(w ln 2) and 2k/ln 2 (sigmoid2's
+  // exponents), 2/w, 1/tau_d, 1/tau_r, 1/tau_si, 2k/tau_si, 1/tau_0, 1/tau_v+,
+  // 1/tau_w-, 1/tau_w+
+  float eh, es, tihw, itd, itr, itsi, ksi, it0, itvp, itwm, itwp;
 };
 
+// Currents and gate rates of a cell (dv/dt = A, dw/dt = B), their derivatives
+// (of -A and -B), and the products that both share with the time constants'.
 struct FkEval {
-  float I, Gv, Gw;
-  float dIdu, dIdv, dIdw, dGvdu, dGvdv, dGwdu, dGwdw;
-  float p, pc, Jfi, Jsi;  // what the time-constant derivatives are made of
+  float I, A, B;
+  float Iu, Iv, Iw, Gvu, Gvv, Gwu, Gww;
+  float p, vpf, ws, upc, vp, pw;
 };
 
 // Correctly rounded 1/t: the hardware reciprocal (within 1 ulp) and one
@@ -56,88 +60,64 @@ __device__ __forceinline__ float recip(float t) {
   return __builtin_fmaf(__builtin_fmaf(-t, r, 1.0f), r, r);
 }
 
-// s = sigmoid(2y) = 0.5*(1 + tanh y) and its complement sc = 1 - s, both
-// from a = exp(-2|y|) in (0, 1] with the hardware exp2 and reciprocal:
-// the larger is 1/(1 + a), the smaller a/(1 + a), so each keeps a relative
-// error of a few ulp (1 - 2/(exp(2y) + 1) loses the smaller one, and
-// 1 - tanh^2, to cancellation: 2e-3 relative at |y| = 5).
-__device__ __forceinline__ void sigmoid2(float y, float* s, float* sc) {
+// s = sigmoid(e ln 2 x) = 0.5*(1 + tanh(e ln 2 x/2)) and its complement
+// sc = 1 - s, both from a = exp2(-e|x|) in (0, 1] with the hardware exp2 and
+// reciprocal: the larger is 1/(1 + a), the smaller a/(1 + a), so each keeps a
+// relative error of a few ulp (1 - 2/(exp(2y) + 1) loses the smaller one, and
+// 1 - tanh^2, to cancellation: 2e-3 relative at tanh's argument 5).
+__device__ __forceinline__ void sigmoid2(float x, float e, float* s, float* sc) {
 #pragma clang fp contract(off)
-  const float a = __builtin_amdgcn_exp2f(-2.8853900817779268f * __builtin_fabsf(y));  // 2/ln 2
+  const float a = __builtin_amdgcn_exp2f(-e * __builtin_fabsf(x));
   const float big = __builtin_amdgcn_rcpf(1.0f + a);
   const float small = a * big;
-  *s = y >= 0.0f ? big : small;
-  *sc = y >= 0.0f ? small : big;
+  *s = x >= 0.0f ? big : small;
+  *sc = x >= 0.0f ? small : big;
 }
 
-// Smoothed Heaviside h = 0.5*(1 + tanh(x/w)), its complement hc = 1 - h and
-// its derivative dh = (1 - tanh^2)/(2w) = (2/w) h (1 - h).
-__device__ __forceinline__ void heav(float x, float iw, float tiw, float* h, float* hc,
-                                     float* dh) {
-#pragma clang fp contract(off)
-  sigmoid2(x * iw, h, hc);
-  *dh = tiw * (*h * *hc);
-}
-
-// Fenton & Karma 1998 currents and derivatives (smoothed Heaviside).  No
-// FMA contraction here or in adj_fwd_cell: every operation rounds on its
-// own, so the kernels that inline them agree bit for bit.  pc = 1 - p and
-// qc = 1 - q come from heav(); 1 + tanh(k(u - u_csi)) = 2 ss and
-// 1 - tanh^2 = 4 ss ssc with (ss, ssc) = sigmoid2(k(u - u_csi)).
+// Fenton & Karma 1998 currents and derivatives with the Heaviside smoothed to
+// p = 0.5*(1 + tanh((u - u_c)/w)) (q at u_v), p' = (2/w) p (1 - p).  Every fma
+// is written out and contraction is off, here and in what is built on it, so
+// the kernels that inline them agree bit for bit.  A step is bound by VALU
+// issue, so the sums share their products and constants are folded: a reverse
+// step takes about 115 instructions in a ring cell and 155 in a tile cell, 165
+// and 290 with the formulas as they stand and every operation rounded.  The
+// gradients are as far from 64 bits as those (256 x 256, 2000 steps: 6e-6).
 __device__ __forceinline__ FkEval fk_eval(const AdjK& k, float u, float v, float w) {
 #pragma clang fp contract(off)
   FkEval r;
-  float p, pc, dp, q, qc, dq, ss, ssc;
-  heav(u - k.uc, k.ihw, k.tihw, &p, &pc, &dp);
-  heav(u - k.uv, k.ihw, k.tihw, &q, &qc, &dq);
-  const float f = (1.0f - u) * (u - k.uc);
-  const float df = 1.0f + k.uc - 2.0f * u;
-  const float Jfi = -v * p * f * k.itd;
-  const float Jso = u * pc * k.it0 + p * k.itr;
-  sigmoid2(k.kk * (u - k.ucsi), &ss, &ssc);
-  const float opth = 2.0f * ss;           // 1 + tanh
-  const float sech2 = 4.0f * (ss * ssc);  // 1 - tanh^2
-  const float Jsi = -w * opth * k.ihtsi;
-  r.I = Jfi + Jso + Jsi;
-  r.dIdu = -v * (dp * f + p * df) * k.itd + pc * k.it0 - u * dp * k.it0 + dp * k.itr -
-           w * k.kk * sech2 * k.ihtsi;
-  r.dIdv = -p * f * k.itd;
-  r.dIdw = -opth * k.ihtsi;
-  const float tvm = qc * k.tv1m + q * k.tv2m;
-  const float itvm = recip(tvm);
-  const float dtvm = dq * (k.tv2m - k.tv1m);
-  const float A = pc * (1.0f - v) * itvm - p * v * k.itvp;
-  const float dAdu = -dp * (1.0f - v) * itvm - pc * (1.0f - v) * dtvm * (itvm * itvm) -
-                     dp * v * k.itvp;
-  const float dAdv = -pc * itvm - p * k.itvp;
-  const float B = pc * (1.0f - w) * k.itwm - p * w * k.itwp;
-  const float dBdu = -dp * (1.0f - w) * k.itwm - dp * w * k.itwp;
-  const float dBdw = -pc * k.itwm - p * k.itwp;
-  r.Gv = -A;
-  r.Gw = -B;
-  r.dGvdu = -dAdu;
-  r.dGvdv = -dAdv;
-  r.dGwdu = -dBdu;
-  r.dGwdw = -dBdw;
+  float p, pc, q, qc, ss, ssc;
+  const float a = u - k.uc;
+  sigmoid2(a, k.eh, &p, &pc);
+  sigmoid2(u - k.uv, k.eh, &q, &qc);
+  sigmoid2(u - k.ucsi, k.es, &ss, &ssc);
+  const float f = (1.0f - u) * a, pf = p * f;
   r.p = p;
-  r.pc = pc;
-  r.Jfi = Jfi;
-  r.Jsi = Jsi;
+  r.vp = v * p;
+  r.pw = w * p;
+  r.vpf = v * pf;
+  r.ws = w * ss;
+  r.upc = u * pc;
+  // J_fi = -v p f/tau_d, J_so = u (1 - p)/tau_0 + p/tau_r, J_si = -w ss/tau_si
+  r.I = __builtin_fmaf(-r.ws, k.itsi,
+                       __builtin_fmaf(-r.vpf, k.itd, __builtin_fmaf(r.upc, k.it0, p * k.itr)));
+  const float itvm = recip(__builtin_fmaf(q, k.tv2m, qc * k.tv1m));
+  const float ov = (1.0f - v) * itvm, ow = (1.0f - w) * k.itwm;
+  const float open = pc * ov;
+  r.A = __builtin_fmaf(-r.vp, k.itvp, open);
+  r.B = __builtin_fmaf(-r.pw, k.itwp, pc * ow);
+  const float dp = k.tihw * (p * pc), dq = k.tihw * (q * qc);
+  const float dpf = __builtin_fmaf(dp, f, p * __builtin_fmaf(-2.0f, u, k.uc1));
+  float Iu = __builtin_fmaf(-u, dp, pc) * k.it0;
+  Iu = __builtin_fmaf(dp, k.itr, Iu);
+  Iu = __builtin_fmaf(-(v * dpf), k.itd, Iu);
+  r.Iu = __builtin_fmaf(-(r.ws * ssc), k.ksi, Iu);
+  r.Iv = -(pf * k.itd);
+  r.Iw = -(ss * k.itsi);
+  r.Gvu = __builtin_fmaf(open * itvm, dq * k.dtv, dp * __builtin_fmaf(v, k.itvp, ov));
+  r.Gvv = __builtin_fmaf(p, k.itvp, pc * itvm);
+  r.Gwu = dp * __builtin_fmaf(w, k.itwp, ow);
+  r.Gww = __builtin_fmaf(p, k.itwp, pc * k.itwm);
   return r;
-}
-
-// The terms of dL/dtau (tau_d, tau_r, tau_si, tau_0, tau_v+, tau_w+) of one
-// cell and step, from mu, mv, mw = lambda of the step's result.
-__device__ __forceinline__ void fk_taus(const AdjK& k, const FkEval& r, float u, float v, float w,
-                                        float mu, float mv, float mw, float gt[6]) {
-#pragma clang fp contract(off)
-  const float tdt = k.tc * k.dt;
-  gt[0] = mu * (-tdt * (-r.Jfi * k.itd));
-  gt[1] = mu * (-tdt * (-r.p * (k.itr * k.itr)));
-  gt[2] = mu * (-tdt * (-2.0f * r.Jsi * k.ihtsi));
-  gt[3] = mu * (-tdt * (-u * r.pc * (k.it0 * k.it0)));
-  gt[4] = mv * (-tdt * (-r.p * v * (k.itvp * k.itvp)));
-  gt[5] = mw * (-tdt * (-r.p * w * (k.itwp * k.itwp)));
 }
 
 struct Coef4 {
@@ -170,19 +150,21 @@ __device__ __forceinline__ Coef4 coef_from_code(uint32_t b) {
   r.S = (float)((q >> 6) & 3u);
   return r;
 }
-constexpr uint8_t kCodeAllOnes = 0x55;  // cW = cE = cN = cS = 1: no mask
 
 // ---------------------------------------------------------------- forward
-// Diffusion weights of a cell, c * (D_c + D_n) / 2 per direction: constant
-// through the steps.
+// Weights r (D_c + D_n) of a cell's four links, r = tc dt/(2h^2), and the
+// cell's own coefficients times them: constant through the steps.
 struct AdjDif {
   float W, E, N, S;
 };
-__device__ __forceinline__ AdjDif adj_dif(const Coef4& cf, float Dc, float DW, float DE, float DN,
-                                          float DS) {
+__device__ __forceinline__ AdjDif adj_links(const AdjK& k, float Dc, float DW, float DE, float DN,
+                                            float DS) {
 #pragma clang fp contract(off)
-  return AdjDif{cf.W * 0.5f * (Dc + DW), cf.E * 0.5f * (Dc + DE), cf.N * 0.5f * (Dc + DN),
-                cf.S * 0.5f * (Dc + DS)};
+  return AdjDif{k.rxt * (Dc + DW), k.rxt * (Dc + DE), k.ryt * (Dc + DN), k.ryt * (Dc + DS)};
+}
+__device__ __forceinline__ AdjDif adj_dif(const Coef4& c, const AdjDif& l) {
+#pragma clang fp contract(off)
+  return AdjDif{c.W * l.W, c.E * l.E, c.N * l.N, c.S * l.S};
 }
 
 // One forward step of one cell from its state, its four (mirror) neighbours'
@@ -192,12 +174,14 @@ __device__ __forceinline__ void adj_fwd_cell(const AdjK& k, float u, float v, fl
                                              float uE, float uN, float uS, const AdjDif& a,
                                              bool tissue, float& un, float& vn, float& wn) {
 #pragma clang fp contract(off)
-  const float lap = k.rxh * (a.W * (uW - u) + a.E * (uE - u)) +
-                    k.ryh * (a.N * (uN - u) + a.S * (uS - u));
+  float d = a.W * (uW - u);
+  d = __builtin_fmaf(a.E, uE - u, d);
+  d = __builtin_fmaf(a.N, uN - u, d);
+  d = __builtin_fmaf(a.S, uS - u, d);
   const FkEval r = fk_eval(k, u, v, w);
-  un = tissue ? u + k.tc * (lap - k.dt * r.I) : 0.0f;
-  vn = tissue ? v + k.tc * (-k.dt * r.Gv) : 0.0f;
-  wn = tissue ? w + k.tc * (-k.dt * r.Gw) : 0.0f;
+  un = tissue ? u + __builtin_fmaf(-k.tdt, r.I, d) : 0.0f;
+  vn = tissue ? __builtin_fmaf(k.tdt, r.A, v) : 0.0f;
+  wn = tissue ? __builtin_fmaf(k.tdt, r.B, w) : 0.0f;
 }
 
 __global__ __launch_bounds__(256) void k_adj_fwd(const AdjK k, CFields in, Fields out,
@@ -216,7 +200,7 @@ __global__ __launch_bounds__(256) void k_adj_fwd(const AdjK k, CFields in, Field
   const float* U = in.f[0];
   float un, vn, wn;
   adj_fwd_cell(k, U[c], in.f[1][c], in.f[2][c], U[W], U[E], U[N], U[S],
-               adj_dif(cf, D[c], D[W], D[E], D[N], D[S]), cf.sc, un, vn, wn);
+               adj_dif(cf, adj_links(k, D[c], D[W], D[E], D[N], D[S])), cf.sc, un, vn, wn);
   out.f[0][c] = un;
   out.f[1][c] = vn;
   out.f[2][c] = wn;
@@ -295,7 +279,9 @@ __device__ __forceinline__ AdjAt adj_at(const AdjCell& c, int ox0, int oy0, int 
                c.y > 0 ? l - kAdjStride : l + kAdjStride};
 }
 
-// K forward steps.  Outputs: with seg, the state after every step into seg
+// K forward steps, their states written through to memory (left dirty in the
+// XCD's L2 they delay the end of the launch: 10.1 against 9.4 us for 8 steps of
+// 256 x 256).  Outputs: with seg, the state after every step into seg
 // slots slot0+1 .. slot0+K; otherwise the final state into out.  Sensor traces for every step with step % rec == 0.
 template <bool MASKED>
 __global__ __launch_bounds__(kAdjThreads) void k_adj_fwd_tiled(
@@ -304,7 +290,8 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_fwd_tiled(
     int rec, float* __restrict__ traces, int ns, float* __restrict__ seg, size_t n, int slot0) {
   __shared__ float s_u[2][kAdjLds], s_D[kAdjLds];
   const int nx = k.nx, ny = k.ny;
-  const int ty = blockIdx.x / t.tiles_x, tx = blockIdx.x - ty * t.tiles_x;
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int ty = tile / t.tiles_x, tx = tile - ty * t.tiles_x;
   const int ox0 = tx * t.tw, oy0 = ty * t.th;
   const AdjCell q = adj_cell(threadIdx.x, ox0, oy0, t, K, nx, ny);
   const AdjAt at = adj_at(q, ox0, oy0, K, nx, ny);
@@ -324,7 +311,8 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_fwd_tiled(
   }
   __syncthreads();
   AdjDif a{};
-  if (q.m < K) a = adj_dif(cf, Dc, s_D[at.W], s_D[at.E], s_D[at.N], s_D[at.S]);
+  if (q.m < K)
+    a = adj_dif(cf, adj_links(k, Dc, s_D[at.W], s_D[at.E], s_D[at.N], s_D[at.S]));
   // the state after step step0 + s + 1, and the recorded steps to come: `left`
   // steps to the next one, whose row is `row`
   float* slot = seg ? seg + (size_t)(slot0 + 1) * 3 * n : nullptr;
@@ -342,13 +330,13 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_fwd_tiled(
       s_u[(s & 1) ^ 1][at.l] = u;
       if (q.m == 0) {
         if (seg) {
-          slot[c] = u;
-          slot[n + c] = v;
-          slot[2 * n + c] = w;
+          store_through(slot, (uint32_t)c, u);
+          store_through(slot + n, (uint32_t)c, v);
+          store_through(slot + 2 * n, (uint32_t)c, w);
         } else if (s == K - 1) {
-          out.f[0][c] = u;
-          out.f[1][c] = v;
-          out.f[2][c] = w;
+          store_through(out.f[0], (uint32_t)c, u);
+          store_through(out.f[1], (uint32_t)c, v);
+          store_through(out.f[2], (uint32_t)c, w);
         }
         if (left == 1 && sensor >= 0) row[sensor] = u;
       }
@@ -405,74 +393,80 @@ static hipError_t launch_adj_fwd_tiled(const AdjK& k, const AdjTile& t, CFields 
 }
 
 // ---------------------------------------------------------------- reverse
-// One reverse step of one cell (i, j): lam_out = J(X)^T lam_in (+ source),
-// its dL/dD term gd and its dL/dtau terms gt.  X is the state the forward
-// step started from.  The accessor gives u of X, D, lambda_u of lam_in and
-// the stencil code at offsets (di, dj) from the cell; every offset used is a
-// cell of the domain.  Shared by both reverse kernels (no contraction), so
-// they agree bit for bit on lambda and on each step's terms.
-template <class Acc>
-__device__ __forceinline__ void adj_rev_cell(const AdjK& k, const Acc& A, int i, int j, float v,
-                                             float w, float lv_in, float lw_in, float src,
-                                             float& lu, float& lv, float& lw, double& gd,
-                                             float gt[6]) {
+// The transposed operator at a cell: cw the coefficients with which the updates
+// of its west, east, north and south neighbours read it, an edge neighbour's
+// mirror image of it included (0 where there is no neighbour), from the
+// neighbours' own coefficients; a = cw times the links' weights, and one the
+// cell's own row, 1 - the sum of its weights.
+struct AdjCol {
+  Coef4 cw;
+  AdjDif a;
+  float one;
+};
+__device__ __forceinline__ AdjCol adj_col(const AdjDif& l, int x, int y, int nx, int ny,
+                                          const Coef4& cf, const Coef4& cW, const Coef4& cE,
+                                          const Coef4& cN, const Coef4& cS) {
 #pragma clang fp contract(off)
-  const int nx = k.nx, ny = k.ny;
-  const Coef4 cf = coef_from_code(A.code(0, 0));
-  const float u = A.U(0, 0);
-  const float m = cf.sc ? 1.0f : 0.0f;
-  const float mu = m * A.LU(0, 0), mv = m * lv_in, mw = m * lw_in;
-  const float Dc = A.D(0, 0);
-  const float tc = k.tc;
-  // own diffusion terms, neighbours W, E, N, S by mirror (helper_functions.cu:69-79)
-  const int ox[4] = {i > 0 ? -1 : 1, i < nx - 1 ? 1 : -1, 0, 0};
-  const int oy[4] = {0, 0, j < ny - 1 ? 1 : -1, j > 0 ? -1 : 1};
-  const float co[4] = {cf.W, cf.E, cf.N, cf.S};
-  const float rr[4] = {k.rxh, k.rxh, k.ryh, k.ryh};
-  float asum = 0.0f;
-  gd = 0.0;
-#pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    asum += rr[d] * co[d] * 0.5f * (Dc + A.D(ox[d], oy[d]));
-    gd += (double)(tc * mu * rr[d] * co[d] * 0.5f * (A.U(ox[d], oy[d]) - u));
-  }
-  // coefficients pointing at this cell from its neighbours (gather)
-  float lin = 0.0f;
-  auto from = [&](int di, int dj, float coef_c, float r) {
-    const float mc = A.LU(di, dj) * (coef_c != 0.0f ? 1.0f : 0.0f);  // coef 0 also covers holes
-    const float a = r * coef_c * 0.5f * (A.D(di, dj) + Dc);
-    lin += tc * mc * a;
-    gd += (double)(tc * mc * r * coef_c * 0.5f * (u - A.U(di, dj)));
-  };
-  if (i + 1 < nx) from(1, 0, coef_from_code(A.code(1, 0)).W, k.rxh);
-  if (i - 1 >= 0) from(-1, 0, coef_from_code(A.code(-1, 0)).E, k.rxh);
-  if (i == 1) from(-1, 0, coef_from_code(A.code(-1, 0)).W, k.rxh);
-  if (i == nx - 2) from(1, 0, coef_from_code(A.code(1, 0)).E, k.rxh);
-  if (j + 1 < ny) from(0, 1, coef_from_code(A.code(0, 1)).S, k.ryh);
-  if (j - 1 >= 0) from(0, -1, coef_from_code(A.code(0, -1)).N, k.ryh);
-  if (j == 1) from(0, -1, coef_from_code(A.code(0, -1)).S, k.ryh);
-  if (j == ny - 2) from(0, 1, coef_from_code(A.code(0, 1)).N, k.ryh);
-  const FkEval r = fk_eval(k, u, v, w);
-  const float tdt = tc * k.dt;
-  lu = mu * (1.0f - tc * asum - tdt * r.dIdu) + lin - mv * tdt * r.dGvdu - mw * tdt * r.dGwdu;
-  lv = -mu * tdt * r.dIdv + mv * (1.0f - tdt * r.dGvdv);
-  lw = -mu * tdt * r.dIdw + mw * (1.0f - tdt * r.dGwdw);
-  lu += src;
-  fk_taus(k, r, u, v, w, mu, mv, mw, gt);
+  AdjCol o;
+  o.cw.W = (x >= 1 ? cW.E : 0.0f) + (x == 1 ? cW.W : 0.0f);
+  o.cw.E = (x + 1 < nx ? cE.W : 0.0f) + (x == nx - 2 ? cE.E : 0.0f);
+  o.cw.N = (y + 1 < ny ? cN.S : 0.0f) + (y == ny - 2 ? cN.N : 0.0f);
+  o.cw.S = (y >= 1 ? cS.N : 0.0f) + (y == 1 ? cS.S : 0.0f);
+  o.a = adj_dif(o.cw, l);
+  const AdjDif d = adj_dif(cf, l);
+  o.one = 1.0f - ((d.W + d.E) + (d.N + d.S));
+  return o;
 }
 
-// Accessor over device fields (row stride nx, cell index c).
-struct GlobalAcc {
-  const float *Uf, *Df, *LUf;
-  const uint8_t* codes;
-  int c, nx;
-  __device__ float U(int di, int dj) const { return Uf[c + di + nx * dj]; }
-  __device__ float D(int di, int dj) const { return Df[c + di + nx * dj]; }
-  __device__ float LU(int di, int dj) const { return LUf[c + di + nx * dj]; }
-  __device__ uint32_t code(int di, int dj) const {
-    return codes ? codes[c + di + nx * dj] : kCodeAllOnes;
-  }
-};
+// One reverse step of one cell: lambda of the state the forward step started
+// from (r its currents) out of lambda of the step's result, m* the cell's own
+// (0 in holes) and L* its neighbours' lambda_u.
+__device__ __forceinline__ void adj_rev_cell(const AdjK& k, const FkEval& r, const AdjCol& o,
+                                             float mu, float mv, float mw, float LW, float LE,
+                                             float LN, float LS, float src, float& lu, float& lv,
+                                             float& lw) {
+#pragma clang fp contract(off)
+  float l = LW * o.a.W;
+  l = __builtin_fmaf(LE, o.a.E, l);
+  l = __builtin_fmaf(LN, o.a.N, l);
+  l = __builtin_fmaf(LS, o.a.S, l);
+  const float tmu = k.tdt * mu, tmv = k.tdt * mv, tmw = k.tdt * mw;
+  l = __builtin_fmaf(mu, __builtin_fmaf(-k.tdt, r.Iu, o.one), l);
+  l = __builtin_fmaf(-tmv, r.Gvu, l);
+  lu = __builtin_fmaf(-tmw, r.Gwu, l) + src;
+  lv = __builtin_fmaf(-tmu, r.Iv, mv * __builtin_fmaf(-k.tdt, r.Gvv, 1.0f));
+  lw = __builtin_fmaf(-tmu, r.Iw, mw * __builtin_fmaf(-k.tdt, r.Gww, 1.0f));
+}
+
+// The cell's term of dL/dD in that step: over its links r (c mu - cw L_n)
+// (u_n - u), du* the differences.
+__device__ __forceinline__ double adj_gD(const AdjK& k, const Coef4& cf, const Coef4& cw, float mu,
+                                         float LW, float LE, float LN, float LS, float duW,
+                                         float duE, float duN, float duS) {
+#pragma clang fp contract(off)
+  const float gW = __builtin_fmaf(-LW, cw.W, mu * cf.W), gE = __builtin_fmaf(-LE, cw.E, mu * cf.E);
+  const float gN = __builtin_fmaf(-LN, cw.N, mu * cf.N), gS = __builtin_fmaf(-LS, cw.S, mu * cf.S);
+  const float x = __builtin_fmaf(gE, duE, gW * duW), y = __builtin_fmaf(gN, duN, gS * duS);
+  return (double)__builtin_fmaf(k.rxt, x, k.ryt * y);
+}
+
+// Its terms of dL/dtau (tau_d, tau_r, tau_si, tau_0, tau_v+, tau_w+) without
+// their constant factors, which adj_tau_factors() puts to the sums.
+__device__ __forceinline__ void adj_gtau(const FkEval& r, float mu, float mv, float mw,
+                                         double gt[6]) {
+#pragma clang fp contract(off)
+  gt[0] += (double)(mu * r.vpf);
+  gt[1] += (double)(mu * r.p);
+  gt[2] += (double)(mu * r.ws);
+  gt[3] += (double)(mu * r.upc);
+  gt[4] += (double)(mv * r.vp);
+  gt[5] += (double)(mw * r.pw);
+}
+// -tc dt d(1/tau) of the term each sum multiplies: J_fi and J_si enter with a
+// minus, J_so's two with a plus, and the gates close with p v/tau_v+, p w/tau_w+.
+static void adj_tau_factors(double tdt, const double tau[6], double f[6]) {
+  for (int q = 0; q < 6; ++q) f[q] = (q == 0 || q == 2 ? -tdt : tdt) / (tau[q] * tau[q]);
+}
 
 // The sums of gt over the first NT threads of a workgroup, those that hold any
 // (FP64, fixed order), added to the workgroup's slot, whose value before
@@ -511,22 +505,31 @@ __global__ __launch_bounds__(256) void k_adj_rev(const AdjK k, CFields X, CField
   double gtd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   if (i < k.nx && j < k.ny) {
     const int c = i + k.nx * j;
-    GlobalAcc A{X.f[0], D, lam_in.f[0], codes, c, k.nx};
+    const int W = mirror(i - 1, k.nx) + k.nx * j, E = mirror(i + 1, k.nx) + k.nx * j;
+    const int N = i + k.nx * mirror(j + 1, k.ny), S = i + k.nx * mirror(j - 1, k.ny);
     float src = 0.0f;
     if (src_row) {
       const int s = smap[c];
       if (s >= 0) src = src_row[s];
     }
-    float lu, lv, lw, gt[6];
-    double gd;
-    adj_rev_cell(k, A, i, j, X.f[1][c], X.f[2][c], lam_in.f[1][c], lam_in.f[2][c], src, lu, lv,
-                 lw, gd, gt);
+    const Coef4 cf = coef_of(codes, c);
+    const AdjCol o = adj_col(adj_links(k, D[c], D[W], D[E], D[N], D[S]), i, j, k.nx, k.ny, cf,
+                             coef_of(codes, W), coef_of(codes, E), coef_of(codes, N),
+                             coef_of(codes, S));
+    const float *U = X.f[0], *L = lam_in.f[0];
+    const float u = U[c], LW = L[W], LE = L[E], LN = L[N], LS = L[S];
+    const float m = cf.sc ? 1.0f : 0.0f;
+    const float mu = m * L[c], mv = m * lam_in.f[1][c], mw = m * lam_in.f[2][c];
+    const FkEval r = fk_eval(k, u, X.f[1][c], X.f[2][c]);
+    float lu, lv, lw;
+    adj_rev_cell(k, r, o, mu, mv, mw, LW, LE, LN, LS, src, lu, lv, lw);
+    const double gd = adj_gD(k, cf, o.cw, mu, LW, LE, LN, LS, U[W] - u, U[E] - u, U[N] - u,
+                             U[S] - u);
+    adj_gtau(r, mu, mv, mw, gtd);
     lam_out.f[0][c] = lu;
     lam_out.f[1][c] = lv;
     lam_out.f[2][c] = lw;
     gD[c] += gd;
-#pragma unroll
-    for (int q = 0; q < 6; ++q) gtd[q] = (double)gt[q];
   }
   double* slot = gtau_part + (size_t)(blockIdx.y * gridDim.x + blockIdx.x) * 6;
   const int tid = threadIdx.y * blockDim.x + threadIdx.x;
@@ -539,10 +542,10 @@ __global__ __launch_bounds__(256) void k_adj_rev(const AdjK k, CFields X, CField
 // double buffer.  A thread keeps its lambda_v, lambda_w, its row and column of
 // the transposed operator (constant through the steps), and, in the tile, its
 // dL/dD and dL/dtau sums (FP64).  u, v, w and the sensor source of a step are
-// loaded two steps ahead.  A step is bound by VALU issue: about 165
-// instructions a ring cell and 290 a tile cell, and 8 steps of a 16 x 16 tile
-// are 21 wave-steps on the busiest SIMD: 8 us of a 14.6 us launch at 256 x 256
-// (25.4 us with per-step index arithmetic; the forward 12.8 -> 9.2 us).
+// loaded two steps ahead.  A step is bound by VALU issue (see fk_eval): 8 steps
+// of a 16 x 16 tile are 21 wave-steps on the busiest SIMD.  Launches of 8 steps
+// at 256 x 256: 25.4 us with per-step index arithmetic, 15.5 with a thread a
+// cell, 13.0 with fewer instructions a step; the forward's 12.8, 10.1, 8.6.
 template <bool MASKED>
 __global__ __launch_bounds__(kAdjThreads) void k_adj_rev_tiled(
     const AdjK k, const float* __restrict__ seg, const float* __restrict__ x0, size_t n,
@@ -554,14 +557,12 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_rev_tiled(
   __shared__ float s_U[2][kAdjLds], s_L[2][kAdjLds], s_D[kAdjLds];
   __shared__ uint8_t s_c[MASKED ? kAdjLds : 1];
   const int nx = k.nx, ny = k.ny;
-  const int ty = blockIdx.x / t.tiles_x, tx = blockIdx.x - ty * t.tiles_x;
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int ty = tile / t.tiles_x, tx = tile - ty * t.tiles_x;
   const int ox0 = tx * t.tw, oy0 = ty * t.th;
   const AdjCell q = adj_cell(threadIdx.x, ox0, oy0, t, K, nx, ny);
   const AdjAt at = adj_at(q, ox0, oy0, K, nx, ny);
   const size_t c = (size_t)q.x + (size_t)nx * q.y;
-  // tiles that hold cells next to an edge cell have mirror terms
-  const bool edges = ox0 - K <= 1 || oy0 - K <= 1 || ox0 + t.tw + K >= nx - 1 ||
-                     oy0 + t.th + K >= ny - 1;
   const int sensor = src && q.m < K ? smap[c] : -1;
   struct Ahead {
     float u = 0.0f, v = 0.0f, w = 0.0f, src = 0.0f;
@@ -597,45 +598,21 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_rev_tiled(
     }
   }
   __syncthreads();
-  // own row: 1 - tc * sum of the weights.  Column: the weights with which the
-  // neighbours' updates read this cell, a = r c (D_c + D_n)/2, from the east,
-  // west, north, south neighbour, and x.. a second time from an edge cell,
-  // whose mirror neighbour this cell is.  h = c/2 for the dL/dD terms.
-  const float tc = k.tc;
-  float one = 0.0f, aE = 0.0f, aW = 0.0f, aN = 0.0f, aS = 0.0f, xE = 0.0f, xW = 0.0f, xN = 0.0f,
-        xS = 0.0f;
-  float hE = 0.0f, hW = 0.0f, hN = 0.0f, hS = 0.0f, yE = 0.0f, yW = 0.0f, yN = 0.0f, yS = 0.0f;
+  AdjCol o{};
   const float m = !MASKED || cf.sc ? 1.0f : 0.0f;
   if (q.m < K) {
-    const float DW = s_D[at.W], DE = s_D[at.E], DN = s_D[at.N], DS = s_D[at.S];
-    float asum = 0.0f;
-    asum += k.rxh * cf.W * 0.5f * (Dc + DW);
-    asum += k.rxh * cf.E * 0.5f * (Dc + DE);
-    asum += k.ryh * cf.N * 0.5f * (Dc + DN);
-    asum += k.ryh * cf.S * 0.5f * (Dc + DS);
-    one = 1.0f - tc * asum;
-    Coef4 cE{1.f, 1.f, 1.f, 1.f, true}, cW = cE, cN = cE, cS = cE;
+    Coef4 cW{1.f, 1.f, 1.f, 1.f, true}, cE = cW, cN = cW, cS = cW;
     if (MASKED) {
-      cE = coef_from_code(s_c[at.E]);
       cW = coef_from_code(s_c[at.W]);
+      cE = coef_from_code(s_c[at.E]);
       cN = coef_from_code(s_c[at.N]);
       cS = coef_from_code(s_c[at.S]);
     }
-    auto weight = [&](bool there, float coef, float r, float Dn, float& a, float& h) {
-      a = there ? r * coef * 0.5f * (Dn + Dc) : 0.0f;
-      h = there ? coef * 0.5f : 0.0f;
-    };
-    weight(q.x + 1 < nx, cE.W, k.rxh, DE, aE, hE);
-    weight(q.x - 1 >= 0, cW.E, k.rxh, DW, aW, hW);
-    weight(q.y + 1 < ny, cN.S, k.ryh, DN, aN, hN);
-    weight(q.y - 1 >= 0, cS.N, k.ryh, DS, aS, hS);
-    weight(q.x == 1, cW.W, k.rxh, DW, xW, yW);
-    weight(q.x == nx - 2, cE.E, k.rxh, DE, xE, yE);
-    weight(q.y == 1, cS.S, k.ryh, DS, xS, yS);
-    weight(q.y == ny - 2, cN.N, k.ryh, DN, xN, yN);
+    o = adj_col(adj_links(k, Dc, s_D[at.W], s_D[at.E], s_D[at.N], s_D[at.S]), q.x, q.y, nx, ny,
+                cf, cW, cE, cN, cS);
   }
   // what the sums are added to at the end, read now
-  double* gt_slot = gtau_part + (size_t)blockIdx.x * 6;
+  double* gt_slot = gtau_part + (size_t)tile * 6;
   const double gD_was = q.m == 0 ? gD[c] : 0.0;
   const double gt_was = threadIdx.x < 6 ? gt_slot[threadIdx.x] : 0.0;
   double gd = 0.0, gtd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
@@ -645,50 +622,15 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_rev_tiled(
     if (q.m < K - s) {
       const float* L = s_L[b];
       const float LE = L[at.E], LW = L[at.W], LN = L[at.N], LS = L[at.S];
-      const float u = cur.u, v = cur.v, w = cur.w;
       const float mu = m * Lu, mv = m * Lv, mw = m * Lw;
-      const float tE = tc * LE, tW = tc * LW, tN = tc * LN, tS = tc * LS;
-      float lin = tE * aE;
-      lin += tW * aW;
-      if (edges) {
-        lin += tW * xW;
-        lin += tE * xE;
-      }
-      lin += tN * aN;
-      lin += tS * aS;
-      if (edges) {
-        lin += tS * xS;
-        lin += tN * xN;
-      }
-      const FkEval r = fk_eval(k, u, v, w);
-      const float tdt = tc * k.dt;
+      const FkEval r = fk_eval(k, cur.u, cur.v, cur.w);
+      adj_rev_cell(k, r, o, mu, mv, mw, LW, LE, LN, LS, cur.src, Lu, Lv, Lw);
       if (q.m == 0) {  // dL/dD and dL/dtau of the tile's cells
         const float* U = s_U[b];
-        const float dE = U[at.E] - u, dW = U[at.W] - u, dN = U[at.N] - u, dS = U[at.S] - u;
-        const float tm = tc * mu, tx = tm * k.rxh, ty = tm * k.ryh;
-        gd += (double)(tx * (cf.W * 0.5f) * dW);
-        gd += (double)(tx * (cf.E * 0.5f) * dE);
-        gd += (double)(ty * (cf.N * 0.5f) * dN);
-        gd += (double)(ty * (cf.S * 0.5f) * dS);
-        gd -= (double)(tE * k.rxh * hE * dE);
-        gd -= (double)(tW * k.rxh * hW * dW);
-        gd -= (double)(tN * k.ryh * hN * dN);
-        gd -= (double)(tS * k.ryh * hS * dS);
-        if (edges) {
-          gd -= (double)(tW * k.rxh * yW * dW);
-          gd -= (double)(tE * k.rxh * yE * dE);
-          gd -= (double)(tS * k.ryh * yS * dS);
-          gd -= (double)(tN * k.ryh * yN * dN);
-        }
-        float gt[6];
-        fk_taus(k, r, u, v, w, mu, mv, mw, gt);
-#pragma unroll
-        for (int e = 0; e < 6; ++e) gtd[e] += (double)gt[e];
+        gd += adj_gD(k, cf, o.cw, mu, LW, LE, LN, LS, U[at.W] - cur.u, U[at.E] - cur.u,
+                     U[at.N] - cur.u, U[at.S] - cur.u);
+        adj_gtau(r, mu, mv, mw, gtd);
       }
-      Lu = mu * (one - tdt * r.dIdu) + lin - mv * tdt * r.dGvdu - mw * tdt * r.dGwdu;
-      Lv = -mu * tdt * r.dIdv + mv * (1.0f - tdt * r.dGvdv);
-      Lw = -mu * tdt * r.dIdw + mw * (1.0f - tdt * r.dGwdw);
-      Lu += cur.src;
       s_L[b ^ 1][at.l] = Lu;
     }
     if (q.m <= 1) s_U[b ^ 1][at.l] = next.u;
@@ -697,9 +639,9 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_rev_tiled(
     __syncthreads();
   }
   if (q.m == 0) {
-    lam_out.f[0][c] = Lu;
-    lam_out.f[1][c] = Lv;
-    lam_out.f[2][c] = Lw;
+    store_through(lam_out.f[0], (uint32_t)c, Lu);
+    store_through(lam_out.f[1], (uint32_t)c, Lv);
+    store_through(lam_out.f[2], (uint32_t)c, Lw);
     gD[c] = gD_was + gd;
   }
   adj_gtau_block<kAdjTile * kAdjTile>(gtd, gt_was, gt_slot);
@@ -791,6 +733,7 @@ struct yh_adjoint {
   bool have_targets = false, forward_done = false;
   const float* D = nullptr;
   yh::AdjK k{};
+  double tau_f[6] = {};  // adj_tau_factors() of the forward's time constants
   int fwdK = 8;  // steps per launch, forward and reverse: 1 = one-step kernels, else LDS-tiled
   int nparts = 0;  // dL/dtau workgroup slots: the larger of the two reverse grids
   yh::AdjTile tile{};  // output tile of the tiled kernels
@@ -822,34 +765,30 @@ static void adj_k(yh_adjoint* a, const double tau6[6]) {
   const yh_params& p = a->p;
   k.nx = p.nx;
   k.ny = p.ny;
-  k.rxh = (float)(a->d.dt / (a->d.hx * a->d.hx));
-  k.ryh = (float)(a->d.dt / (a->d.hy * a->d.hy));
-  k.dt = (float)a->d.dt;
-  k.tc = (float)p.tc;
-  k.hw = (float)p.heaviside_width;
+  const double tdt = p.tc * a->d.dt, ln2 = std::log(2.0);
+  k.rxt = (float)(0.5 * tdt / (a->d.hx * a->d.hx));
+  k.ryt = (float)(0.5 * tdt / (a->d.hy * a->d.hy));
+  k.tdt = (float)tdt;
   const yh_fk_params& f = p.fk;
-  k.td = (float)tau6[0];
-  k.tr = (float)tau6[1];
-  k.tsi = (float)tau6[2];
-  k.t0 = (float)tau6[3];
-  k.tvp = (float)tau6[4];
-  k.twp = (float)tau6[5];
-  k.tv1m = (float)f.tau_v1m;
-  k.tv2m = (float)f.tau_v2m;
-  k.twm = (float)f.tau_wm;
   k.uc = (float)f.u_c;
   k.uv = (float)f.u_v;
   k.ucsi = (float)f.u_csi;
-  k.kk = (float)f.k;
-  k.ihw = (float)(1.0 / p.heaviside_width);
+  k.uc1 = (float)(1.0 + f.u_c);
+  k.tv1m = (float)f.tau_v1m;
+  k.tv2m = (float)f.tau_v2m;
+  k.dtv = (float)(f.tau_v2m - f.tau_v1m);
+  k.eh = (float)(2.0 / (p.heaviside_width * ln2));
+  k.es = (float)(2.0 * f.k / ln2);
   k.tihw = (float)(2.0 / p.heaviside_width);
   k.itd = (float)(1.0 / tau6[0]);
   k.itr = (float)(1.0 / tau6[1]);
-  k.ihtsi = (float)(0.5 / tau6[2]);
+  k.itsi = (float)(1.0 / tau6[2]);
+  k.ksi = (float)(2.0 * f.k / tau6[2]);
   k.it0 = (float)(1.0 / tau6[3]);
   k.itvp = (float)(1.0 / tau6[4]);
   k.itwp = (float)(1.0 / tau6[5]);
   k.itwm = (float)(1.0 / f.tau_wm);
+  adj_tau_factors(tdt, tau6, a->tau_f);
 }
 
 // Most device memory a problem takes to keep every state of its forward sweep.
@@ -1122,6 +1061,7 @@ int yh_adjoint_backward(yh_adjoint* a, void* stream, double* d_gD, double gtau[6
   for (int q = 0; q < 6; ++q) gtau[q] = 0.0;
   for (int b = 0; b < a->nparts; ++b)
     for (int q = 0; q < 6; ++q) gtau[q] += part[(size_t)b * 6 + q];
+  for (int q = 0; q < 6; ++q) gtau[q] *= a->tau_f[q];
   return YH_OK;
 }
 
