@@ -16,8 +16,9 @@
 // coefficient of every (cell c, direction) whose neighbour is j, including the
 // two mirror images at each edge.  The forward keeps every state where they
 // fit in 4 GiB; a longer run keeps a checkpoint every `ckpt` steps, and each
-// segment is recomputed into a buffer before its reverse sweep.  gD and gtau accumulate in FP64 (gtau per workgroup, in a fixed
-// order, so results are deterministic).
+// segment is recomputed into a buffer before its reverse sweep.  gD and gtau
+// accumulate in FP64 (gtau per workgroup, in a fixed order, so results are
+// deterministic).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -282,7 +283,8 @@ __device__ __forceinline__ AdjAt adj_at(const AdjCell& c, int ox0, int oy0, int 
 // K forward steps, their states written through to memory (left dirty in the
 // XCD's L2 they delay the end of the launch: 10.1 against 9.4 us for 8 steps of
 // 256 x 256).  Outputs: with seg, the state after every step into seg
-// slots slot0+1 .. slot0+K; otherwise the final state into out.  Sensor traces for every step with step % rec == 0.
+// slots slot0+1 .. slot0+K; otherwise the final state into out.  Sensor traces
+// for every step with step % rec == 0.
 template <bool MASKED>
 __global__ __launch_bounds__(kAdjThreads) void k_adj_fwd_tiled(
     const AdjK k, CFields in, Fields out, const float* __restrict__ D,
@@ -536,8 +538,8 @@ __global__ __launch_bounds__(256) void k_adj_rev(const AdjK k, CFields X, CField
   adj_gtau_block<256>(gtd, tid < 6 ? slot[tid] : 0.0, slot);
 }
 
-// K reverse steps, n_top, n_top-1, ..., of one tile (see the tiles section; lambda has
-// the forward's one-cell dependence).  u of each step's state goes through LDS
+// K reverse steps, n_top, n_top-1, ..., of one tile (see the tiles section;
+// lambda has the forward's one-cell dependence).  u of each step's state goes through LDS
 // (the neighbours of the tile's cells read it for dL/dD), lambda_u through a
 // double buffer.  A thread keeps its lambda_v, lambda_w, its row and column of
 // the transposed operator (constant through the steps), and, in the tile, its

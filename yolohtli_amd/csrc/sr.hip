@@ -356,8 +356,9 @@ __global__ __launch_bounds__(kSliceBX* kSliceBY) void k_sr_slices(
 
 // ----------------------------------------------------------------- solve
 // Column q of the partials (stored column-major, [12][nparts]) summed by one
-// wave in a fixed order (lane-strided, then the pairs of a shuffle tree), so the integrals do not depend on
-// scheduling and every wave that sums a column gets the same bits.  The total is in lane 0.
+// wave in a fixed order (lane-strided, then the pairs of a shuffle tree), so
+// the integrals do not depend on scheduling and every wave that sums a column
+// gets the same bits.  The total is in lane 0.
 __device__ __forceinline__ double sr_column_sum(const double* partials, int nparts, int q) {
   const int lane = __lane_id();
   double s = 0.0;

@@ -10,7 +10,8 @@
 //   k_direct       one step, one thread per cell, reads the raw mask; writes
 //                  velTan when asked (the reactionDiffusion_wrapper surface)
 //   k_direct_codes one step from stencil codes (the k=1 plan path)
-//   k_tiled        K fused steps per launch (temporal blocking): a workgroup
+//   k_tiled        (tiled.h, built per model by tiled_2v.hip and tiled_fk.hip)
+//                  K fused steps per launch (temporal blocking): a workgroup
 //                  owns a 64 x (NW*R) region, each lane one column, each wave
 //                  R consecutive rows kept in registers.  West/east neighbours
 //                  come from ds_bpermute (no LDS memory), north/south from the
