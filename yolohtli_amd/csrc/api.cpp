@@ -299,7 +299,7 @@ int yh_rd_step_dev_ex(const yh_params* p, float* const out[3], const float* cons
   int dev = 0, cus = 0;
   YH_HIP(hipGetDevice(&dev));
   YH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  YH_HIP(launch_general(p->model, g, 1, general_shape(p->model, g, 1, 1, cus), ci, co, cv, nullptr,
+  YH_HIP(launch_general(p->model, g, 1, general_table(p->model, g, 1, 1, cus).next(1), ci, co, cv, nullptr,
                         p->solidSwitch ? solid : nullptr, (hipStream_t)stream, nullptr));
   return YH_OK;
 }

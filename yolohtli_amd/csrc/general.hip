@@ -155,7 +155,8 @@ constexpr int kGenPer = 3;                     // rows of a wave, at most
 constexpr int kGenRows = kGenWaves * kGenPer;  // rows of a region, at most
 constexpr int kGenPad = 2;                     // pad cells around the region in LDS
 constexpr int kGenStride = 64 + 2 * kGenPad;
-constexpr int kGenHalo = 8;
+constexpr int kGenHalo = 12;
+static_assert(kGenHalo <= kGenDeepest, "a step takes a ring cell and more");
 
 struct GenRun {
   int K, order, rad, rows, halo, out_w, out_h, tiles_x, ntiles;
@@ -506,39 +507,81 @@ static int general_reach(const GParams& g) {
   return g.neumann && !g.masked && g.aniso ? 2 : 1;
 }
 
-static int general_depth(const GParams& g, int order) {
-  return std::max(1, kGenHalo / (order * general_reach(g)));
+static int general_depth(const GParams& g, int order, int halo) {
+  return std::max(1, halo / (order * general_reach(g)));
 }
 
-// Steps to fuse (at most `steps`) and rows of a region on a device of `cus`
-// compute units: the pair with the least estimated time per step.  A launch
-// takes about 4 us before and after its stages and runs as many rounds as its
+// Steps to fuse and rows of a region on a device of `cus` compute units.  A
+// launch takes about 4 us besides its stages and runs as many rounds as its
 // workgroups (16 waves, one a CU) fill; a row and stage costs c us on a CU.
 // More steps a launch pay its fixed part less often and recompute a wider
 // ring: RK4 with lap4 takes two steps a launch at 512 x 512 (17.3 against 2 x
 // 10.1 us, one round either way) and one at 1024 x 1024 (22.2 us, two rounds,
-// against 48.4, three).
-GenShape general_shape(int model, const GParams& g, int order, int steps, int cus) {
-  double c = model == M2V ? 0.025 : 0.05;
-  if (g.neumann && !g.masked) c += (g.lap4 ? 0.025 : 0.0) + (g.aniso ? 0.02 : 0.0);
+// against 48.4, three).  The first choice is the pair with the least time per
+// step, of up to 8 ring cells.  Where that fills one round, as up to about
+// 512 x 512, 12 ring cells may pay too, and a call takes the depth whose full
+// launches and remainder take the least time together, for an estimated gain of
+// 4%, the estimate's spread (128 x 128, 5 steps of masked RK2: 11.7 us in
+// launches of four and one, 9.2 in one; 40 RK4 steps 150.5 -> 138.9; 17
+// Dirichlet steps at 512 x 512 31.3 -> 28.4).  With several rounds, which
+// overlap in ways the estimate does not know, the same rule lost up to 9% as
+// often as it gained.
+GenTable general_table(int model, const GParams& g, int order, int steps, int cus) {
   const int rad = general_reach(g);
+  const double fit = g.neumann && !g.masked ? (g.lap4 ? 0.025 : 0.0) + (g.aniso ? 0.04 : 0.0) : 0.0;
+  auto rounds = [&](int K, int rows) {  // 0: no such region
+    const int halo = K * order * rad, w = 64 - 2 * halo, h = rows - 2 * halo;
+    if (h < 1) return 0;
+    const int64_t tiles = (int64_t)((g.nx + w - 1) / w) * ((g.ny + h - 1) / h), n = std::max(1, cus);
+    return (int)((tiles + n - 1) / n);
+  };
+  GenTable t;
+  t.limit = std::min(steps, kGenDeepest);
   GenShape best{1, kGenRows};
   double least = 1e300;
-  for (int K = 1; K <= std::min(steps, general_depth(g, order)); ++K) {
-    const int stages = K * order, halo = stages * rad, out_w = 64 - 2 * halo;
-    for (int rows = 8; rows <= kGenRows; rows += 4) {
-      const int out_h = rows - 2 * halo;
-      if (out_h < 1) continue;
-      const double tiles = (double)((g.nx + out_w - 1) / out_w) * ((g.ny + out_h - 1) / out_h);
-      double t = 0.5;
-      for (int s = 1; s <= stages; ++s) t += std::max(0.2, c * (rows - 2 * rad * s));
-      t = (4.0 + t * std::ceil(tiles / std::max(1, cus))) / K;
-      if (t < least) {
-        least = t;
+  const double c = (model == M2V ? 0.025 : 0.05) + fit;
+  for (int K = 1; K <= t.limit; ++K) {
+    for (int rows = 8; rows <= kGenRows && K <= general_depth(g, order, 8); rows += 4) {
+      const int n = rounds(K, rows);
+      if (n == 0) continue;
+      double us = 0.5;
+      for (int s = 1; s <= K * order; ++s) us += std::max(0.2, c * (rows - 2 * rad * s));
+      us = (4.0 + n * us) / K;
+      if (us < least) {
+        least = us;
         best = GenShape{K, rows};
       }
     }
+    t.first[K] = best;
+    t.round[K] = rounds(best.K, best.rows) == 1;
   }
+  // one round: a stage is the chain of the wave with the most rows
+  const double row = (model == M2V ? 0.33 : 0.75) + 16.0 * fit;
+  for (int K = 1; K <= std::min(t.limit, general_depth(g, order, kGenHalo)); ++K) {
+    int rows = 8;  // the fewest that do
+    while (rows <= kGenRows && rounds(K, rows) != 1) rows += 4;
+    if (rows > kGenRows) break;
+    t.us[K] = 4.0;
+    for (int s = 1; s <= K * order; ++s)
+      t.us[K] += row * ((std::max(1, rows - 2 * rad * s) + kGenWaves - 1) / kGenWaves);
+    t.rows[K] = rows;
+    t.deepest = K;
+  }
+  return t;
+}
+
+// The next launch of a call with `steps` steps to go.
+GenShape GenTable::next(int steps) const {
+  const int n = std::min(steps, limit);
+  if (!round[n] || first[n].K > deepest) return first[n];
+  auto call = [&](int K) { return (steps / K) * us[K] + us[steps % K]; };
+  GenShape best = first[n];
+  double least = 0.96 * call(best.K);
+  for (int K = 1; K <= std::min(n, deepest); ++K)
+    if (call(K) < least) {
+      least = call(K);
+      best = GenShape{K, rows[K]};
+    }
   return best;
 }
 
@@ -547,7 +590,7 @@ hipError_t launch_general(int model, const GParams& g, int order, GenShape shape
                           const ApdState* apd) {
   if (order != 1 && order != 2 && order != 4) return hipErrorInvalidValue;
   const int K = shape.K;
-  if (K < 1 || K > general_depth(g, order) || shape.rows > kGenRows) return hipErrorInvalidValue;
+  if (K < 1 || K > general_depth(g, order, kGenHalo) || shape.rows > kGenRows) return hipErrorInvalidValue;
   // :70-95, RK4 weights as the reference writes them
   GenRun r = {};
   r.K = K;

@@ -235,8 +235,10 @@ int plan_advance(yh_plan* pl, int nsteps, hipStream_t s) {
     const int order = pl->p.timeIntOrder;
     const GParams g = make_gparams(pl->p, pl->stim_on, pl->stim_x, pl->stim_y);
     if (!pl->prev_u) YH_HIP(hipMalloc(&pl->prev_u, pl->n * sizeof(float)));
+    if (!pl->general.limit)
+      pl->general = general_table(pl->p.model, g, order, kGenDeepest, pl->cus);
     while (remaining > 0) {
-      const GenShape shape = general_shape(pl->p.model, g, order, remaining, pl->cus);
+      const GenShape shape = pl->general.next(remaining);
       const int K = shape.K;
       CFields ci;
       Fields co;

@@ -83,6 +83,7 @@ struct yh_plan {
   int tipcap = 0;
   int* flag_d = nullptr;
   yh_kernel_cfg cfg{YH_KERNEL_AUTO, 4, 8, 8, 1};
+  yh::GenTable general;    // launches of the general path
   yh::AutoTable table[2];  // without and with the APD update
   int64_t count = 0;
   bool keep_prev = true;

@@ -351,7 +351,18 @@ inline bool standard_branch(const yh_params& p) {
 struct GenShape {
   int K, rows;
 };
-GenShape general_shape(int model, const GParams& g, int order, int steps, int cus);
+constexpr int kGenDeepest = 12;  // steps of a launch, at most
+// The launches that calls of up to `steps` steps choose from (general.hip).
+struct GenTable {
+  int limit = 0;               // `steps`; 0: not made yet
+  GenShape first[kGenDeepest + 1] = {};  // of a call of n steps, or of the last n and more
+  bool round[kGenDeepest + 1] = {};      // first[n] fills no more than one round
+  int deepest = 0;             // one-round launches: rows and time of each depth
+  int rows[kGenDeepest + 1] = {};
+  double us[kGenDeepest + 1] = {};
+  GenShape next(int steps) const;
+};
+GenTable general_table(int model, const GParams& g, int order, int steps, int cus);
 // shape.K steps of the general path in one launch, from `in` to `out` (never
 // the same).  prev (may be null) receives u one step before the end, vt
 // (entries may be null) the last step's velocity; solid is null without a mask.
