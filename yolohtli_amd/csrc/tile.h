@@ -48,11 +48,13 @@ struct TileLds {
 // With APD, every substep also updates the action-potential-duration state of
 // the cells this tile outputs (their value is exact at every substep), so
 // the measurement costs no extra launch.  A cell crosses the threshold twice
-// a beat of thousands of steps: a substep only tests for it, the division and
-// the updates run in the waves where a lane crosses, durations go straight to
+// a beat of thousands of steps: a substep only compares u with it, once a cell,
+// and where a lane changed sides (a scalar test of the two ballots) takes the
+// exact test, the division and the update; durations go straight to
 // memory, and only cells that crossed are written back (a launch of 16 masked
 // FK steps at 512 x 512: 29.4 us with the update, two divisions, on every cell
-// and all five fields loaded and stored, 20.9 us now, 17.3 without APD).  With PREV, u of
+// and all five fields loaded and stored, 20.9 with the exact test, four
+// comparisons, everywhere, 20.3 now, 17.3 without APD).  With PREV, u of
 // the output cells one substep before the end is written to prev_u (0 in
 // holes): the previous state the tip test needs, without a single-step tail.
 // K >= 1 (the launchers reject K < 1).
@@ -154,6 +156,7 @@ __device__ __forceinline__ void tile_advance(const KParams& k, CFields in, Field
   uint32_t a_first[CW];  // bit r: cell (r, c) has had its first duration
   uint32_t crossed[CW];  // bit r: its APD state has changed
   float a_th[CW];        // no value crosses the threshold of a lane without output cells
+  uint64_t above[APD ? R : 1][CW];  // lanes whose u is over it, per row
   if (APD) {
 #pragma unroll
     for (int c = 0; c < CW; ++c) {
@@ -166,6 +169,7 @@ __device__ __forceinline__ void tile_advance(const KParams& k, CFields in, Field
 #pragma unroll
       for (int c = 0; c < CW; ++c) {
         a_front[APD ? r : 0][c] = a_back[APD ? r : 0][c] = 0.0f;
+        above[APD ? r : 0][c] = __builtin_amdgcn_ballot_w64(X[0][r][c] > a_th[c]);
         if (!(out_x[c] && lr >= K && lr < H - K && gy < ny)) continue;
         const uint32_t idx = (uint32_t)gy * (uint32_t)nx + (uint32_t)(gx0 + c);
         a_front[APD ? r : 0][c] = *at32(apd.front, idx);
@@ -277,18 +281,24 @@ __device__ __forceinline__ void tile_advance(const KParams& k, CFields in, Field
           } else {
             M::step(k, dif[0][c], dif[ND - 1][c], X[0][r][c], X[1][r][c]);
           }
-          if (APD && lr >= K && lr < H - K && gy0 + r < ny &&
-              apd_crosses(u_old, X[0][r][c], a_th[c]) && !(MASKED && ((hole[c] >> r) & 1u))) {
-            // a completed duration goes straight to memory
-            float d;
-            const bool done = apd_crossing(u_old, X[0][r][c], apd.count0 + s + 1, apd.dt, apd.th,
-                                           a_front[APD ? r : 0][c], a_back[APD ? r : 0][c], d);
-            crossed[c] |= 1u << r;
-            if (done) {
-              const uint32_t idx =
-                  (uint32_t)(gy0 + r) * (uint32_t)nx + (uint32_t)(gx0 + c);
-              *at32((a_first[c] >> r) & 1u ? apd.apd2 : apd.apd1, idx) = d;
-              a_first[c] ^= 1u << r;
+          if (APD && lr >= K && lr < H - K && gy0 + r < ny) {
+            // one comparison a cell; the exact test where a lane changed sides
+            const uint64_t now = __builtin_amdgcn_ballot_w64(X[0][r][c] > a_th[c]);
+            const uint64_t turned = now ^ above[APD ? r : 0][c];
+            above[APD ? r : 0][c] = now;
+            if (turned != 0 && apd_crosses(u_old, X[0][r][c], a_th[c]) &&
+                !(MASKED && ((hole[c] >> r) & 1u))) {
+              // a completed duration goes straight to memory
+              float d;
+              const bool done = apd_crossing(u_old, X[0][r][c], apd.count0 + s + 1, apd.dt, apd.th,
+                                             a_front[APD ? r : 0][c], a_back[APD ? r : 0][c], d);
+              crossed[c] |= 1u << r;
+              if (done) {
+                const uint32_t idx =
+                    (uint32_t)(gy0 + r) * (uint32_t)nx + (uint32_t)(gx0 + c);
+                *at32((a_first[c] >> r) & 1u ? apd.apd2 : apd.apd1, idx) = d;
+                a_first[c] ^= 1u << r;
+              }
             }
           }
           if (s == K - 1) {
