@@ -1,0 +1,65 @@
+"""A batch that nobody tuned, stepped by calls of two sizes in turn that take
+different shapes at the same depth: each shape keeps its own work list.
+
+The results equal single-step launches bit for bit.  Once both sizes were seen
+a call allocates and rebuilds nothing, so calls in turn take the time of the
+same calls in a row (a rebuilt list costs a synchronisation, two allocations and
+two uploads, more than a call of this batch; 1.5 leaves room for noise).
+"""
+import time
+
+import numpy as np
+import pytest
+
+from yolohtli_amd import abi_types as T
+from yolohtli_amd.batch import Batch, batched_workload
+
+pytestmark = pytest.mark.gpu
+
+PAIRS = ((4, 16), (4, 22), (4, 28), (5, 11), (5, 17), (5, 23), (6, 18), (6, 13))
+
+
+def _batch(model):
+    params, masks, fields = batched_workload(ntissues=12, config=90, model=model,
+                                             sides=(128, 256), max_holes=1)
+    b = Batch(params)
+    for t, (m, f) in enumerate(zip(masks, fields)):
+        b.set_mask(t, m)
+        b.set_state(t, *f)
+    return b
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("model", [T.YH_MODEL_2V_REF, T.YH_MODEL_3V_FK])
+def test_calls_of_two_sizes_in_turn(torch_cuda, model, graph):
+    torch = torch_cuda
+    b, ref = _batch(model), _batch(model)
+    b.set_graph(graph)
+    ref.set_kernel(substeps=1, rows=8, waves=8, cols=1, persistent=0)
+    for pair in PAIRS:
+        for n in pair + pair:
+            b.step(n)
+    ref.step(2 * sum(map(sum, PAIRS)))
+    for t in range(12):
+        for x, y in zip(b.get_state(t), ref.get_state(t)):
+            np.testing.assert_array_equal(x, y)
+    ref.close()
+
+    def timed(order):
+        best = float("inf")
+        for _ in range(6):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            for n in order:
+                b.step(n)
+            torch.cuda.synchronize()
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    slow = {}
+    for p, q in PAIRS:
+        turn, row = timed((p, q) * 8), timed((p,) * 8) + timed((q,) * 8)
+        if turn > 1.5 * row:
+            slow[p, q] = (turn, row)
+    b.close()
+    assert not slow

@@ -171,14 +171,16 @@ struct yh_batch {
   double cfg_us[8];  // the same estimate of cfg's launches of 0 .. 6 steps
   bool use_graph = true;
   int64_t count = 0;
-  // per-K work lists: K -> (tissue table, items, nitems)
+  // work lists: (K, rows, waves, cols) -> (tissue table, items, nitems).  Calls
+  // of different sizes take different shapes at the same depth, so each pair
+  // has its own list, and a list in use (by captured graphs, too) is never
+  // replaced.
   struct WL {
     yh::BatchTissue* tissues = nullptr;
     int2* items = nullptr;
     int nitems = 0;
-    yh_kernel_cfg cfg{};
   };
-  std::map<int, WL> wl;
+  std::map<std::tuple<int, int, int, int>, WL> wl;
   // graph cache: (nsteps, cur, K, rows, waves, cols, persistent) -> exec
   std::map<std::tuple<int, int, int, int, int, int, int>, hipGraphExec_t> graphs;
   std::vector<hipGraph_t> graph_objs;
@@ -204,18 +206,11 @@ static void batch_clear_graphs(yh_batch* b) {
 
 static int batch_worklist(yh_batch* b, const yh_kernel_cfg& c, yh_batch::WL** out) {
   const int K = c.substeps;
-  auto it = b->wl.find(K);
-  if (it != b->wl.end() && it->second.cfg.rows == c.rows && it->second.cfg.waves == c.waves &&
-      it->second.cfg.cols == c.cols) {
+  const auto key = std::make_tuple(K, c.rows, c.waves, c.cols);
+  auto it = b->wl.find(key);
+  if (it != b->wl.end()) {
     *out = &it->second;
     return YH_OK;
-  }
-  if (it != b->wl.end()) {
-    batch_clear_graphs(b);  // captured launches point at the list being replaced
-    (void)hipDeviceSynchronize();
-    (void)hipFree(it->second.tissues);
-    (void)hipFree(it->second.items);
-    b->wl.erase(it);
   }
   const int wout = 64 * c.cols - 2 * K, hout = c.rows * c.waves - 2 * K;
   if (wout <= 0 || hout <= 0) return YH_EINVAL;
@@ -230,7 +225,6 @@ static int batch_worklist(yh_batch* b, const yh_kernel_cfg& c, yh_batch::WL** ou
     for (int q = 0; q < tab[t].tiles_x * tiles_y; ++q) items.push_back(make_int2(t, q));
   }
   yh_batch::WL w;
-  w.cfg = c;
   w.nitems = (int)items.size();
   hipError_t e = hipMalloc(&w.tissues, sizeof(BatchTissue) * b->nt);
   if (e == hipSuccess) e = hipMalloc(&w.items, sizeof(int2) * items.size());
@@ -243,8 +237,7 @@ static int batch_worklist(yh_batch* b, const yh_kernel_cfg& c, yh_batch::WL** ou
     if (w.items) (void)hipFree(w.items);
     return hip_fail(e, "batch work list");
   }
-  b->wl[K] = w;
-  *out = &b->wl[K];
+  *out = &b->wl.emplace(key, w).first->second;
   return YH_OK;
 }
 
@@ -631,7 +624,11 @@ int yh_batch_autotune(yh_batch* b, int steps, void* stream, yh_kernel_cfg* best,
   for (int a = 0; a < b->nv; ++a)
     (void)hipMemcpyAsync(b->buf[b->cur][a], save[a], sizeof(float) * b->total,
                          hipMemcpyDeviceToDevice, s);
-  (void)hipStreamSynchronize(s);
+  // the candidates' lists go, and with them the graphs that point at lists,
+  // once no stream runs one any more
+  (void)hipDeviceSynchronize();
+  batch_clear_graphs(b);
+  batch_clear_wl(b);
   for (int a = 0; a < b->nv; ++a) (void)hipFree(save[a]);
   b->use_graph = graph0;
   b->count = count0;
