@@ -63,3 +63,37 @@ def test_calls_of_two_sizes_in_turn(torch_cuda, model, graph):
             slow[p, q] = (turn, row)
     b.close()
     assert not slow
+
+
+@pytest.mark.parametrize("model,ntissues,sides", [(0, 16, (128, 256, 384, 512, 768)),
+                                                  (1, 24, (300, 500)), (0, 8, (768,)),
+                                                  (1, 3, (128, 256))])
+def test_untuned_batch_is_not_slower_than_one_shape(torch_cuda, model, ntissues, sides):
+    """Calls before a kernel is chosen against launches of the default shape
+    and depth only (K=6, 8 x 8): the estimate's choice may not cost time (5% are
+    for the clock)."""
+    torch = torch_cuda
+    params, masks, fields = batched_workload(ntissues=ntissues, model=model, sides=sides,
+                                             max_holes=10)
+    batches = []
+    for fixed in (False, True):
+        b = Batch(params)
+        for t, (m, f) in enumerate(zip(masks, fields)):
+            b.set_mask(t, m)
+            b.set_state(t, *f)
+        if fixed:
+            b.set_kernel(substeps=6, rows=8, waves=8, cols=1, persistent=0)
+        batches.append(b)
+    best = [float("inf")] * 2
+    for _ in range(8):
+        for q, b in enumerate(batches):
+            b.step(200)
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            b.step(200)
+            b.step(200)
+            torch.cuda.synchronize()
+            best[q] = min(best[q], time.perf_counter() - t)
+    for b in batches:
+        b.close()
+    assert best[0] < 1.05 * best[1]

@@ -243,7 +243,12 @@ static int batch_worklist(yh_batch* b, const yh_kernel_cfg& c, yh_batch::WL** ou
 
 // Estimated time (us) of a launch, as the plan's tiled_time (plan.cpp) over the
 // tiles of all tissues: the constants are fits to 960 timings of each kernel
-// family on batches of 2 to 100 tissues of sides 64 to 768.
+// family on batches of 2 to 100 tissues of sides 64 to 768.  It compares depths
+// of one shape well, and shapes that fill one round of workgroups; in several
+// rounds the shapes overlap one workgroup's loads with another's substeps
+// differently, which it does not know (24 masked FK tissues of 300 and 500:
+// 7 x 16 at K=4 estimated 9% under 8 x 8 at K=6, measured 22% over).  So only
+// 8 x 8, the shape without a table, is taken for several rounds; < 0: not taken.
 static double batch_time(const yh_batch* b, int rows, int waves, int K, int cus, int resident) {
   static const double fit[2][2][4] = {
       // substep, row of a wave, issue, load and store
@@ -256,14 +261,15 @@ static double batch_time(const yh_batch* b, int rows, int waves, int K, int cus,
     tiles += (int64_t)((p.nx + wout - 1) / wout) * ((p.ny + hout - 1) / hout);
   const int64_t per_cu = std::max(1, resident / cus);
   const int64_t L = (tiles + cus - 1) / cus, q = (L + per_cu - 1) / per_cu;
+  if (q > 1 && !(rows == 8 && waves == 8)) return -1.0;
   const double computed = (double)K * H - (double)K * (K + 1);
   return 4.2 + q * K * (c[0] + c[1] * rows) + L * (computed * c[2] + H * c[3]);
 }
 
 // Whether a call of n steps takes the table's launches rather than cfg's: while
-// no kernel was chosen, for an estimated gain of 3% (in the timings above never
-// more than 1.3% slower, 18% faster in the mean; a batch of a few small tissues
-// twice as fast, since cfg was picked on 256).
+// no kernel was chosen, for an estimated gain of 3% (57 other batches of 2 to 32
+// tissues, 0.03 to 8 M cells: never slower, 16% faster in the mean; a batch of a
+// few small tissues twice as fast, since cfg was picked on 256).
 static int batch_auto(yh_batch* b, int n, bool* wins) {
   *wins = false;
   if (b->chosen) return YH_OK;
