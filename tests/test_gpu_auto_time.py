@@ -1,0 +1,51 @@
+"""A plan left on AUTO against the same plan on the fixed shape and depth that
+AUTO reports: the launches an estimate chooses instead may not cost time (5% are
+for the clock).  The cases are ones where an estimate is easily off: with the
+APD update, whose rows cost their own time, and a few steps on large grids.
+"""
+import time
+
+import numpy as np
+import pytest
+
+import yolohtli_amd as Y
+from yolohtli_amd import abi_types as T
+
+pytestmark = pytest.mark.gpu
+
+
+def _times(torch, nx, ny, model, masked, apd, steps):
+    p = T.grid_params(nx, ny, model=model, solidSwitch=masked)
+    f = list(Y.initGates(nx, ny, rest=float(model), refr=float(1 - model), nvars=2 + model))
+    plans = []
+    for fixed in (False, True):
+        pl = Y.Plan(p)
+        if masked:
+            pl.set_mask(Y.make_holes(nx, ny, 20, 3.0, 9.0, 5))
+        pl.set_state(*f)
+        if apd:
+            pl.apd_enable()
+        if fixed:
+            c = pl.get_kernel()
+            pl.set_kernel(c.variant, c.substeps, c.rows, c.waves, c.cols)
+        plans.append(pl)
+    best = [float("inf")] * 2
+    for _ in range(12):
+        for q, pl in enumerate(plans):
+            pl.step(steps)
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            for _ in range(20):
+                pl.step(steps)
+            torch.cuda.synchronize()
+            best[q] = min(best[q], time.perf_counter() - t)
+    for pl in plans:
+        pl.close()
+    return best
+
+
+@pytest.mark.parametrize("nx,ny,model,masked,steps", [
+    (2912, 861, 0, 0, 33), (1345, 1723, 0, 0, 100), (2817, 121, 1, 1, 33), (136, 1708, 0, 0, 11)])
+def test_auto_with_apd(torch_cuda, nx, ny, model, masked, steps):
+    auto, fixed = _times(torch_cuda, nx, ny, model, masked, True, steps)
+    assert auto < 1.05 * fixed

@@ -110,16 +110,21 @@ static int tiled_per_cu(const yh_plan* pl, int rows, int waves, int cols, bool p
 // issue of its rows still computed (the region shrinks by two rows a substep)
 // and the loads and stores of all its rows.  Alone on a CU a workgroup does
 // not overlap them with another's, and issues less densely.  The constants are
-// least-squares fits to 1600 (shape, depth, grid) timings of each kernel
-// family, grids from 64 x 64 to 2048 x 2048 with ragged and elongated ones
-// among them, weighed towards the shapes near the best (within 8%).
-static double tiled_time(int model, bool masked, int nx, int ny, int rows, int waves, int K,
-                         int cus, int per_cu) {
-  static const double fit[2][2][5] = {
+// least-squares fits to timings of each kernel family over shapes, depths and
+// grids from 64 x 64 to 2048 x 2048, ragged and elongated ones among them, that
+// are weighed towards the shapes near the best: 4000 timings a family (within
+// 8%), 1150 with the APD update, whose crossing test makes a row cost 0.16 us
+// a substep on any shape (an estimate without it is 28% short).
+static double tiled_time(int model, bool masked, bool apd, int nx, int ny, int rows, int waves,
+                         int K, int cus, int per_cu) {
+  static const double fit[2][2][2][5] = {
       // substep, row of a wave, issue, load and store, issue alone
-      {{0.192, 0.0094, 0.0113, 0.0086, 0.0015}, {0.149, 0.0476, 0.0091, 0.0170, 0.0010}},  // 2V
-      {{0.051, 0.0514, 0.0085, 0.0201, 0.0011}, {0.030, 0.0443, 0.0086, 0.0300, 0.0025}}};  // FK
-  const double* c = fit[model == M2V ? 0 : 1][masked ? 1 : 0];
+      {{{0.192, 0.0094, 0.0113, 0.0086, 0.0015}, {0.149, 0.0476, 0.0091, 0.0170, 0.0010}},  // 2V
+       {{0.051, 0.0514, 0.0085, 0.0201, 0.0011}, {0.030, 0.0443, 0.0086, 0.0300, 0.0025}}},  // FK
+      // with APD
+      {{{0.127, 0.1296, 0.0032, 0.0522, 0.0005}, {0.068, 0.1542, 0.0018, 0.0658, 0.0008}},  // 2V
+       {{0.023, 0.1595, 0.0010, 0.0651, 0.0018}, {0.000, 0.1652, 0.0006, 0.0792, 0.0026}}}};  // FK
+  const double* c = fit[apd ? 1 : 0][model == M2V ? 0 : 1][masked ? 1 : 0];
   const int64_t tiles = tile_count(nx, ny, rows, waves, 1, K);
   const int64_t L = (tiles + cus - 1) / cus, b = (L + per_cu - 1) / per_cu;
   const int H = rows * waves;
@@ -135,7 +140,7 @@ static double tiled_time(int model, bool masked, int nx, int ny, int rows, int w
 void auto_table(int model, bool masked, const KParams& k, int cus, bool apd, AutoTable* t) {
   t->fill(std::min(k.nx, k.ny) - 1, [&](int rows, int waves, int K) {
     if (apd && !tiled_apd_supported(rows, waves, 1)) return -1.0;
-    return tiled_time(model, masked, k.nx, k.ny, rows, waves, K, std::max(1, cus),
+    return tiled_time(model, masked, apd, k.nx, k.ny, rows, waves, K, std::max(1, cus),
                       tiled_per_cu(model, masked, k, rows, waves, 1, false, apd));
   });
 }
@@ -151,7 +156,7 @@ bool auto_wins(const AutoTable& t, int model, bool masked, const KParams& k, int
   const int per_cu = tiled_per_cu(model, masked, k, c.rows, c.waves, c.cols, false, apd);
   const int K = c.substeps, r = n % K;
   auto us = [&](int d) {
-    return tiled_time(model, masked, k.nx, k.ny, c.rows, c.waves, d, std::max(1, cus), per_cu);
+    return tiled_time(model, masked, apd, k.nx, k.ny, c.rows, c.waves, d, std::max(1, cus), per_cu);
   };
   return t.of(n) < 0.97 * ((n / K) * us(K) + (r ? us(r) : 0.0));
 }
