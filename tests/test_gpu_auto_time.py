@@ -49,3 +49,10 @@ def _times(torch, nx, ny, model, masked, apd, steps):
 def test_auto_with_apd(torch_cuda, nx, ny, model, masked, steps):
     auto, fixed = _times(torch_cuda, nx, ny, model, masked, True, steps)
     assert auto < 1.05 * fixed
+
+
+@pytest.mark.parametrize("nx,ny,model,masked,steps", [
+    (1136, 2590, 0, 0, 3), (1914, 1515, 0, 0, 3), (1686, 1875, 0, 1, 5), (2159, 1607, 1, 0, 5)])
+def test_auto_with_few_steps_on_large_grids(torch_cuda, nx, ny, model, masked, steps):
+    auto, fixed = _times(torch_cuda, nx, ny, model, masked, False, steps)
+    assert auto < 1.05 * fixed

@@ -146,11 +146,15 @@ void auto_table(int model, bool masked, const KParams& k, int cus, bool apd, Aut
 }
 
 // Whether a call of n steps takes the table's launches rather than launches of
-// the fixed configuration c (auto_cfg): only for an estimated gain of 3%, the
-// estimate's spread near the best.  In the timings above that is never slower
-// and 13% faster in the mean; 20-40% on ragged grids whose tiles of the fixed
-// shape would fill a last round badly (1300 x 1300 masked FK: 2.76 against
-// 3.89 us a step), 10-25% below 400 x 400 (4 x 8 regions at K=12).
+// the fixed configuration c (auto_cfg): for an estimated gain of 3%.  On 1200
+// other grids from 64 to 3000 a side (4700 calls of 1 to 100 steps) calls take
+// 14% less time in the mean than with c, 20-40% on ragged grids whose tiles of
+// the fixed shape would fill a last round badly (1300 x 1300 masked FK: 2.76
+// against 3.89 us a step), 10-25% below 400 x 400 (4 x 8 regions at K=12), and
+// at most 5% more.  A call of a few steps where c is 8 x 8, a single launch on
+// a large grid, needs 10%: it moves the state once for little arithmetic, and
+// what the estimate says of shapes that do that alike was off by up to 13%
+// (1136 x 2590 2V, 3 steps: 12.9 us, and 14.4 on 7 x 16).
 bool auto_wins(const AutoTable& t, int model, bool masked, const KParams& k, int cus,
                const yh_kernel_cfg& c, bool apd, int n) {
   const int per_cu = tiled_per_cu(model, masked, k, c.rows, c.waves, c.cols, false, apd);
@@ -158,7 +162,8 @@ bool auto_wins(const AutoTable& t, int model, bool masked, const KParams& k, int
   auto us = [&](int d) {
     return tiled_time(model, masked, apd, k.nx, k.ny, c.rows, c.waves, d, std::max(1, cus), per_cu);
   };
-  return t.of(n) < 0.97 * ((n / K) * us(K) + (r ? us(r) : 0.0));
+  const double gain = n <= K && c.rows == 8 && c.waves == 8 && !apd ? 0.90 : 0.97;
+  return t.of(n) < gain * ((n / K) * us(K) + (r ? us(r) : 0.0));
 }
 
 yh_kernel_cfg resolve_cfg(const yh_plan* pl) {
