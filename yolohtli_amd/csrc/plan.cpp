@@ -226,6 +226,18 @@ static int write_through(const yh_plan* pl, int rows, int waves, int cols, int K
                              tiled_per_cu(pl, rows, waves, cols, prev));
 }
 
+// Allocates prev_u unless `s` is being captured; it stays null on failure.
+static void alloc_prev_u(yh_plan* pl, hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  hipError_t e = hipStreamIsCapturing(s, &st);
+  if (e == hipSuccess && st == hipStreamCaptureStatusNone)
+    e = hipMalloc(&pl->prev_u, pl->n * sizeof(float));
+  if (e != hipSuccess) {
+    pl->prev_u = nullptr;
+    (void)hipGetLastError();
+  }
+}
+
 int plan_advance(yh_plan* pl, int nsteps, hipStream_t s) {
   if (nsteps < 0) return YH_EINVAL;
   if (nsteps == 0) return YH_OK;
@@ -246,14 +258,19 @@ int plan_advance(yh_plan* pl, int nsteps, hipStream_t s) {
     const GParams g = make_gparams(pl->p, pl->stim_on, pl->stim_x, pl->stim_y);
     if (!pl->general.limit)
       pl->general = general_table(pl->p.model, g, order, kGenDeepest, pl->cus);
+    // prev_u may be missing: no memory for it, or first steps that a stream
+    // capture records, when none may be allocated.  Then a call ends on a launch
+    // of one step.
+    if (!pl->prev_u && nsteps > 1) alloc_prev_u(pl, s);
     while (remaining > 0) {
-      const GenShape shape = pl->general.next(remaining);
+      GenShape shape = pl->general.next(remaining);
+      if (!pl->prev_u && shape.K == remaining && remaining > 1)
+        shape = pl->general.next(remaining - 1);
       const int K = shape.K;
       // u one step before the end: a launch of several steps writes it, one of a
       // single step leaves it in the other state buffer (a fifth of such a
       // launch's traffic: one Dirichlet step of 4096 x 4096 145 -> 117 us)
       const bool prev = K == remaining && K > 1;
-      if (prev && !pl->prev_u) YH_HIP(hipMalloc(&pl->prev_u, pl->n * sizeof(float)));
       CFields ci;
       Fields co;
       fields(pl->cur, &ci, &co);
@@ -387,9 +404,6 @@ int yh_plan_create(const yh_params* p, yh_plan** out) {
   const size_t bytes = pl->n * sizeof(float);
   for (int b = 0; b < 2 && e == hipSuccess; ++b)
     for (int a = 0; a < pl->nv && e == hipSuccess; ++a) e = hipMalloc(&pl->buf[b][a], bytes);
-  // the general path keeps u of the step before the last on every call
-  if (e == hipSuccess && !standard_branch(*p) && p->timeIntOrder == 1)
-    e = hipMalloc(&pl->prev_u, bytes);
   if (e == hipSuccess) e = hipMalloc(&pl->tips_d, sizeof(yh_tip) * pl->tipcap);
   if (e == hipSuccess) e = hipMalloc(&pl->keys_d, sizeof(int) * pl->tipcap);
   if (e == hipSuccess) e = hipMalloc(&pl->tipcount_d, sizeof(int));
