@@ -405,6 +405,7 @@ __global__ __launch_bounds__(kGenThreads) void k_general(
         const int ox[8] = {-1, 1, 0, 0, -1, 1, 1, -1}, oy[8] = {0, 0, 1, -1, -1, 1, -1, 1};
 #pragma unroll
         for (int n = 0; n < 8; ++n) {
+          if (n >= 4 && !g.aniso) break;  // only the cross term reads the diagonals
           const int ni = gi + ox[n], nj = gj + oy[n];
           const bool inside = ni >= 0 && ni < nx && nj >= 0 && nj < ny;
           if (inside && sc && (!solid || solid[ni + nx * nj] != 0))
