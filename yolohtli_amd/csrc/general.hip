@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 
 #include "plan.h"
@@ -65,26 +66,26 @@ GParams make_gparams(const yh_params& p, int stim_on, int stim_x, int stim_y) {
   g.u_v = (float)f.u_v;
   g.u_csi = (float)f.u_csi;
   g.kk = (float)f.k;
-  g.tau_d = (float)f.tau_d;
-  g.tau_r = (float)f.tau_r;
-  g.tau_si = (float)f.tau_si;
-  g.tau_0 = (float)f.tau_0;
-  g.tau_vp = (float)f.tau_vp;
-  g.tau_v1m = (float)f.tau_v1m;
-  g.tau_v2m = (float)f.tau_v2m;
-  g.tau_wp = (float)f.tau_wp;
-  g.tau_wm = (float)f.tau_wm;
-  g.tau_2si = 2.0f * g.tau_si;
-  auto recip = [](float t) { return (float)(1.0 / (double)t); };
-  g.r_d = recip(g.tau_d);
-  g.r_r = recip(g.tau_r);
-  g.r_2si = recip(g.tau_2si);
-  g.r_0 = recip(g.tau_0);
-  g.r_vp = recip(g.tau_vp);
-  g.r_v1m = recip(g.tau_v1m);
-  g.r_v2m = recip(g.tau_v2m);
-  g.r_wp = recip(g.tau_wp);
-  g.r_wm = recip(g.tau_wm);
+  // The constants that currents and rates are divided by, as g_quotient takes
+  // them: t and r = 1/t.  An infinite one (or past the range of a float) switches
+  // its term off, a quotient of 0, which t = r = 0 gives; with the infinity the
+  // remainder would be a NaN.  One below the least normal float, whose reciprocal
+  // may overflow, counts as that.
+  auto divisor = [](float tau, float& t, float& r) {
+    t = r = 0.0f;
+    if (!(tau <= FLT_MAX)) return;
+    t = std::max(tau, FLT_MIN);
+    r = (float)(1.0 / (double)t);
+  };
+  divisor((float)f.tau_d, g.tau_d, g.r_d);
+  divisor((float)f.tau_r, g.tau_r, g.r_r);
+  divisor(2.0f * (float)f.tau_si, g.tau_2si, g.r_2si);
+  divisor((float)f.tau_0, g.tau_0, g.r_0);
+  divisor((float)f.tau_vp, g.tau_vp, g.r_vp);
+  divisor((float)f.tau_v1m, g.tau_v1m, g.r_v1m);
+  divisor((float)f.tau_v2m, g.tau_v2m, g.r_v2m);
+  divisor((float)f.tau_wp, g.tau_wp, g.r_wp);
+  divisor((float)f.tau_wm, g.tau_wm, g.r_wm);
   g.stim_on = stim_on;
   g.stim_x = stim_x;
   g.stim_y = stim_y;
@@ -94,7 +95,9 @@ GParams make_gparams(const yh_params& p, int stim_on, int stim_x, int stim_y) {
 // a / t from the reciprocal r of t, itself correctly rounded: the quotient
 // estimate a*r and its exact remainder give the correctly rounded quotient
 // (Markstein, IBM J. Res. Dev. 34(1), 1990), in 3 instructions where a
-// division takes 11; the FK currents have eight.  An infinite a gives NaN.
+// division takes 11; the FK currents have eight.  A quotient that is not finite
+// may come out as a NaN.  t and r are normal, or both 0 for a quotient of 0
+// (make_gparams).
 __device__ __forceinline__ float g_quotient(float a, float t, float r) {
   const float e = a * r;
   return __builtin_fmaf(__builtin_fmaf(-t, e, a), r, e);

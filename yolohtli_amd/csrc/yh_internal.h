@@ -335,7 +335,7 @@ struct GParams {
   int nx, ny, masked, neumann, lap4, aniso, vdiff;
   float rx, ry, rxy, rbx, rby, q4, fx4, fy4, dt, tc, rscale, bval;  // q4 = qx4 + qy4
   float mu, alpha, beta, gamma, delta, eps, theta;
-  float u_c, u_v, u_csi, kk, tau_d, tau_r, tau_si, tau_0, tau_vp, tau_v1m, tau_v2m, tau_wp,
+  float u_c, u_v, u_csi, kk, tau_d, tau_r, tau_0, tau_vp, tau_v1m, tau_v2m, tau_wp,
       tau_wm;
   float tau_2si, r_d, r_r, r_2si, r_0, r_vp, r_v1m, r_v2m, r_wp, r_wm;  // 2 tau_si; reciprocals
   int stim_on, stim_x, stim_y;
