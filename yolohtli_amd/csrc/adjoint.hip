@@ -55,7 +55,8 @@ struct FkEval {
 
 // Correctly rounded 1/t: the hardware reciprocal (within 1 ulp) and one
 // Newton step by its exact residual (Markstein, IBM J. Res. Dev. 34(1), 1990;
-// equal to the quotient 1.0f/t for every significand), 3 instructions for 11.
+// equal to the quotient 1.0f/t for every significand), 3 instructions for 11;
+// t must be normal and 1/t as well.
 __device__ __forceinline__ float recip(float t) {
   const float r = __builtin_amdgcn_rcpf(t);
   return __builtin_fmaf(__builtin_fmaf(-t, r, 1.0f), r, r);
@@ -776,9 +777,12 @@ static void adj_k(yh_adjoint* a, const double tau6[6]) {
   k.uv = (float)f.u_v;
   k.ucsi = (float)f.u_csi;
   k.uc1 = (float)(1.0 + f.u_c);
-  k.tv1m = (float)f.tau_v1m;
-  k.tv2m = (float)f.tau_v2m;
-  k.dtv = (float)(f.tau_v2m - f.tau_v1m);
+  // recip() needs a finite sum of the two: one that is infinite, or past the range
+  // of a float, switches its recovery off, as 1e30 ms does
+  const double tv1m = std::min(f.tau_v1m, 1e30), tv2m = std::min(f.tau_v2m, 1e30);
+  k.tv1m = (float)tv1m;
+  k.tv2m = (float)tv2m;
+  k.dtv = (float)(tv2m - tv1m);
   k.eh = (float)(2.0 / (p.heaviside_width * ln2));
   k.es = (float)(2.0 * f.k / ln2);
   k.tihw = (float)(2.0 / p.heaviside_width);
