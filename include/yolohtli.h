@@ -355,6 +355,15 @@ int yh_batch_autotune(yh_batch* batch, int steps, void* stream, yh_kernel_cfg* b
 typedef struct yh_adjoint yh_adjoint;
 int yh_adjoint_create(const yh_params* p, int nsteps, int rec_every, int ckpt_every,
                       const int* sensors, int nsensors, yh_adjoint** out);
+/* The same with the most bytes of device memory that kept states may take, in
+ * place of 4 GiB: 0 for checkpoints always, which bound the memory to
+ * (nsteps/ckpt_every + ckpt_every) states; negative for the 4 GiB.  (yh_adjoint_create
+ * passes -1.) */
+int yh_adjoint_create_keep(const yh_params* p, int nsteps, int rec_every, int ckpt_every,
+                           int64_t keep_bytes, const int* sensors, int nsensors,
+                           yh_adjoint** out);
+/* Whether every state is kept (1) or checkpoints are (0). */
+int yh_adjoint_keeps_states(const yh_adjoint* adj);
 void yh_adjoint_destroy(yh_adjoint* adj);
 /* Steps per launch of the forward and the reverse sweep, 1..8 (default 8):
  * 1 runs one step per launch, more run that many steps of a tile through LDS

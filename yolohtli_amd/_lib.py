@@ -74,6 +74,8 @@ PROTOTYPES = {
     "yh_batch_step_each": (I, [P, I, P]),
     "yh_batch_autotune": (I, [P, I, P, C.POINTER(YhKernelCfg), C.POINTER(C.c_float)]),
     "yh_adjoint_create": (I, [PARAMS_P, I, I, I, P, I, C.POINTER(P)]),
+    "yh_adjoint_create_keep": (I, [PARAMS_P, I, I, I, C.c_int64, P, I, C.POINTER(P)]),
+    "yh_adjoint_keeps_states": (I, [P]),
     "yh_adjoint_destroy": (None, [P]),
     "yh_adjoint_set_substeps": (I, [P, I]),
     "yh_adjoint_set_mask": (I, [P, P]),

@@ -23,9 +23,14 @@ def _protos():
 
 
 class SensorProblem:
-    """Forward + adjoint of one FK tissue with sensors (owns device buffers)."""
+    """Forward + adjoint of one FK tissue with sensors (owns device buffers).
 
-    def __init__(self, p, nsteps, sensors, x0, rec_every=1, ckpt_every=100, mask=None):
+    keep_bytes: the most device memory that the forward's states may take, all
+    kept (4 GiB by default); with more to keep, and always with 0, a state
+    every ckpt_every steps is kept and the backward recomputes the others."""
+
+    def __init__(self, p, nsteps, sensors, x0, rec_every=1, ckpt_every=100, mask=None,
+                 keep_bytes=None):
         L = _protos()
         self.p = T.copy_params(p)
         self.nsteps = int(nsteps)
@@ -33,8 +38,9 @@ class SensorProblem:
         self.sensors = np.ascontiguousarray(sensors, dtype=np.int32)
         self.nrec = self.nsteps // self.rec
         h = C.c_void_p()
-        check(L.yh_adjoint_create(C.byref(self.p), self.nsteps, self.rec, int(ckpt_every),
-                                  _ptr(self.sensors), len(self.sensors), C.byref(h)),
+        check(L.yh_adjoint_create_keep(C.byref(self.p), self.nsteps, self.rec, int(ckpt_every),
+                                       -1 if keep_bytes is None else int(keep_bytes),
+                                       _ptr(self.sensors), len(self.sensors), C.byref(h)),
               "yh_adjoint_create")
         self._h = h
         if mask is not None:
@@ -45,6 +51,11 @@ class SensorProblem:
               "yh_adjoint_set_initial")
         self._last = None
         self._gen = 0
+
+    @property
+    def keeps_states(self):
+        """Whether every state of the forward is kept."""
+        return bool(_protos().yh_adjoint_keeps_states(self._h))
 
     def set_substeps(self, k):
         """Steps per launch of the forward and reverse sweeps (1: one-step

@@ -800,8 +800,9 @@ static void adj_k(yh_adjoint* a, const double tau6[6]) {
   adj_tau_factors(tdt, tau6, a->tau_f);
 }
 
-// Most device memory a problem takes to keep every state of its forward sweep.
-constexpr size_t kAdjKeep = (size_t)4 << 30;
+// Most device memory a problem takes to keep every state of its forward sweep,
+// unless the caller sets another limit.
+constexpr int64_t kAdjKeep = (int64_t)4 << 30;
 
 static inline float* slot(float* base, size_t n, int s, int var) {
   return base + ((size_t)s * 3 + var) * n;
@@ -815,6 +816,12 @@ extern "C" {
 
 int yh_adjoint_create(const yh_params* p, int nsteps, int rec_every, int ckpt_every,
                       const int* sensors, int nsensors, yh_adjoint** out) {
+  return yh_adjoint_create_keep(p, nsteps, rec_every, ckpt_every, -1, sensors, nsensors, out);
+}
+
+int yh_adjoint_create_keep(const yh_params* p, int nsteps, int rec_every, int ckpt_every,
+                           int64_t keep_bytes, const int* sensors, int nsensors,
+                           yh_adjoint** out) {
   if (!p || !out || nsteps < 1 || rec_every < 1 || ckpt_every < 1 || nsensors < 1 || !sensors)
     return YH_EINVAL;
   if (p->model != YH_MODEL_3V_FK || !(p->heaviside_width > 0) || p->reduceSym)
@@ -866,13 +873,14 @@ int yh_adjoint_create(const yh_params* p, int nsteps, int rec_every, int ckpt_ev
       M((void**)&a->lam[b][q], n * 4);
     }
   for (int q = 0; q < 3; ++q) M((void**)&a->X0[q], n * 4);
-  // All states where they take at most kAdjKeep and a quarter of what is free
+  // All states where they take at most the limit and a quarter of what is free
   // on the device: recomputing each segment is a second forward sweep (2.4 of
   // 9.0 ms per gradient at 256 x 256 x 2000, whose states are 1.6 GB of 288).
   // If they cannot be had, the checkpoints the caller asked for.
   const size_t all = (size_t)(nsteps + 1) * 3 * n * 4;
   size_t avail = 0, total = 0;
-  if (e == hipSuccess && all <= kAdjKeep && hipMemGetInfo(&avail, &total) == hipSuccess &&
+  const size_t limit = (size_t)(keep_bytes < 0 ? kAdjKeep : keep_bytes);
+  if (e == hipSuccess && all <= limit && hipMemGetInfo(&avail, &total) == hipSuccess &&
       all <= avail / 4) {
     a->keep = hipMalloc(&a->seg, all) == hipSuccess;
     if (!a->keep) {
@@ -906,6 +914,8 @@ void yh_adjoint_destroy(yh_adjoint* a) {
   if (a) (void)hipDeviceSynchronize();
   adj_free(a);
 }
+
+int yh_adjoint_keeps_states(const yh_adjoint* a) { return a && a->keep ? 1 : 0; }
 
 int yh_adjoint_set_substeps(yh_adjoint* a, int k) {
   if (!a || k < 1 || k > kAdjKmax) return YH_EINVAL;
