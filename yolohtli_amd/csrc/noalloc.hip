@@ -37,9 +37,10 @@ static int g_cus[kMaxDevices] = {};
 // The device address of this device's copy of `scratch` (the host-side name
 // is a stand-in, not a device address) and the device's CU count, looked up
 // once per device with that device current.
-static int scratch_of_current_device(unsigned char** ptr, int* cus) {
+static int scratch_of_current_device(unsigned char** ptr, int* cus, int* device) {
   int dev = 0;
   YH_HIP(hipGetDevice(&dev));
+  *device = dev;
   if (dev < 0 || dev >= kMaxDevices) return YH_EINVAL;
   std::lock_guard<std::mutex> lock(g_mu);
   if (!g_scratch[dev]) {
@@ -53,6 +54,41 @@ static int scratch_of_current_device(unsigned char** ptr, int* cus) {
   *ptr = g_scratch[dev];
   *cus = g_cus[dev];
   return YH_OK;
+}
+
+// The launches of a YH_KERNEL_AUTO call, which depend on what a Key holds.
+struct Auto {
+  struct Key {
+    int dev, model, masked, iso, nx, ny;
+    bool operator==(const Key& o) const {
+      return dev == o.dev && model == o.model && masked == o.masked && iso == o.iso && nx == o.nx &&
+             ny == o.ny;
+    }
+  };
+  Key key{-1, 0, 0, 0, 0, 0};
+  yh_kernel_cfg cfg{};
+  AutoTable table;
+};
+
+// The last few of them, in fixed storage: a call of few steps is made in a tight
+// loop, where the table's 95 estimates took as long as a launch (one step of
+// 512 x 512 FK, calls back to back: 3.8 us, 7.6 with a table a call).
+static Auto auto_of(const Auto::Key& key, const KParams& k, int cus) {
+  static std::mutex mu;
+  static Auto last[8];
+  static int turn = 0;
+  std::lock_guard<std::mutex> lock(mu);
+  for (const Auto& a : last)
+    if (a.key == key) return a;
+  Auto& a = last[turn];
+  turn = (turn + 1) % 8;
+  a.key = Auto::Key{-1, 0, 0, 0, 0, 0};
+  const bool masked = key.masked != 0;
+  const bool pairs = tiled_per_cu(key.model, masked, k, 4, 16, 1, false, false) >= 2;
+  a.cfg = auto_cfg(key.nx, key.ny, cus, pairs);
+  auto_table(key.model, masked, k, cus, false, &a.table);
+  a.key = key;
+  return a;
 }
 
 }  // namespace yh
@@ -81,8 +117,8 @@ int yh_step_noalloc(const yh_params* p, float* const out[3], const float* const 
     return YH_OK;
   }
   unsigned char* base = nullptr;
-  int cus = 0;
-  rc = scratch_of_current_device(&base, &cus);
+  int cus = 0, dev = 0;
+  rc = scratch_of_current_device(&base, &cus, &dev);
   if (rc) return rc;
   float* mid[3] = {nullptr, nullptr, nullptr};
   for (int a = 0; a < nv; ++a) mid[a] = reinterpret_cast<float*>(base + a * kFieldBytes);
@@ -95,10 +131,9 @@ int yh_step_noalloc(const yh_params* p, float* const out[3], const float* const 
   // (neither the split, the remainder merge it may use nor the store policy
   // changes a value: the result does not depend on where launches split, so it
   // equals yh_step's bit for bit)
-  const bool pairs = tiled_per_cu(p->model, masked, k, 4, 16, 1, false, false) >= 2;
-  const yh_kernel_cfg c = auto_cfg(p->nx, p->ny, cus, pairs);
-  AutoTable t;
-  auto_table(p->model, masked, k, cus, false, &t);
+  const Auto a = auto_of({dev, p->model, masked, k.iso, p->nx, p->ny}, k, cus);
+  const AutoTable& t = a.table;
+  const yh_kernel_cfg& c = a.cfg;
   const bool split = auto_wins(t, p->model, masked, k, cus, c, false, nsteps);
   auto next = [&](int remaining) {
     yh_kernel_cfg l = split ? t.next(remaining) : c;
