@@ -339,8 +339,11 @@ int yh_batch_step(yh_batch* batch, int nsteps, void* stream);
  * tissue per k-step chunk (the comparison the batched launch is measured
  * against). */
 int yh_batch_step_each(yh_batch* batch, int nsteps, void* stream);
-/* Times tile shapes x substep depths x {persistent, one-per-item} on the
- * batch's own state (restored afterwards) and installs the fastest. */
+/* Times tile shapes x substep depths x {persistent, one-per-item} in whole calls
+ * of `steps` steps on the batch's own state (restored afterwards) and installs the
+ * fastest.  Where the launches of a batch without a chosen kernel are, the batch
+ * goes back to those; best and yh_batch_get_kernel then hold the kernel it
+ * started as. */
 int yh_batch_autotune(yh_batch* batch, int steps, void* stream, yh_kernel_cfg* best,
                       float* best_ms);
 

@@ -97,3 +97,44 @@ def test_untuned_batch_is_not_slower_than_one_shape(torch_cuda, model, ntissues,
     for b in batches:
         b.close()
     assert best[0] < 1.05 * best[1]
+
+
+@pytest.mark.parametrize("model,ntissues,sides,steps", [(1, 1, (64,), 15), (0, 2, (64,), 16),
+                                                        (1, 3, (128, 256), 13)])
+def test_tuned_batch_is_not_slower_than_an_untuned_one(torch_cuda, model, ntissues, sides, steps):
+    """The launches of a batch without a chosen kernel are among the tuner's
+    candidates, in whole calls of the size it is given (8% are for the clock); the
+    state is as before the tuning, and the steps after it are the same bits."""
+    torch = torch_cuda
+    params, masks, fields = batched_workload(ntissues=ntissues, model=model, sides=sides,
+                                             max_holes=4)
+    batches = []
+    for tuned in (False, True):
+        b = Batch(params)
+        for t, (m, f) in enumerate(zip(masks, fields)):
+            b.set_mask(t, m)
+            b.set_state(t, *f)
+        b.step(9)
+        if tuned:
+            cfg, ms = b.autotune(steps=steps)
+            assert cfg[0] == T.YH_KERNEL_TILED and ms > 0
+            assert cfg == b.get_kernel()[0]
+        b.step(steps)
+        batches.append(b)
+    for t in range(ntissues):
+        for x, y in zip(batches[0].get_state(t), batches[1].get_state(t)):
+            np.testing.assert_array_equal(x, y)
+    best = [float("inf")] * 2
+    for _ in range(12):
+        for q, b in enumerate(batches):
+            b.step(steps)
+            b.step(steps)
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            for _ in range(40):
+                b.step(steps)
+            torch.cuda.synchronize()
+            best[q] = min(best[q], time.perf_counter() - t)
+    for b in batches:
+        b.close()
+    assert best[1] < 1.08 * best[0]

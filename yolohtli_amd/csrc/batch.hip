@@ -163,6 +163,7 @@ struct yh_batch {
   // capped at creation by the smallest tissue (reflected halos are exact for
   // at most min(nx, ny) - 1 substeps)
   yh_kernel_cfg cfg{YH_KERNEL_TILED, 6, 8, 8, 1};
+  yh_kernel_cfg first{};  // cfg as created
   int persistent = 0;
   // until a kernel is set or tuned, calls may take other shapes and depths
   // (the same results) where an estimate of their time is lower
@@ -305,6 +306,18 @@ static yh_kernel_cfg batch_next(const yh_batch* b, bool table, int remaining) {
   return c;
 }
 
+// The work lists of a call of nsteps (they allocate).
+static int batch_lists(yh_batch* b, int nsteps, bool table) {
+  for (int rem = nsteps; rem > 0;) {
+    const yh_kernel_cfg c = batch_next(b, table, rem);
+    yh_batch::WL* w = nullptr;
+    const int rc = batch_worklist(b, c, &w);
+    if (rc) return rc;
+    rem -= c.substeps;
+  }
+  return YH_OK;
+}
+
 // Enqueue nsteps.
 static int batch_enqueue(yh_batch* b, int nsteps, bool table, hipStream_t s) {
   int remaining = nsteps;
@@ -392,6 +405,7 @@ int yh_batch_create(const yh_params* per_tissue, int ntissues, yh_batch** out) {
   b->mask_set.assign(ntissues, 0);
   for (int t = 0; t < ntissues; ++t)
     b->cfg.substeps = std::min(b->cfg.substeps, std::min(b->p[t].nx, b->p[t].ny) - 1);
+  b->first = b->cfg;
   hipError_t e = hipSuccess;
   for (int q = 0; q < 2 && e == hipSuccess; ++q)
     for (int a = 0; a < b->nv && e == hipSuccess; ++a) {
@@ -508,14 +522,9 @@ int yh_batch_step(yh_batch* b, int nsteps, void* stream) {
   int nlaunch = 0;
   for (int rem = nsteps; rem > 0; rem -= batch_next(b, table, rem).substeps) ++nlaunch;
   if (it == b->graphs.end()) {
-    // build the work lists outside the capture (they allocate)
-    for (int rem = nsteps; rem > 0;) {
-      const yh_kernel_cfg c = batch_next(b, table, rem);
-      yh_batch::WL* w = nullptr;
-      rc = batch_worklist(b, c, &w);
-      if (rc) return rc;
-      rem -= c.substeps;
-    }
+    // build the work lists outside the capture
+    rc = batch_lists(b, nsteps, table);
+    if (rc) return rc;
     int res = 0;
     rc = batch_resident(b->model, b->masked, b->iso, b->cfg.rows, b->cfg.waves, b->cfg.cols,
                             &res);
@@ -581,7 +590,7 @@ int yh_batch_autotune(yh_batch* b, int steps, void* stream, yh_kernel_cfg* best,
   }
   const yh_kernel_cfg cfg0 = b->cfg;
   const int pers0 = b->persistent;
-  const bool graph0 = b->use_graph;
+  const bool graph0 = b->use_graph, chosen0 = b->chosen;
   const int64_t count0 = b->count;
   b->use_graph = false;
   hipEvent_t e0, e1;
@@ -592,38 +601,54 @@ int yh_batch_autotune(yh_batch* b, int steps, void* stream, yh_kernel_cfg* best,
   const int shapes[][3] = {{4, 8, 1}, {8, 8, 1}, {4, 16, 1}, {8, 16, 1}, {7, 16, 1},
                            {4, 8, 2}, {4, 16, 2}};
   const int Ks[] = {2, 4, 6, 8, 9, 10, 12};
-  yh_kernel_cfg bestc = cfg0;
-  int bestp = pers0;
+  // The time of a step in whole calls of `steps` (64 steps and more of them), a
+  // call's last launch included; the lists are made and the kernels have run
+  // before.
+  auto time_calls = [&](bool table, float* ms_per_step) {
+    const int calls = (63 + steps) / steps;
+    int r = batch_lists(b, steps, table);
+    if (!r) r = batch_enqueue(b, std::min(steps, 256), table, s);
+    if (r) return r;
+    if (hipEventRecord(e0, s) != hipSuccess) return (int)YH_EHIP;
+    for (int i = 0; i < calls && !r; ++i) r = batch_enqueue(b, steps, table, s);
+    if (r) return r;
+    if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess)
+      return (int)YH_EHIP;
+    float ms = 0.f;
+    (void)hipEventElapsedTime(&ms, e0, e1);
+    *ms_per_step = ms / ((float)calls * steps);
+    return (int)YH_OK;
+  };
+  // first the launches of a batch without a choice, so that one is made only
+  // where it is faster
+  yh_kernel_cfg bestc = b->first;
+  int bestp = 0;
+  bool bestauto = true, table = false;
   float bestt = 1e30f;
-  int rc = YH_OK;
+  b->cfg = b->first;
+  b->persistent = 0;
+  b->chosen = false;
+  int rc = batch_auto(b, steps, &table);
+  if (!rc) rc = time_calls(table, &bestt);
   for (int K : Ks) {
+    if (rc) break;
     if (K > minside - 1) continue;
     for (auto& sh : shapes) {
+      if (rc) break;
       if (2 * K >= 64 * sh[2] || 2 * K >= sh[0] * sh[1]) continue;
-      for (int pers = 0; pers < 2; ++pers) {
+      for (int pers = 0; pers < 2 && !rc; ++pers) {
         b->cfg = yh_kernel_cfg{YH_KERNEL_TILED, K, sh[0], sh[1], sh[2]};
         b->persistent = pers;
-        const int n = std::max(K, (steps / K) * K);
-        rc = batch_enqueue(b, K, false, s);
-        if (rc) break;
-        if (hipEventRecord(e0, s) != hipSuccess) { rc = YH_EHIP; break; }
-        rc = batch_enqueue(b, n, false, s);
-        if (rc) break;
-        if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess) {
-          rc = YH_EHIP;
-          break;
-        }
-        float ms = 0.f;
-        (void)hipEventElapsedTime(&ms, e0, e1);
-        if (ms / n < bestt) {
-          bestt = ms / n;
+        float t = 0.f;
+        rc = time_calls(false, &t);
+        if (!rc && t < bestt) {
+          bestt = t;
           bestc = b->cfg;
           bestp = pers;
+          bestauto = false;
         }
       }
-      if (rc) break;
     }
-    if (rc) break;
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
@@ -641,11 +666,12 @@ int yh_batch_autotune(yh_batch* b, int steps, void* stream, yh_kernel_cfg* best,
   if (rc) {
     b->cfg = cfg0;
     b->persistent = pers0;
+    b->chosen = chosen0;
     return rc;
   }
   b->cfg = bestc;
   b->persistent = bestp;
-  b->chosen = true;
+  b->chosen = !bestauto;
   if (best) *best = bestc;
   if (best_ms) *best_ms = bestt;
   return YH_OK;
