@@ -341,9 +341,9 @@ int yh_batch_step(yh_batch* batch, int nsteps, void* stream);
 int yh_batch_step_each(yh_batch* batch, int nsteps, void* stream);
 /* Times tile shapes x substep depths x {persistent, one-per-item} in whole calls
  * of `steps` steps on the batch's own state (restored afterwards) and installs the
- * fastest.  Where the launches of a batch without a chosen kernel are, the batch
- * goes back to those; best and yh_batch_get_kernel then hold the kernel it
- * started as. */
+ * fastest, which best and yh_batch_get_kernel hold.  Where the launches of a
+ * batch without a chosen kernel are faster still, the batch steps by those
+ * until yh_batch_set_kernel (best_ms is their time). */
 int yh_batch_autotune(yh_batch* batch, int steps, void* stream, yh_kernel_cfg* best,
                       float* best_ms);
 

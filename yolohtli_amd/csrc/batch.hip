@@ -165,11 +165,12 @@ struct yh_batch {
   yh_kernel_cfg cfg{YH_KERNEL_TILED, 6, 8, 8, 1};
   yh_kernel_cfg first{};  // cfg as created
   int persistent = 0;
-  // until a kernel is set or tuned, calls may take other shapes and depths
-  // (the same results) where an estimate of their time is lower
-  bool chosen = false;
+  // until a kernel is set or tuned, calls may take other shapes and depths than
+  // `first` (the same results) where an estimate of their time is lower; the
+  // tuner may find that faster than cfg, the fastest kernel it timed
+  bool free = true;
   yh::AutoTable table;
-  double cfg_us[8];  // the same estimate of cfg's launches of 0 .. 6 steps
+  double first_us[8];  // the same estimate of first's launches of 0 .. 6 steps
   bool use_graph = true;
   int64_t count = 0;
   // work lists: (K, rows, waves, cols) -> (tissue table, items, nitems).  Calls
@@ -267,14 +268,14 @@ static double batch_time(const yh_batch* b, int rows, int waves, int K, int cus,
   return 4.2 + q * K * (c[0] + c[1] * rows) + L * (computed * c[2] + H * c[3]);
 }
 
-// Whether a call of n steps takes the table's launches rather than cfg's: while
-// no kernel was chosen, for an estimated gain of 3% (57 other batches of 2 to 32
+// Whether a call of n steps takes the table's launches rather than first's: while
+// the batch is free, for an estimated gain of 3% (57 other batches of 2 to 32
 // tissues, 0.03 to 8 M cells: never slower, 16% faster in the mean; a batch of a
-// few small tissues twice as fast, since cfg was picked on 256).
+// few small tissues twice as fast, since first was picked on 256).
 static int batch_auto(yh_batch* b, int n, bool* wins) {
   *wins = false;
-  if (b->chosen) return YH_OK;
-  const int K0 = b->cfg.substeps;
+  if (!b->free) return YH_OK;
+  const int K0 = b->first.substeps;
   if (!b->table.ready) {
     int dev = 0, cus = 0, rc = YH_OK, side = 1 << 30;
     YH_HIP(hipGetDevice(&dev));
@@ -288,20 +289,20 @@ static int batch_auto(yh_batch* b, int n, bool* wins) {
     };
     for (const yh_params& p : b->p) side = std::min({side, p.nx, p.ny});
     b->table.fill(side - 1, us);
-    for (int K = 1; K <= K0; ++K) b->cfg_us[K] = us(b->cfg.rows, b->cfg.waves, K);
-    b->cfg_us[0] = 0.0;
+    for (int K = 1; K <= K0; ++K) b->first_us[K] = us(b->first.rows, b->first.waves, K);
+    b->first_us[0] = 0.0;
     if (rc) {
       b->table.ready = false;
       return rc;
     }
   }
-  *wins = b->table.of(n) < 0.97 * ((n / K0) * b->cfg_us[K0] + b->cfg_us[n % K0]);
+  *wins = b->table.of(n) < 0.97 * ((n / K0) * b->first_us[K0] + b->first_us[n % K0]);
   return YH_OK;
 }
 
 // The launch with `remaining` steps to go.
 static yh_kernel_cfg batch_next(const yh_batch* b, bool table, int remaining) {
-  yh_kernel_cfg c = table ? b->table.next(remaining) : b->cfg;
+  yh_kernel_cfg c = table ? b->table.next(remaining) : b->free ? b->first : b->cfg;
   c.substeps = std::min(c.substeps, remaining);
   return c;
 }
@@ -327,7 +328,7 @@ static int batch_enqueue(yh_batch* b, int nsteps, bool table, hipStream_t s) {
     int rc = batch_worklist(b, c, &w);
     if (rc) return rc;
     int grid = w->nitems;
-    if (b->persistent && !table) {
+    if (b->persistent && !b->free) {
       int res = 0;
       rc = batch_resident(b->model, b->masked, b->iso, c.rows, c.waves, c.cols, &res);
       if (rc) return rc;
@@ -488,7 +489,7 @@ int yh_batch_set_kernel(yh_batch* b, const yh_kernel_cfg* cfg, int persistent) {
     if (cfg->substeps > std::min(b->p[t].nx, b->p[t].ny) - 1) return YH_EINVAL;
   b->cfg = *cfg;
   b->persistent = persistent ? 1 : 0;
-  b->chosen = true;
+  b->free = false;
   return YH_OK;
 }
 
@@ -514,10 +515,11 @@ int yh_batch_step(yh_batch* b, int nsteps, void* stream) {
     b->count += nsteps;
     return YH_OK;
   }
+  // (a free batch's launches follow from the number of steps)
   const auto key =
-      table ? std::make_tuple(nsteps, b->cur, 0, 0, 0, 0, 0)
-            : std::make_tuple(nsteps, b->cur, b->cfg.substeps, b->cfg.rows, b->cfg.waves,
-                              b->cfg.cols, b->persistent);
+      b->free ? std::make_tuple(nsteps, b->cur, 0, 0, 0, 0, 0)
+              : std::make_tuple(nsteps, b->cur, b->cfg.substeps, b->cfg.rows, b->cfg.waves,
+                                b->cfg.cols, b->persistent);
   auto it = b->graphs.find(key);
   int nlaunch = 0;
   for (int rem = nsteps; rem > 0; rem -= batch_next(b, table, rem).substeps) ++nlaunch;
@@ -590,7 +592,7 @@ int yh_batch_autotune(yh_batch* b, int steps, void* stream, yh_kernel_cfg* best,
   }
   const yh_kernel_cfg cfg0 = b->cfg;
   const int pers0 = b->persistent;
-  const bool graph0 = b->use_graph, chosen0 = b->chosen;
+  const bool graph0 = b->use_graph, free0 = b->free;
   const int64_t count0 = b->count;
   b->use_graph = false;
   hipEvent_t e0, e1;
@@ -619,17 +621,14 @@ int yh_batch_autotune(yh_batch* b, int steps, void* stream, yh_kernel_cfg* best,
     *ms_per_step = ms / ((float)calls * steps);
     return (int)YH_OK;
   };
-  // first the launches of a batch without a choice, so that one is made only
-  // where it is faster
   yh_kernel_cfg bestc = b->first;
   int bestp = 0;
-  bool bestauto = true, table = false;
-  float bestt = 1e30f;
-  b->cfg = b->first;
-  b->persistent = 0;
-  b->chosen = false;
+  bool table = false;
+  float bestt = 1e30f, freet = 1e30f;
+  b->free = true;
   int rc = batch_auto(b, steps, &table);
-  if (!rc) rc = time_calls(table, &bestt);
+  if (!rc) rc = time_calls(table, &freet);
+  b->free = false;
   for (int K : Ks) {
     if (rc) break;
     if (K > minside - 1) continue;
@@ -645,7 +644,6 @@ int yh_batch_autotune(yh_batch* b, int steps, void* stream, yh_kernel_cfg* best,
           bestt = t;
           bestc = b->cfg;
           bestp = pers;
-          bestauto = false;
         }
       }
     }
@@ -666,14 +664,14 @@ int yh_batch_autotune(yh_batch* b, int steps, void* stream, yh_kernel_cfg* best,
   if (rc) {
     b->cfg = cfg0;
     b->persistent = pers0;
-    b->chosen = chosen0;
+    b->free = free0;
     return rc;
   }
   b->cfg = bestc;
   b->persistent = bestp;
-  b->chosen = !bestauto;
+  b->free = freet <= bestt;
   if (best) *best = bestc;
-  if (best_ms) *best_ms = bestt;
+  if (best_ms) *best_ms = std::min(freet, bestt);
   return YH_OK;
 }
 
