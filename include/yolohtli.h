@@ -274,8 +274,10 @@ int yh_contour(yh_plan* plan, int mode, double th1, double th2, double th3, cons
  * masked, call size) for the process.  steps: the number of steps per
  * yh_step call the plan will be driven with (capped at 2000); each
  * candidate is timed over whole calls of that size, at least 400 steps in
- * all, so a call's remainder launch counts.  best / best_ms (ms per step)
- * may be NULL. */
+ * all, so a call's remainder launch counts.  Where the launches of
+ * YH_KERNEL_AUTO are faster than the fastest configuration the plan steps by
+ * those until yh_set_kernel; best and yh_get_kernel hold the configuration.
+ * best / best_ms (ms per step) may be NULL. */
 int yh_autotune(yh_plan* plan, int steps, void* stream, yh_kernel_cfg* best, float* best_ms);
 
 /* ----------------------------------------------------- symmetry reduction */

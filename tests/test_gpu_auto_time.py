@@ -56,3 +56,40 @@ def test_auto_with_apd(torch_cuda, nx, ny, model, masked, steps):
 def test_auto_with_few_steps_on_large_grids(torch_cuda, nx, ny, model, masked, steps):
     auto, fixed = _times(torch_cuda, nx, ny, model, masked, False, steps)
     assert auto < 1.05 * fixed
+
+
+@pytest.mark.parametrize("nx,ny,model,masked,steps", [(801, 775, 1, 1, 37), (64, 64, 1, 0, 47),
+                                                      (1300, 1300, 1, 1, 20)])
+def test_tuned_plan_is_not_slower_than_auto(torch_cuda, nx, ny, model, masked, steps):
+    """AUTO's split, here of unequal launches, is a candidate of the tuner."""
+    torch = torch_cuda
+    p = T.grid_params(nx, ny, model=model, solidSwitch=masked, diff_per=0.0004)
+    f = Y.init_random(nx, ny, 4, nvars=2 + model)
+    plans = [Y.Plan(p), Y.Plan(p)]
+    for pl in plans:
+        if masked:
+            pl.set_mask(Y.make_holes(nx, ny, 10, 2.0, 6.0, 3))
+        pl.set_state(*f)
+    cfg, ms = plans[1].autotune(steps=steps)
+    got = plans[1].get_kernel()
+    assert ms > 0 and (got.variant, got.substeps, got.rows, got.waves, got.cols) == cfg
+    ratios = []
+    for _ in range(3):  # the gain is 2-3%: measured again where the clock hides it
+        best = [float("inf")] * 2
+        for _ in range(12):
+            for q, pl in enumerate(plans):
+                pl.step(steps)
+                torch.cuda.synchronize()
+                t = time.perf_counter()
+                for _ in range(30):
+                    pl.step(steps)
+                torch.cuda.synchronize()
+                best[q] = min(best[q], time.perf_counter() - t)
+        ratios.append(best[1] / best[0])
+        if ratios[-1] < 1.015:
+            break
+    for a, b in zip(plans[0].get_state(), plans[1].get_state()):
+        np.testing.assert_array_equal(a, b)
+    for pl in plans:
+        pl.close()
+    assert min(ratios) < 1.015, ratios

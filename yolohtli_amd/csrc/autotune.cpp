@@ -15,7 +15,12 @@ namespace {
 
 using Key = std::tuple<int, int, int, int, int>;
 std::mutex g_mu;
-std::map<Key, std::pair<yh_kernel_cfg, float>> g_cache;
+struct Choice {
+  yh_kernel_cfg cfg;  // the fastest configuration
+  float ms;
+  bool split;  // YH_KERNEL_AUTO's launches are faster still, and ms their time
+};
+std::map<Key, Choice> g_cache;
 
 std::vector<yh_kernel_cfg> candidates(const yh_plan* pl) {
   std::vector<yh_kernel_cfg> c;
@@ -67,9 +72,10 @@ extern "C" int yh_autotune(yh_plan* pl, int steps, void* stream, yh_kernel_cfg* 
     std::lock_guard<std::mutex> g(g_mu);
     auto it = g_cache.find(key);
     if (it != g_cache.end()) {
-      pl->cfg = it->second.first;
-      if (best) *best = it->second.first;
-      if (best_ms) *best_ms = it->second.second;
+      pl->cfg = it->second.cfg;
+      pl->split = it->second.split;
+      if (best) *best = it->second.cfg;
+      if (best_ms) *best_ms = it->second.ms;
       return YH_OK;
     }
   }
@@ -101,10 +107,13 @@ extern "C" int yh_autotune(yh_plan* pl, int steps, void* stream, yh_kernel_cfg* 
   // (the previous-u and merged-remainder variants) are loaded and their
   // occupancy known before the caller's first call.
   const bool apd0 = pl->apd_on;  // the timed steps must not touch the APD state
+  const bool split0 = pl->split;
   std::vector<yh_kernel_cfg> cands = candidates(pl);
+  cands.push_back({YH_KERNEL_AUTO, 1, 0, 0, 1});
   pl->apd_on = false;
+  pl->split = false;
   yh_kernel_cfg bestc = cfg0;
-  float bestt = 1e30f;
+  float bestt = 1e30f, autot = 1e30f;
   int rc = YH_OK;
   for (const yh_kernel_cfg& c : cands) {
     pl->cfg = c;
@@ -120,7 +129,9 @@ extern "C" int yh_autotune(yh_plan* pl, int steps, void* stream, yh_kernel_cfg* 
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, e0, e1);
     const float per_step = ms / ((float)calls * call);
-    if (per_step < bestt) {
+    if (c.variant == YH_KERNEL_AUTO) {
+      autot = per_step;
+    } else if (per_step < bestt) {
       bestt = per_step;
       bestc = c;
     }
@@ -139,14 +150,18 @@ extern "C" int yh_autotune(yh_plan* pl, int steps, void* stream, yh_kernel_cfg* 
   pl->past_prev_u = false;
   if (rc) {
     pl->cfg = cfg0;
+    pl->split = split0;
     return rc;
   }
   pl->cfg = bestc;
+  // (of tiled configurations alone, whose results AUTO's equal bit for bit)
+  pl->split = bestc.variant == YH_KERNEL_TILED && autot < bestt;
+  const float ms = pl->split ? autot : bestt;
   {
     std::lock_guard<std::mutex> g(g_mu);
-    g_cache[key] = {bestc, bestt};
+    g_cache[key] = {bestc, ms, pl->split};
   }
   if (best) *best = bestc;
-  if (best_ms) *best_ms = bestt;
+  if (best_ms) *best_ms = ms;
   return YH_OK;
 }

@@ -166,8 +166,7 @@ bool auto_wins(const AutoTable& t, int model, bool masked, const KParams& k, int
   return t.of(n) < gain * ((n / K) * us(K) + (r ? us(r) : 0.0));
 }
 
-yh_kernel_cfg resolve_cfg(const yh_plan* pl) {
-  yh_kernel_cfg c = pl->cfg;
+yh_kernel_cfg resolve_cfg(const yh_plan* pl, yh_kernel_cfg c) {
   if (c.variant == YH_KERNEL_AUTO)
     c = auto_cfg(pl->p.nx, pl->p.ny, pl->cus, tiled_per_cu(pl, 4, 16, 1, false) >= 2);
   if (c.variant == YH_KERNEL_TILED) {
@@ -243,7 +242,9 @@ int plan_advance(yh_plan* pl, int nsteps, hipStream_t s) {
   if (nsteps == 0) return YH_OK;
   if (pl->p.solidSwitch && !pl->mask_set) return YH_ESTATE;
   pl->state_epoch += 1;
-  const yh_kernel_cfg c = resolve_cfg(pl);
+  const bool automatic = pl->cfg.variant == YH_KERNEL_AUTO || pl->split;
+  const yh_kernel_cfg c =
+      resolve_cfg(pl, automatic ? yh_kernel_cfg{YH_KERNEL_AUTO, 1, 0, 0, 1} : pl->cfg);
   const bool masked = pl->p.solidSwitch != 0;
   int remaining = nsteps;
   auto fields = [&](int b, CFields* ci, Fields* co) {
@@ -296,7 +297,7 @@ int plan_advance(yh_plan* pl, int nsteps, hipStream_t s) {
   const int tail = (pl->keep_prev && !prev_fused) ? 1 : 0;
   if (prev_fused && !pl->prev_u) YH_HIP(hipMalloc(&pl->prev_u, pl->n * sizeof(float)));
   bool split = false;  // the launches of the AUTO table
-  if (tiled && pl->cfg.variant == YH_KERNEL_AUTO && remaining > tail) {
+  if (tiled && automatic && remaining > tail) {
     AutoTable& t = pl->table[ap ? 1 : 0];
     if (!t.ready) auto_table(pl->p.model, masked, pl->k, pl->cus, ap != nullptr, &t);
     split = auto_wins(t, pl->p.model, masked, pl->k, pl->cus, c, ap != nullptr, remaining - tail);
@@ -488,12 +489,13 @@ int yh_set_kernel(yh_plan* pl, const yh_kernel_cfg* cfg) {
       return YH_EINVAL;
   }
   pl->cfg = *cfg;
+  pl->split = false;
   return YH_OK;
 }
 
 int yh_get_kernel(const yh_plan* pl, yh_kernel_cfg* cfg) {
   if (!pl || !cfg) return YH_EINVAL;
-  *cfg = resolve_cfg(pl);
+  *cfg = resolve_cfg(pl, pl->cfg);
   return YH_OK;
 }
 

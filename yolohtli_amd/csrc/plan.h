@@ -83,6 +83,7 @@ struct yh_plan {
   int tipcap = 0;
   int* flag_d = nullptr;
   yh_kernel_cfg cfg{YH_KERNEL_AUTO, 4, 8, 8, 1};
+  bool split = false;  // the tuner found AUTO's launches faster than cfg, its fastest
   yh::GenTable general;    // launches of the general path
   yh::AutoTable table[2];  // without and with the APD update
   int64_t count = 0;
@@ -123,8 +124,8 @@ int64_t tiled_tile_count(int nx, int ny, int rows, int waves, int cols, int K);
 // Whether a tiled launch of `tiles` workgroups, `per_cu` per CU at most,
 // writes its outputs through to memory (KParams::wt).
 bool tiled_write_through(int64_t tiles, int cus, int per_cu);
-// Resolve YH_KERNEL_AUTO to a concrete configuration for this plan.
-yh_kernel_cfg resolve_cfg(const yh_plan* pl);
+// A configuration of this plan with YH_KERNEL_AUTO resolved to a concrete one.
+yh_kernel_cfg resolve_cfg(const yh_plan* pl, yh_kernel_cfg c);
 // Advance `nsteps` on the plan's buffers, keeping u of the step before the
 // last (for the tip test) when keep_prev: the last tiled launch writes it to
 // prev_u, or a single-step tail leaves it in buf[cur^1].
