@@ -137,11 +137,20 @@ static double tiled_time(int model, bool masked, bool apd, int nx, int ny, int r
 // the shape, the depth or where launches split, so a call may mix them: the
 // table holds the best shape of every depth, the depth with the least time
 // per step, and for the last steps of a call the split with the least time.
+//
+// With APD a CU holds one region of 16 waves.  Where it holds three of 4 x 8 (all
+// but masked fibres, FK) the large ones are taken only if all are resident at
+// once: in several rounds the small ones' loads overlap better than the estimate
+// knows (2048 x 2048 FK: 8 x 16 at K=6 estimated best, 16% over 4 x 8 at K=5).
 void auto_table(int model, bool masked, const KParams& k, int cus, bool apd, AutoTable* t) {
+  const int64_t n = std::max(1, cus);
+  auto held = [&](int rows, int waves) { return tiled_per_cu(model, masked, k, rows, waves, 1, false, apd); };
+  const bool small = apd && held(4, 8) >= 3;
   t->fill(std::min(k.nx, k.ny) - 1, [&](int rows, int waves, int K) {
     if (apd && !tiled_apd_supported(rows, waves, 1)) return -1.0;
-    return tiled_time(model, masked, apd, k.nx, k.ny, rows, waves, K, std::max(1, cus),
-                      tiled_per_cu(model, masked, k, rows, waves, 1, false, apd));
+    const int per_cu = held(rows, waves);
+    if (small && waves == 16 && tile_count(k.nx, k.ny, rows, waves, 1, K) > n * per_cu) return -1.0;
+    return tiled_time(model, masked, apd, k.nx, k.ny, rows, waves, K, (int)n, per_cu);
   });
 }
 
