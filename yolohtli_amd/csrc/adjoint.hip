@@ -442,18 +442,21 @@ __device__ __forceinline__ void adj_rev_cell(const AdjK& k, const FkEval& r, con
 }
 
 // The cell's term of dL/dD in that step: over its links r (c mu - cw L_n)
-// (u_n - u), du* the differences.  The factors are exact products' differences
-// rounded once, their products and sums FP64 (FP32 sums, 1e-7 of a link's term
-// off, made 5.51 ms of 256 x 256 x 2000 5.48).
-__device__ __forceinline__ double adj_gD(const AdjK& k, const Coef4& cf, const Coef4& cw, float mu,
-                                         float LW, float LE, float LN, float LS, float duW,
-                                         float duE, float duN, float duS) {
+// (u_n - u), du* the differences, added to the sums of each axis (adj_gD_of()
+// weighs them with r).  The factors are exact products' differences rounded once,
+// products and sums FP64.
+__device__ __forceinline__ void adj_gD(const Coef4& cf, const Coef4& cw, float mu, float LW,
+                                       float LE, float LN, float LS, float duW, float duE,
+                                       float duN, float duS, double gd[2]) {
 #pragma clang fp contract(off)
   const float gW = __builtin_fmaf(-LW, cw.W, mu * cf.W), gE = __builtin_fmaf(-LE, cw.E, mu * cf.E);
   const float gN = __builtin_fmaf(-LN, cw.N, mu * cf.N), gS = __builtin_fmaf(-LS, cw.S, mu * cf.S);
-  const double x = __builtin_fma((double)gE, (double)duE, (double)gW * (double)duW);
-  const double y = __builtin_fma((double)gN, (double)duN, (double)gS * (double)duS);
-  return __builtin_fma((double)k.rxt, x, (double)k.ryt * y);
+  gd[0] = __builtin_fma((double)gE, (double)duE, __builtin_fma((double)gW, (double)duW, gd[0]));
+  gd[1] = __builtin_fma((double)gN, (double)duN, __builtin_fma((double)gS, (double)duS, gd[1]));
+}
+__device__ __forceinline__ double adj_gD_of(const AdjK& k, const double gd[2]) {
+#pragma clang fp contract(off)
+  return __builtin_fma((double)k.rxt, gd[0], (double)k.ryt * gd[1]);
 }
 
 // Its terms of dL/dtau (tau_d, tau_r, tau_si, tau_0, tau_v+, tau_w+) without
@@ -529,13 +532,13 @@ __global__ __launch_bounds__(256) void k_adj_rev(const AdjK k, CFields X, CField
     const FkEval r = fk_eval(k, u, X.f[1][c], X.f[2][c]);
     float lu, lv, lw;
     adj_rev_cell(k, r, o, mu, mv, mw, LW, LE, LN, LS, src, lu, lv, lw);
-    const double gd = adj_gD(k, cf, o.cw, mu, LW, LE, LN, LS, U[W] - u, U[E] - u, U[N] - u,
-                             U[S] - u);
+    double gd[2] = {0.0, 0.0};
+    adj_gD(cf, o.cw, mu, LW, LE, LN, LS, U[W] - u, U[E] - u, U[N] - u, U[S] - u, gd);
     adj_gtau(r, mu, mv, mw, gtd);
     lam_out.f[0][c] = lu;
     lam_out.f[1][c] = lv;
     lam_out.f[2][c] = lw;
-    gD[c] += gd;
+    gD[c] += adj_gD_of(k, gd);
   }
   double* slot = gtau_part + (size_t)(blockIdx.y * gridDim.x + blockIdx.x) * 6;
   const int tid = threadIdx.y * blockDim.x + threadIdx.x;
@@ -621,7 +624,7 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_rev_tiled(
   double* gt_slot = gtau_part + (size_t)tile * 6;
   const double gD_was = q.m == 0 ? gD[c] : 0.0;
   const double gt_was = threadIdx.x < 6 ? gt_slot[threadIdx.x] : 0.0;
-  double gd = 0.0, gtd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  double gd[2] = {0.0, 0.0}, gtd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   for (int s = 0; s < K; ++s) {
     const int b = s & 1;
     const Ahead then = fetch(s + 2);
@@ -633,8 +636,8 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_rev_tiled(
       adj_rev_cell(k, r, o, mu, mv, mw, LW, LE, LN, LS, cur.src, Lu, Lv, Lw);
       if (q.m == 0) {  // dL/dD and dL/dtau of the tile's cells
         const float* U = s_U[b];
-        gd += adj_gD(k, cf, o.cw, mu, LW, LE, LN, LS, U[at.W] - cur.u, U[at.E] - cur.u,
-                     U[at.N] - cur.u, U[at.S] - cur.u);
+        adj_gD(cf, o.cw, mu, LW, LE, LN, LS, U[at.W] - cur.u, U[at.E] - cur.u,
+               U[at.N] - cur.u, U[at.S] - cur.u, gd);
         adj_gtau(r, mu, mv, mw, gtd);
       }
       s_L[b ^ 1][at.l] = Lu;
@@ -648,7 +651,7 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_rev_tiled(
     store_through(lam_out.f[0], (uint32_t)c, Lu);
     store_through(lam_out.f[1], (uint32_t)c, Lv);
     store_through(lam_out.f[2], (uint32_t)c, Lw);
-    gD[c] = gD_was + gd;
+    gD[c] = gD_was + adj_gD_of(k, gd);
   }
   adj_gtau_block<kAdjTile * kAdjTile>(gtd, gt_was, gt_slot);
 }
