@@ -68,7 +68,8 @@ typedef struct yh_fk_params {
  * diff_par != diff_per) act on the square domain, and with Dirichlet the
  * anisotropic term also with a mask; with a mask and Neumann both have no
  * effect, as in the reference.  The standard branch (Neumann, Euler, 5-point)
- * runs on the temporally blocked kernels; the others on a per-stage path. */
+ * runs on the temporally blocked kernels; the others on the general path, which
+ * takes several Runge-Kutta stages a launch. */
 typedef struct yh_params {
   int nx, ny;
   double Lx, Ly;                 /* cm */
@@ -201,7 +202,10 @@ int yh_get_kernel(const yh_plan* plan, yh_kernel_cfg* cfg);
  * With a tiled kernel of one column per lane, a remainder of nsteps % K
  * steps may run inside the call's last launch on the shape one row taller
  * per wave; the result does not depend on how steps are split into
- * launches. */
+ * launches.  The launches alternate between the plan's two state buffers, and
+ * their number is the library's choice: a call recorded into a graph goes on
+ * from its own result at the next replay only where that number is even.
+ * yh_step_noalloc is the call to record. */
 int yh_step(yh_plan* plan, int nsteps, void* stream);
 /* yh_step without any device allocation, on caller-owned device fields (no
  * counterpart in the reference: for callers that cannot allocate device
@@ -232,7 +236,7 @@ int yh_check_finite(yh_plan* plan, void* stream);
 /* Mouse stimulus of the plan's steps (stimLockMouse and point,
  * reactionDiffusion.cu:54-61,134): on != 0 applies the current 24.7 within
  * radius^2 < 400 cells of (x, y) in every following step until switched off.
- * While on, the plan steps on the per-stage path. */
+ * While on, the plan steps on the general path. */
 int yh_set_stimulus(yh_plan* plan, int on, int x, int y);
 
 /* Plan options.  YH_OPT_SR_LAUNCHES (default 2): launches per symmetry-

@@ -517,7 +517,8 @@ static int general_depth(const GParams& g, int order, int halo) {
 
 // Steps to fuse and rows of a region on a device of `cus` compute units.  A
 // launch takes about 4 us besides its stages and runs as many rounds as its
-// workgroups (16 waves, one a CU) fill; a row and stage costs c us on a CU.
+// workgroups fill, counted one a CU (16 waves; two of the square rule's without
+// APD fit, of all others one); a row and stage costs c us on a CU.
 // More steps a launch pay its fixed part less often and recompute a wider
 // ring: RK4 with lap4 takes two steps a launch at 512 x 512 (17.3 against 2 x
 // 10.1 us, one round either way) and one at 1024 x 1024 (22.2 us, two rounds,

@@ -8,8 +8,7 @@
 namespace yh {
 
 // v of the lane that DPP control CTRL names, 0 where it names none: 0x100 + n
-// the lane n up in its row of 16, 0x110 + n the lane n down, 0x142 (0x143) the
-// last lane of the row (half) before.
+// the lane n up in its row of 16.
 template <int CTRL>
 __device__ __forceinline__ double dpp_double(double v) {
   const long long b = __double_as_longlong(v);

@@ -142,6 +142,8 @@ static double tiled_time(int model, bool masked, bool apd, int nx, int ny, int r
 // but masked fibres, FK) the large ones are taken only if all are resident at
 // once: in several rounds the small ones' loads overlap better than the estimate
 // knows (2048 x 2048 FK: 8 x 16 at K=6 estimated best, 16% over 4 x 8 at K=5).
+// (8 x 16 of masked FK keeps 12 to 44 bytes a lane in scratch; its timings, and
+// so the constants, hold that.)
 void auto_table(int model, bool masked, const KParams& k, int cus, bool apd, AutoTable* t) {
   const int64_t n = std::max(1, cus);
   auto held = [&](int rows, int waves) { return tiled_per_cu(model, masked, k, rows, waves, 1, false, apd); };

@@ -103,7 +103,7 @@ struct yh_plan {
 };
 
 namespace yh {
-// Steps of this plan run on the general per-stage path (another branch, or
+// Steps of this plan run on the general path (general.hip: another branch, or
 // the mouse stimulus on).
 inline bool plan_general(const yh_plan* pl) { return !standard_branch(pl->p) || pl->stim_on; }
 // The YH_KERNEL_AUTO rule for an nx x ny grid on a device of `cus` compute

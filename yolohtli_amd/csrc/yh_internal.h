@@ -364,8 +364,9 @@ struct GenTable {
 };
 GenTable general_table(int model, const GParams& g, int order, int steps, int cus);
 // shape.K steps of the general path in one launch, from `in` to `out` (never
-// the same).  prev (may be null) receives u one step before the end, vt
-// (entries may be null) the last step's velocity; solid is null without a mask.
+// the same).  prev (may be null) receives u one step before the end, vt (every
+// entry of the model, or all null) the last step's velocity; solid is null
+// without a mask.
 hipError_t launch_general(int model, const GParams& g, int order, GenShape shape, CFields in,
                           Fields out, Fields vt, float* prev, const uint8_t* solid,
                           hipStream_t s, const ApdState* apd);
