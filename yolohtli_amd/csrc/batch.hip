@@ -249,8 +249,10 @@ static int batch_worklist(yh_batch* b, const yh_kernel_cfg& c, yh_batch::WL** ou
 // of one shape well, and shapes that fill one round of workgroups; in several
 // rounds the shapes overlap one workgroup's loads with another's substeps
 // differently, which it does not know (24 masked FK tissues of 300 and 500:
-// 7 x 16 at K=4 estimated 9% under 8 x 8 at K=6, measured 22% over).  So only
-// 8 x 8, the shape without a table, is taken for several rounds; < 0: not taken.
+// 7 x 16 at K=4 estimated 9% under 8 x 8 at K=6, measured 22% over).  So for
+// several rounds the others are taken for a few steps only, mostly loads and
+// stores, which it does know (120 tissues of 128, 2V, 3 steps: 17.7 us, 8 x 8
+// 19.8): regions of 16 waves up to K=3, 4 x 8 up to K=5.  < 0: not taken.
 static double batch_time(const yh_batch* b, int rows, int waves, int K, int cus, int resident) {
   static const double fit[2][2][4] = {
       // substep, row of a wave, issue, load and store
@@ -263,7 +265,8 @@ static double batch_time(const yh_batch* b, int rows, int waves, int K, int cus,
     tiles += (int64_t)((p.nx + wout - 1) / wout) * ((p.ny + hout - 1) / hout);
   const int64_t per_cu = std::max(1, resident / cus);
   const int64_t L = (tiles + cus - 1) / cus, q = (L + per_cu - 1) / per_cu;
-  if (q > 1 && !(rows == 8 && waves == 8)) return -1.0;
+  const int few = rows == 8 && waves == 8 ? 16 : waves == 8 ? 5 : 3;
+  if (q > 1 && K > few) return -1.0;
   const double computed = (double)K * H - (double)K * (K + 1);
   return 4.2 + q * K * (c[0] + c[1] * rows) + L * (computed * c[2] + H * c[3]);
 }
