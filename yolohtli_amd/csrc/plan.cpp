@@ -162,10 +162,13 @@ void auto_table(int model, bool masked, const KParams& k, int cus, bool apd, Aut
 // 14% less time in the mean than with c, 20-40% on ragged grids whose tiles of
 // the fixed shape would fill a last round badly (1300 x 1300 masked FK: 2.76
 // against 3.89 us a step), 10-25% below 400 x 400 (4 x 8 regions at K=12), and
-// at most 5% more.  A call of a few steps where c is 8 x 8, a single launch on
-// a large grid, needs 10%: it moves the state once for little arithmetic, and
-// what the estimate says of shapes that do that alike was off by up to 13%
-// (1136 x 2590 2V, 3 steps: 12.9 us, and 14.4 on 7 x 16).
+// at most 6% more.  A call of a few steps where c is one launch of 8 x 8 on a
+// large grid moves the state once for little arithmetic; there an estimated gain
+// of 3 to 10% is real with 4 x 8 and 4 x 16 regions (measured 5 to 10%) but not
+// with taller ones of 16 waves (a loss of 1% in the mean, of 17% at worst; 1136 x
+// 2590 2V, 3 steps: 12.9 us, and 14.4 on 7 x 16), which need 10%, except for one
+// step with two on a CU (a gain of 8%).  Of 3832 calls of 1 to 8 steps on grids of
+// 0.7 to 6 M cells 2% then take 3 to 14% more than with c, all 5.5% less in the mean.
 bool auto_wins(const AutoTable& t, int model, bool masked, const KParams& k, int cus,
                const yh_kernel_cfg& c, bool apd, int n) {
   const int per_cu = tiled_per_cu(model, masked, k, c.rows, c.waves, c.cols, false, apd);
@@ -173,7 +176,13 @@ bool auto_wins(const AutoTable& t, int model, bool masked, const KParams& k, int
   auto us = [&](int d) {
     return tiled_time(model, masked, apd, k.nx, k.ny, c.rows, c.waves, d, std::max(1, cus), per_cu);
   };
-  const double gain = n <= K && c.rows == 8 && c.waves == 8 && !apd ? 0.90 : 0.97;
+  double gain = 0.97;
+  if (n <= K && c.rows == 8 && c.waves == 8 && !apd) {
+    const yh_kernel_cfg& l = t.next(n);
+    if (l.rows > 4 && l.waves == 16 &&
+        (n > 1 || tiled_per_cu(model, masked, k, l.rows, l.waves, l.cols, false, apd) < 2))
+      gain = 0.90;
+  }
   return t.of(n) < gain * ((n / K) * us(K) + (r ? us(r) : 0.0));
 }
 
