@@ -6,11 +6,10 @@ a call allocates and rebuilds nothing, so calls in turn take the time of the
 same calls in a row (a rebuilt list costs a synchronisation, two allocations and
 two uploads, more than a call of this batch; 1.5 leaves room for noise).
 """
-import time
-
 import numpy as np
 import pytest
 
+from timing import ratio
 from yolohtli_amd import abi_types as T
 from yolohtli_amd.batch import Batch, batched_workload
 
@@ -45,22 +44,15 @@ def test_calls_of_two_sizes_in_turn(torch_cuda, model, graph):
             np.testing.assert_array_equal(x, y)
     ref.close()
 
-    def timed(order):
-        best = float("inf")
-        for _ in range(6):
-            torch.cuda.synchronize()
-            t = time.perf_counter()
-            for n in order:
-                b.step(n)
-            torch.cuda.synchronize()
-            best = min(best, time.perf_counter() - t)
-        return best
+    def calls(order):
+        for n in order:
+            b.step(n)
 
     slow = {}
     for p, q in PAIRS:
-        turn, row = timed((p, q) * 8), timed((p,) * 8) + timed((q,) * 8)
-        if turn > 1.5 * row:
-            slow[p, q] = (turn, row)
+        r = ratio(torch, lambda: calls((p, q) * 8), lambda: calls((p,) * 8 + (q,) * 8), 1, 1.5)
+        if r >= 1.5:
+            slow[p, q] = r
     b.close()
     assert not slow
 
@@ -84,19 +76,10 @@ def test_untuned_batch_is_not_slower_than_one_shape(torch_cuda, model, ntissues,
         if fixed:
             b.set_kernel(substeps=6, rows=8, waves=8, cols=1, persistent=0)
         batches.append(b)
-    best = [float("inf")] * 2
-    for _ in range(8):
-        for q, b in enumerate(batches):
-            b.step(200)
-            torch.cuda.synchronize()
-            t = time.perf_counter()
-            b.step(200)
-            b.step(200)
-            torch.cuda.synchronize()
-            best[q] = min(best[q], time.perf_counter() - t)
+    least = ratio(torch, lambda: batches[0].step(200), lambda: batches[1].step(200), 2, 1.05)
     for b in batches:
         b.close()
-    assert best[0] < 1.05 * best[1]
+    assert least < 1.05
 
 
 @pytest.mark.parametrize("model,ntissues,sides,steps", [(1, 1, (64,), 15), (0, 2, (64,), 16),
@@ -130,17 +113,7 @@ def test_tuned_batch_is_not_slower_than_an_untuned_one(torch_cuda, model, ntissu
     for t in range(ntissues):
         for x, y in zip(batches[0].get_state(t), batches[1].get_state(t)):
             np.testing.assert_array_equal(x, y)
-    best = [float("inf")] * 2
-    for _ in range(12):
-        for q, b in enumerate(batches):
-            b.step(steps)
-            b.step(steps)
-            torch.cuda.synchronize()
-            t = time.perf_counter()
-            for _ in range(40):
-                b.step(steps)
-            torch.cuda.synchronize()
-            best[q] = min(best[q], time.perf_counter() - t)
+    least = ratio(torch, lambda: batches[1].step(steps), lambda: batches[0].step(steps), 40, 1.08)
     for b in batches:
         b.close()
-    assert best[1] < 1.08 * best[0]
+    assert least < 1.08

@@ -1,11 +1,10 @@
 """The previous u of the general path's calls (the tip test's input): a launch of
 several steps writes it, a single step leaves it in the other state buffer."""
-import time
-
 import numpy as np
 import pytest
 
 import yolohtli_amd as Y
+from timing import ratio
 from yolohtli_amd import abi_types as T
 
 pytestmark = pytest.mark.gpu
@@ -95,16 +94,6 @@ def test_single_step_moves_no_more_than_the_wrapper(torch_cuda):
     pl.set_state(*f)
     a = [torch.from_numpy(x).cuda() for x in f]
     b = [torch.empty_like(x) for x in a]
-    best = [float("inf")] * 2
-    for _ in range(8):
-        for q, one in enumerate((lambda: pl.step(1),
-                                 lambda: Y.reactionDiffusion_wrapper(p, b, a))):
-            one()
-            torch.cuda.synchronize()
-            t = time.perf_counter()
-            for _ in range(20):
-                one()
-            torch.cuda.synchronize()
-            best[q] = min(best[q], time.perf_counter() - t)
+    least = ratio(torch, lambda: pl.step(1), lambda: Y.reactionDiffusion_wrapper(p, b, a), 20, 1.1)
     pl.close()
-    assert best[0] < 1.1 * best[1]
+    assert least < 1.1

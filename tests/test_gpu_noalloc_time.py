@@ -4,12 +4,12 @@ with the launch table made on every call it took twice as long).  Calls of
 alternating grids and models keep their tables; a call of more grids than are kept
 gives the same bits."""
 import ctypes as C
-import time
 
 import numpy as np
 import pytest
 
 import yolohtli_amd as Y
+from timing import ratio
 from yolohtli_amd import abi_types as T
 from yolohtli_amd._lib import lib
 
@@ -30,19 +30,15 @@ def test_one_step_is_one_launch(torch_cuda, model):
     torch = torch_cuda
     sets = [(p, *_arrays(torch, p)) for p in (T.grid_params(n, n, model=model) for n in (64, 200, 256))]
     s = torch.cuda.current_stream().cuda_stream
-    fns = (lambda p, o, i: lib().yh_step_noalloc(C.byref(p), o, i, None, 1, s),
-           lambda p, o, i: lib().yh_rd_step_dev(C.byref(p), o, i, None, None, s))
-    best = [float("inf")] * 2
-    for _ in range(10):
-        for q, fn in enumerate(fns):
-            torch.cuda.synchronize()
-            t = time.perf_counter()
-            for _ in range(40):
-                for p, _, _, (o, i), _ in sets:
-                    assert fn(p, o, i) == 0
-            torch.cuda.synchronize()
-            best[q] = min(best[q], time.perf_counter() - t)
-    assert best[0] < 1.4 * best[1], best
+
+    def calls(fn):
+        for p, _, _, (o, i), _ in sets:
+            assert fn(p, o, i) == 0
+
+    assert ratio(torch,
+                 lambda: calls(lambda p, o, i: lib().yh_step_noalloc(C.byref(p), o, i, None, 1, s)),
+                 lambda: calls(lambda p, o, i: lib().yh_rd_step_dev(C.byref(p), o, i, None, None, s)),
+                 40, 1.4) < 1.4
 
 
 def test_more_grids_than_are_kept(torch_cuda):
