@@ -272,9 +272,10 @@ static double batch_time(const yh_batch* b, int rows, int waves, int K, int cus,
 }
 
 // Whether a call of n steps takes the table's launches rather than first's: while
-// the batch is free, for an estimated gain of 3% (57 other batches of 2 to 32
-// tissues, 0.03 to 8 M cells: never slower, 16% faster in the mean; a batch of a
-// few small tissues twice as fast, since first was picked on 256).
+// the batch is free, for an estimated gain of 3% (200 steps of 57 other batches
+// of 2 to 32 tissues, 0.03 to 8 M cells: never slower, 16% faster in the mean; 2 to
+// 40 steps of 38 more: 5% slower at most, 17% faster; a batch of a few small
+// tissues twice as fast, since first was picked on 256).
 static int batch_auto(yh_batch* b, int n, bool* wins) {
   *wins = false;
   if (!b->free) return YH_OK;
